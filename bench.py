@@ -57,7 +57,7 @@ def parse_args():
                     help="0: one update call per weight group instead of one call batching all groups' factor work")
     ap.add_argument("--rq16", type=int, default=1, help="0: keep R Q in fp32 between the Procrustes products (option 7)")
     ap.add_argument("--f32kc", type=int, default=1,
-                    help="0: fp32 products on the general engine instead of the k-contiguous kernel's fp32 twin (option 8)")
+                    help="0: fp32 products on fp32 MFMAs instead of six bf16 products of exact splits (option 8)")
     ap.add_argument("--vmm", type=int, default=-1,
                     help="V A kernel of the norm bounds (option 4): -1 by shape, 0 split-K, 1 column blocks, 2 LDS rows, "
                          "3 upper tiles in tournament-paired rounds")
@@ -381,7 +381,7 @@ def bench_vitb(args):
     agg, syrk = aggregate(recs, peak)
     kid = max(agg, key=lambda k: agg[k][1])
     n_l, ms_tot, fl_tot, by_tot, roof_tot = agg[kid]
-    prec_of = "bf16" if (kid >= 5000 or (kid % 1000) // 100 == 1) else "fp32"
+    prec_of = "fp32" if kid // 1000 == 6 or kid in (7001, 7003) else "bf16"
     ai = fl_tot / by_tot
     mfma_bound = ai >= PEAK[prec_of] / PEAK_HBM
     achieved = fl_tot / (ms_tot * 1e-3) / 1e12 if mfma_bound else by_tot / (ms_tot * 1e-3) / 1e9

@@ -70,10 +70,10 @@ int psgdk_symm(int prec, int side, int sign, int64_t n, int64_t p, int b_dtype, 
 int psgdk_trmm(int prec, int64_t n, int64_t p, int b_dtype, int nb, const float* const* Q, int64_t ldq,
                const void* const* B, int64_t ldb, float* const* C, int64_t ldc, psgdk_stream_t stream);
 
-/* psgdk_trmm with a workspace: the operands are converted once (triu(Q) with zeros below the diagonal, and for
- * prec bf16 B^T, in bf16) and multiplied on the k-contiguous MFMA kernel, each output tile's k loop starting at the
- * diagonal (n(n+1)p flops in place of 2 n^2 p). Needs n and p multiples of 8 (bf16) or 4 (fp32, with fp32 B and n
- * > 32); other shapes take psgdk_trmm and need no workspace. Q's strict lower triangle is never read. */
+/* psgdk_trmm with a workspace: for prec bf16 with n and p multiples of 8 the operands are converted once (triu(Q) with
+ * zeros below the diagonal, and B^T, in bf16) and multiplied on the k-contiguous MFMA kernel, each output tile's k loop
+ * starting at the diagonal (n(n+1)p flops in place of 2 n^2 p). Everything else takes psgdk_trmm and needs no
+ * workspace. Q's strict lower triangle is never read. */
 int psgdk_trmm_ws(int prec, int64_t n, int64_t p, int b_dtype, int nb, const float* const* Q, int64_t ldq,
                   const void* const* B, int64_t ldb, float* const* C, int64_t ldc, void* ws, size_t* ws_bytes,
                   psgdk_stream_t stream);
@@ -304,11 +304,10 @@ int psgdk_fill_normal(void* out, int64_t n, int dtype, uint64_t seed, uint64_t s
 /* Launch profiling (diagnostic, per host thread): after psgdk_profile_start every MFMA-engine launch the thread makes is
  * bracketed by a pair of HIP events on its stream. psgdk_profile_stop ends the recording and, with out non-NULL,
  * waits for the recorded events and fills one record per launch: the kernel instantiation id
- * (general engine: cfg * 1000 + prec * 100 + a_dtype * 10 + b_dtype, cfg 0 = 128 x 128 tiles, 1 = 32 x 128;
- * bf16 engine: 5000 + cfg * 10 + epilogue, cfg as option 1 below, epilogue 0 = store, 1 = factor update, 2 = Procrustes
+ * (bf16 engine: 5000 + cfg * 10 + epilogue, cfg as option 1 below, epilogue 0 = store, 1 = factor update, 2 = Procrustes
  * step, 3 = scale, 4 = R Q with its trace partials, 5 = store with sums of squares, 6 = the r2 trace SYRK's scale
  * applied twice, 7 = Procrustes step reading (R Q)^T in bf16;
- * its fp32 twin: 6000 + cfg * 10 + epilogue; the small-problem kernels: 7000 / 7001 on 64 x 64 tiles, 7002 / 7003
+ * converting engine: 6000 (fp32) or 8000 (bf16 precision) + cfg * 10 + epilogue, cfg as option 13; the small-problem kernels: 7000 / 7001 on 64 x 64 tiles, 7002 / 7003
  * the tiny-product kernel, bf16 / fp32 operands), whether it was a
  * SYRK (triangular grid), the problems in the launch, its device time, its algorithmic flop count (SYRK n(n+1)k,
  * TRMM n(n+1)p, GEMM 2mnk, per problem) and its algorithmic bytes (operands read once, outputs written once). With out NULL only *n_records is set (records kept). */
@@ -343,12 +342,12 @@ int psgdk_profile_stop(psgdk_prof_record_t* out, int max_records, int* n_records
  * 4 m d^2 flops; 0: term1 Q, 2 d^3 flops); option 6 = side streams of psgdk_kron2d_update_groups (default 3; 0 or
  * 1: everything on the caller's stream); option 7 = whether the bf16 update keeps R Q (the Procrustes correction)
  * in bf16 (1, default: only the bf16 (R Q)^T, which the Q update also reads) or fp32 (0) between its two
- * products; option 8 = whether fp32 products with k- or m/n-contiguous operands (M > 32, one k range, no packed
- * output) take the k-contiguous kernel's fp32 twin (1, default) or the general engine (0); option 9 = the most
+ * products; option 8 = whether the converting engine sums fp32 products as six bf16 products of exact three-way
+ * splits (1, default) or on fp32 MFMAs (0, three to four times slower); option 9 = the most
  * factors of one side >= 2048 that psgdk_kron2d_update_groups batches into one launch (1 .. 64, default 64; smaller
  * batches of one side run on different side streams); option 10 = plain-store bf16 GEMMs on k-contiguous operands
  * whose launch has fewer 128 x 128 tiles than this take the small-problem kernel (64 x 64 tiles, k in chunks of 512
- * bytes per row with two in flight); bf16 SYRKs below 1.5 times it and fp32 products below 3 times it (default 128,
+ * bytes per row with two in flight); bf16 SYRKs below 1.5 times it and fp32 products of fewer than 64 64 x 64 tiles (default 128,
  * 0: never; not with a forced tile configuration, option 1); option 11 = of those, a launch with fewer 64 x 64 tiles
  * than this takes the tiny-product kernel (32 x 32 tiles whose four waves split k; results rounded in another
  * order than the other kernels' k-order sums; default 64, 0: never); option 12 = whether launches given 256 x 256
@@ -357,7 +356,9 @@ int psgdk_profile_stop(psgdk_prof_record_t* out, int max_records, int* n_records
  * steps and the r2 trace SYRK), whose registers spill in configuration 3 (three waves per SIMD) and in configuration 4
  * exceed the 128 of two workgroups per CU (1, default; 0: never). On gfx950
  * configurations 0, 1, 3 and 4 round the same sums (their k steps of 32 and 16 accumulate in one order:
- * bitwise-equal products). */
+ * bitwise-equal products). option 13 = tile configuration of the converting engine (-1 chosen by size, 0 = 128 x 256,
+ * 1 = 64 x 64, 2 = 32 x 64 (plain and sum-of-squares products; others as by size), 3 = 64 x 64 with k split over two
+ * wave groups; a product that 0 does not take runs on 1). */
 int psgdk_set_option(int option, int value);
 /* The calling thread's value of a psgdk_set_option switch. */
 int psgdk_get_option(int option, int* value);

@@ -177,22 +177,18 @@ class Workspace:
 
 def kernel_name(kernel_id):
     """Kernel template name of a profiling kernel id."""
+    if kernel_id // 1000 in (6, 8):  # the converting engine: 6000 (fp32) or 8000 (bf16 precision) + 10 cfg + epilogue
+        cfg, epi = divmod(kernel_id % 1000, 10)
+        tile = {0: "128, 256, 4, 1", 1: "64, 64, 2, 1", 2: "32, 64, 2, 2", 3: "64, 64, 2, 2"}[cfg]
+        return f"gemm_cv_kernel<{3 if kernel_id < 7000 else 1}, {tile}, {epi}>"
     if kernel_id >= 7000:  # the small-problem kernels: 7000 / 7001 64-tiles, 7002 / 7003 tiny (bf16 / fp32)
         kind = "tiny" if kernel_id % 10 >= 2 else "small"
         return f"gemm_{kind}_kernel<{'float' if kernel_id % 2 else 'unsigned short'}>"
-    if kernel_id >= 5000:  # 5000 (bf16) or 6000 (fp32 k-contiguous) + 10 cfg + epilogue
-        base = 6000 if kernel_id >= 6000 else 5000
-        cfg, epi = divmod(kernel_id - base, 10)
-        tile = {0: "256, 256, 2, 4", 1: "128, 128, 2, 2", 2: "256, 256, 2, 2", 3: "256, 256, 2, 4",
-                4: "128, 128, 2, 2"}[cfg]
-        ws = ", 4" if cfg in (3, 4) else ""  # the warp-specialized kernels' 4 producer waves
-        return f"gemm_{'f32kc' if base == 6000 else 'bf16'}_kernel<{tile}, {epi}{ws}>"
-    cfg, rest = divmod(kernel_id, 1000)
-    prec, rest = divmod(rest, 100)
-    adt, bdt = divmod(rest, 10)
-    t = {0: "float", 1: "unsigned short"}
-    tile = "32, 128, 1, 4" if cfg else "128, 128, 2, 2"
-    return f"gemm_kernel<{prec}, {t[adt]}, {t[bdt]}, {tile}>"
+    cfg, epi = divmod(kernel_id - 5000, 10)
+    tile = {0: "256, 256, 2, 4", 1: "128, 128, 2, 2", 2: "256, 256, 2, 2", 3: "256, 256, 2, 4",
+            4: "128, 128, 2, 2"}[cfg]
+    ws = ", 4" if cfg in (3, 4) else ""  # the warp-specialized kernels' 4 producer waves
+    return f"gemm_bf16_kernel<{tile}, {epi}{ws}>"
 
 
 def profile_start():

@@ -14,10 +14,10 @@
 #include "elem.h"
 #include "gemm.h"
 #include "gemm_bf16.h"
+#include "gemm_cv.h"
 #include "nlb.h"
 
 namespace psgdk {
-hipError_t gemm_launch(GemmArgs& a, int prec, int adt, int bdt, int cfg, hipStream_t st);
 hipError_t debug_mfma_launch(const float* A, const float* B, float* C, int prec, hipStream_t st);
 hipError_t mfma_rate_launch(int iters, int wgs, float* out, hipStream_t st);
 hipError_t read_rate_launch(const void* buf, long long bytes, int wgs, int iters, long long stride, unsigned* sink,
@@ -73,14 +73,6 @@ size_t esize(int dt) { return dt == PSGDK_BF16 ? 2 : 4; }
 
 bool aligned16(const void* p) { return (reinterpret_cast<uintptr_t>(p) & 15) == 0; }
 
-template <typename P>
-bool vec_ok(P const* ptrs, int nb, int64_t ld, int dt) {
-  if ((ld * (int64_t)esize(dt)) % 16 != 0) return false;
-  for (int b = 0; b < nb; ++b)
-    if (!aligned16(ptrs[b])) return false;
-  return true;
-}
-
 int check_nb(int nb) {  // problems per public call (a launch may batch several calls' problems, up to MAXB)
   if (nb < 1 || nb > PSGDK_MAXB) return fail(PSGDK_EINVAL, "nb = %d: must be in 1..%d", nb, PSGDK_MAXB);
   return PSGDK_OK;
@@ -129,15 +121,6 @@ struct Prof {  // one per host thread: a thread's records cover its own launches
 thread_local Prof g_prof;
 thread_local LaunchShape g_last_launch;  // set by psgdk::note_launch (end of this file)
 
-// Instantiation id of gemm_kernel<PREC, TA, TB, tile config>: cfg * 1000 + prec * 100 + adt * 10 + bdt.
-int kernel_id(int prec, int adt, int bdt, int cfg) { return cfg * 1000 + prec * 100 + adt * 10 + bdt; }
-
-void gemm_init(GemmArgs& a) {
-  std::memset(&a, 0, sizeof a);
-  a.alpha = 1.f;
-  a.splitk = 1;
-}
-
 // Operand description for the GEMM launcher.
 struct Opnd {
   int mode = KC, sign = 1, dt = PSGDK_F32;
@@ -155,71 +138,13 @@ struct EpiSpec {
   float* part[MAXB] = {};
 };
 
-int gemm_cfg(int64_t M) { return M <= 32 ? 1 : 0; }
-int gemm_tiles(int64_t M, int64_t N, int tri) {
-  const int cfg = gemm_cfg(M);
-  const int64_t tm = cfg ? (M + 31) / 32 : (M + 127) / 128, tn = (N + 127) / 128;
-  return (int)(tri ? tm * (tm + 1) / 2 : tm * tn);
-}
-
-// The general engine (gemm.hip): every operand mode, precision, split-K and triangular option.
-int run_gemm_general(int prec, int nb, int64_t M, int64_t N, int64_t K, const Opnd& A, const Opnd& B,
-                     float* const* C, int64_t ldc, const EpiSpec& e, int tri, int out_mode, int kbeg_tri, int splitk,
-                     int64_t kchunk, hipStream_t st) {
-  GemmArgs a;
-  gemm_init(a);
-  a.M = (int)M; a.N = (int)N; a.K = (int)K;
-  a.amode = A.mode; a.asign = A.sign; a.lda = A.ld;
-  a.bmode = B.mode; a.bsign = B.sign; a.ldb = B.ld;
-  a.ldc = ldc; a.ldx = e.ldx;
-  a.alpha = e.alpha; a.beta = e.beta; a.epi = e.epi;
-  a.tri = tri; a.out_mode = out_mode; a.kbeg_tri = kbeg_tri;
-  a.splitk = splitk; a.kchunk = (int)(splitk > 1 ? kchunk : K);
-  a.avec = vec_ok(A.p, nb, A.ld, A.dt);
-  a.bvec = vec_ok(B.p, nb, B.ld, B.dt);
-  a.nb = nb;
-  for (int b = 0; b < nb; ++b) {
-    a.A[b] = A.p[b]; a.B[b] = B.p[b]; a.C[b] = C[b];
-    a.X1[b] = e.X1[b]; a.X2[b] = e.X2[b]; a.s[b] = e.s[b]; a.part[b] = e.part[b];
-  }
-  const int cfg = gemm_cfg(M);
-  if (!g_prof.on) return hip_check(gemm_launch(a, prec, A.dt, B.dt, cfg, st), "gemm launch");
-  ProfRec r;
-  r.kernel_id = kernel_id(prec, A.dt, B.dt, cfg);
-  r.tri = tri;
-  r.nb = nb;
-  if (tri) r.flops = (double)M * (M + 1) * K * nb;                    // SYRK: n(n+1)k
-  else if (kbeg_tri) r.flops = (double)M * (M + 1) * N * nb;         // TRMM: n(n+1)p
-  else r.flops = 2.0 * M * N * K * nb;
-  {  // operands once (a triangle-read operand: its triangle), outputs once, epilogue reads and a beta read of C
-    auto opnd = [&](const Opnd& o, int64_t mn) {
-      const double el = o.mode == SYM ? (double)K * (K + 1) / 2 : (double)mn * K;
-      return el * (double)esize(o.dt);
-    };
-    const double out = tri ? (out_mode == PSGDK_OUT_MIRROR ? (double)M * M : (double)M * (M + 1) / 2) : (double)M * N;
-    double x = 0;
-    if (e.X1[0]) x += out;
-    if (e.X2[0]) x += out;
-    r.bytes = nb * (opnd(A, M) + (tri ? 0.0 : opnd(B, N)) + 4.0 * out * (1 + (e.beta != 0.f) + x / out));
-  }
-  r.a = g_prof.ev();
-  r.b = g_prof.ev();
-  if (!r.a || !r.b) return fail(PSGDK_EHIP, "profiling: hipEventCreate failed");
-  g_last_launch = LaunchShape();
-  PSGDK_HIP(hipEventRecord(r.a, st), "profiling event");
-  PSGDK_TRY(hip_check(gemm_launch(a, prec, A.dt, B.dt, cfg, st), "gemm launch"));
-  PSGDK_HIP(hipEventRecord(r.b, st), "profiling event");
-  r.m = M;
-  r.n = tri ? M : N;
-  r.k = K;
-  r.shape = last_launch();
-  g_prof.recs.push_back(r);
-  return PSGDK_OK;
-}
-// run_gemm_general, or the k-contiguous kernel's fp32 twin where it applies (defined after run_b16)
+// A product of operands in any layout (gemm_cv.hip, or the small-problem kernels where they apply; defined after
+// run_b16). ntiles (optional): the output tiles, i.e. the epilogue's partials per problem.
 int run_gemm(int prec, int nb, int64_t M, int64_t N, int64_t K, const Opnd& A, const Opnd& B, float* const* C,
              int64_t ldc, const EpiSpec& e, int tri, int out_mode, int kbeg_tri, int splitk, int64_t kchunk,
-             hipStream_t st);
+             hipStream_t st, int* ntiles = nullptr);
+// The most partials an epilogue of run_gemm writes for an M x N product
+int max_tiles(int64_t M, int64_t N, int tri) { return gemm_cv_tiles(M, N, tri, 1); }
 
 // ------------------------------------------------------------------------------------------------------------
 // bf16 k-contiguous GEMM (gemm_bf16.hip). A: M x K rows, B: N x K rows (bf16, k contiguous); C = acc A B^T.
@@ -227,7 +152,6 @@ struct B16Out {
   float* C[MAXB] = {};
   bf16_t* Cb[MAXB] = {};
   bf16_t* CTb[MAXB] = {};
-  float* CT[MAXB] = {};  // fp32 kernel only
   int64_t ldc = 0, ldcb = 0, ldct = 0;
 };
 
@@ -246,7 +170,8 @@ thread_local int g_vmm_cols = -1;      // option 4: V A kernel: -1 by shape (3 f
 thread_local int g_t1q_pg = 1;  // option 5: bf16 update forms term1 Q through Pg where cheaper (1) or never (0)
 thread_local int g_upd_streams = 3;  // option 6: side streams of psgdk_kron2d_update_groups (0: the caller's only)
 thread_local int g_rq16 = 1;   // option 7: the bf16 update keeps R Q in bf16 (1) or fp32 (0) for the Q update
-thread_local int g_f32kc = 1;  // option 8: fp32 products with k-contiguous operands take the k-contiguous kernel
+thread_local int g_split = 1;  // option 8: fp32 products as six bf16 products of three-way splits (1) or fp32 MFMAs (0)
+thread_local int g_cv_cfg = -1;  // option 13: tile configuration of the converting engine (-1 chosen by size)
 thread_local int g_big_batch = MAXB;  // option 9: items per batch of the grouped update for factor sides >= 2048
 thread_local int g_small = 128;       // option 10: bf16 plain-store GEMMs with fewer 128 x 128 tiles than this (over
                                       // the launch) take the small-problem kernel; bf16 SYRKs below 1.5 times it, fp32
@@ -320,41 +245,42 @@ int b16_cfg(int64_t M, int64_t N, int64_t K, int tri, int nb, int epi) {
   return ws ? 3 : 0;
 }
 
-// Operand contract of the k-contiguous kernel (gemm_bf16, esz 2; its fp32 twin, esz 4): 16-byte aligned bases,
-// leading dimensions multiples of one 16-byte chunk, each operand under 2 GiB (buffer extent); a k-contiguous
-// operand (rows of the buffer: m or n) needs K a multiple of a chunk, an m/n-contiguous one (fp32 only, amc / bmc:
-// rows of the buffer: k) M or N a multiple of 4.
+// Operand contract of the k-contiguous kernels (esz 2: bf16, 4: fp32): 16-byte aligned bases, K and the leading
+// dimensions multiples of one 16-byte chunk, each operand under 2 GiB (buffer extent).
 template <typename P>
 bool b16_operands_ok(int nb, int64_t M, int64_t N, int64_t K, P const* A, int64_t lda, P const* B, int64_t ldb,
-                     int esz = 2, bool amc = false, bool bmc = false) {
+                     int esz = 2) {
   const int64_t ce = 16 / esz, big = (int64_t)1 << 31;
-  auto one = [&](int64_t mn, int64_t ld, bool mc) {
-    if (ld % ce) return false;
-    if (mc) return mn % ce == 0 && ld >= mn && K * ld * esz < big;
-    return K % ce == 0 && ld >= K && mn * ld * esz < big;
-  };
-  if (!one(M, lda, amc) || !one(N, ldb, bmc)) return false;
+  if (K % ce || lda % ce || ldb % ce || lda < K || ldb < K || M * lda * esz >= big || N * ldb * esz >= big) return false;
   for (int b = 0; b < nb; ++b)
     if (!aligned16(A[b]) || !aligned16(B[b])) return false;
   return true;
 }
 
-// The k-contiguous kernel on bf16 (esz 2) or fp32 (esz 4) operands.
+// Whether an fp32 product of k-contiguous operands takes the small-problem kernels, on fp32 MFMAs: below 64 64-tiles the
+// tiny-product kernel (option 11; with it off, the 64-tile kernel) beats the converting engine (one 512 x 512 SYRK, 36
+// tiles: 8.2 us against 15.1; one 512^3 product, 64 tiles: 16.3 against 12.4).
+bool small_f32(int64_t M, int64_t N, int tri, int nb) {
+  return g_small > 0 && (int64_t)gemm_small_tiles(M, N, tri) * nb < 64;
+}
+
+// The k-contiguous kernel on bf16 operands (esz 2), or the small-problem kernels on fp32 ones (esz 4; the caller has
+// checked small_f32).
 // kbeg: A is upper-triangular with its zeros stored; each tile starts its k loop at its first row (TRMM).
 // kper (optional, bf16 k-contiguous operands): problem b has its own K = kper[b] with lda = ldb = kper[b]; K is then
 // the largest of them (the size rule's K).
 int run_b16(int nb, int64_t M, int64_t N, int64_t K, const void* const* A, int64_t lda, const void* const* B,
             int64_t ldb, const B16Out& o, const EpiSpec& e, int tri, int out_mode, int* ntiles, hipStream_t st,
-            int esz = 2, bool amc = false, bool bmc = false, int kbeg = 0, const int* kper = nullptr) {
+            int esz = 2, int kbeg = 0, const int* kper = nullptr) {
   if (kper) {
-    if (esz != 2 || amc || bmc || kbeg) return fail(PSGDK_EINVAL, "per-problem K: bf16 k-contiguous operands only");
+    if (esz != 2 || kbeg) return fail(PSGDK_EINVAL, "per-problem K: bf16 k-contiguous operands only");
     for (int b = 0; b < nb; ++b) {
       const void* Ab[1] = {A[b]};
       const void* Bb[1] = {tri ? A[b] : B[b]};
       if (kper[b] < 1 || kper[b] > K || !b16_operands_ok(1, M, tri ? M : N, kper[b], Ab, kper[b], Bb, kper[b]))
         return fail(PSGDK_EINVAL, "k-contiguous kernel operand contract violated (problem %d, K = %d)", b, kper[b]);
     }
-  } else if (!b16_operands_ok(nb, M, tri ? M : N, K, A, lda, tri ? A : B, ldb, esz, amc, tri ? amc : bmc)) {
+  } else if (!b16_operands_ok(nb, M, tri ? M : N, K, A, lda, tri ? A : B, ldb, esz)) {
     return fail(PSGDK_EINVAL, "k-contiguous kernel operand contract violated (K, leading dimensions, alignment or size)");
   }
   GB16Args a;
@@ -363,26 +289,22 @@ int run_b16(int nb, int64_t M, int64_t N, int64_t K, const void* const* A, int64
   a.lda = lda; a.ldb = ldb; a.ldc = o.ldc; a.ldcb = o.ldcb; a.ldct = o.ldct; a.ldx = e.ldx;
   a.alpha = e.alpha; a.epi = e.epi; a.tri = tri; a.out_mode = out_mode; a.nb = nb;
   a.vec = g_tile_order;
-  a.amc = amc; a.bmc = tri ? amc : bmc;
   a.kbeg = kbeg;
   a.kper = kper ? 1 : 0;
   for (int b = 0; b < nb; ++b) {
     a.kp[b] = kper ? kper[b] : (int)K;
     a.A[b] = reinterpret_cast<const bf16_t*>(A[b]);
     a.B[b] = reinterpret_cast<const bf16_t*>(B[b]);
-    a.C[b] = o.C[b]; a.Cb[b] = o.Cb[b]; a.CTb[b] = o.CTb[b]; a.CT[b] = o.CT[b];
+    a.C[b] = o.C[b]; a.Cb[b] = o.Cb[b]; a.CTb[b] = o.CTb[b];
     a.X1[b] = e.X1[b]; a.X2[b] = e.X2[b]; a.s[b] = e.s[b]; a.part[b] = e.part[b];
   }
-  int cfg = b16_cfg(M, N, K, tri, nb, e.epi);
-  if (esz == 4) cfg = 1;  // the fp32 kernel: the 128-tile configuration
+  const int cfg = b16_cfg(M, N, K, tri, nb, e.epi);
   // a plain store whose 128-tiles would leave most of the chip idle: the small-problem kernel (64-tiles, k in
   // 512-byte chunks, two in flight). Measured crossovers against the pipelined kernels (launch of nb problems, in
-  // 128-tiles): bf16 GEMMs about 130, bf16 SYRKs (whose triangle the 64-tiles follow more closely) about 200, fp32
-  // products about 400 (the fp32 twin's main loop is the slower one there).
+  // 128-tiles): bf16 GEMMs about 130, bf16 SYRKs (whose triangle the 64-tiles follow more closely) about 200.
   const int64_t t128 = (int64_t)gemm_bf16_tiles(M, N, tri, 1) * nb;
-  const int64_t small_max = esz == 4 ? 3 * (int64_t)g_small : tri ? 3 * (int64_t)g_small / 2 : g_small;
-  const bool small = e.epi == EPI_STORE && !kbeg && !kper && !amc && !(tri ? amc : bmc) && g_force_cfg < 0 &&
-                     t128 < small_max;
+  const int64_t small_max = tri ? 3 * (int64_t)g_small / 2 : g_small;
+  const bool small = esz == 4 || (e.epi == EPI_STORE && !kbeg && !kper && g_force_cfg < 0 && t128 < small_max);
   // ... and one whose 64-tiles would still fill only a fraction of the CUs: the tiny-product kernel
   const bool tiny = small && (int64_t)gemm_small_tiles(M, N, tri) * nb < g_tiny;
   if (ntiles)
@@ -390,11 +312,11 @@ int run_b16(int nb, int64_t M, int64_t N, int64_t K, const void* const* A, int64
   auto launch = [&]() {
     if (tiny) return gemm_tiny_launch(a, esz, st);
     if (small) return gemm_small_launch(a, esz, st);
-    return esz == 4 ? gemm_f32kc_launch(a, cfg, st) : gemm_bf16_launch(a, cfg, st);
+    return gemm_bf16_launch(a, cfg, st);
   };
   if (!g_prof.on) return hip_check(launch(), "k-contiguous gemm launch");
   ProfRec r;
-  r.kernel_id = small ? 7000 + (tiny ? 2 : 0) + (esz == 4 ? 1 : 0) : (esz == 4 ? 6000 : 5000) + cfg * 10 + a.epi;
+  r.kernel_id = small ? 7000 + (tiny ? 2 : 0) + (esz == 4 ? 1 : 0) : 5000 + cfg * 10 + a.epi;
   r.tri = tri;
   r.nb = nb;
   double ksum = (double)K * nb;  // the problems' k extents summed
@@ -411,9 +333,8 @@ int run_b16(int nb, int64_t M, int64_t N, int64_t K, const void* const* A, int64
     if (o.C[0]) by += 4 * out;
     if (o.Cb[0]) by += 2 * out;
     if (o.CTb[0]) by += 2 * out;
-    if (o.CT[0]) by += 4 * out;
     const int ep = e.epi;
-    if (e.X1[0]) by += (ep == EPI_RQ ? esz : 4) * out;  // EPI_RQ reads R in the operand type
+    if (e.X1[0]) by += (ep == EPI_RQ ? 2 : 4) * out;  // EPI_RQ reads R in bf16
     if (e.X2[0]) by += (ep == EPI_PROCB ? 2 : 4) * out;  // EPI_PROCB reads the bf16 (R Q)^T
     r.bytes = by * nb;
   }
@@ -434,26 +355,96 @@ int run_b16(int nb, int64_t M, int64_t N, int64_t K, const void* const* A, int64
   return PSGDK_OK;
 }
 
+// The converting engine's tiles: 32 x 64 for products of at most 32 rows; 64 x 64 on two wave groups that split k where
+// that is at most one workgroup per CU (1024^3 fp32: 25 us against 30 on one group); 128 x 256 where its tiles fill more
+// than half of the CUs (fp32: 6 products of 1536 x 512 x 512, 144 tiles, 46 us against 50; 1531^3, 72 tiles, 115 against
+// 78), in bf16, whose conversion is a larger part, more than one and a half rounds of them (3072^3, 288 tiles, 173 us
+// against 154; two of them 264 against 311); 64 x 64 otherwise, and for fp32 Gram
+// products X^T X, whose diagonal only those tiles sum closely enough (gemm_cv.hip).
+int cv_cfg(int prec, int64_t M, int64_t N, int tri, int nb, int epi, bool narrow, bool gram) {
+  const bool narrow_ok = !tri && (epi == EPI_STORE || epi == EPI_SUMSQ);
+  if (g_cv_cfg == 2 ? narrow_ok : g_cv_cfg >= 0) return narrow && g_cv_cfg == 0 ? 1 : g_cv_cfg;
+  if (M <= 32 && narrow_ok) return 2;
+  if ((int64_t)gemm_cv_tiles(M, N, tri, 3) * nb <= 256) return 3;
+  return !narrow && !gram && (int64_t)gemm_cv_tiles(M, N, tri, 0) * nb >= (prec == PSGDK_PREC_F32 ? 144 : 400) ? 0 : 1;
+}
+
 int run_gemm(int prec, int nb, int64_t M, int64_t N, int64_t K, const Opnd& A, const Opnd& B, float* const* C,
              int64_t ldc, const EpiSpec& e, int tri, int out_mode, int kbeg_tri, int splitk, int64_t kchunk,
-             hipStream_t st) {
-  // fp32 products on the k-contiguous kernel's fp32 twin: fp32 operands stored k- or m/n-contiguous (not a triangle),
-  // M > 32 (the general engine's 128 x 128 tiles, so that per-tile partials count the same), one k range, no packed
-  // output, a plain store only without beta, and a SYRK's single operand.
-  const bool kc_epi = e.epi == EPI_FACTOR || e.epi == EPI_PROC || e.epi == EPI_SCALE || e.epi == EPI_RQ ||
-                      e.epi == EPI_SUMSQ || e.epi == EPI_STRACE || (e.epi == EPI_STORE && e.beta == 0.f);
-  if (g_f32kc && prec == PSGDK_PREC_F32 && A.dt == PSGDK_F32 && B.dt == PSGDK_F32 && M > 32 && splitk == 1 &&
-      !kbeg_tri && out_mode != PSGDK_OUT_PACKED && kc_epi && A.mode != SYM && B.mode != SYM &&
-      (!tri || A.mode == B.mode) &&
-      b16_operands_ok(nb, M, tri ? M : N, K, A.p, A.ld, tri ? A.p : B.p, tri ? A.ld : B.ld, 4, A.mode == MC,
-                      (tri ? A.mode : B.mode) == MC)) {
+             hipStream_t st, int* ntiles) {
+  // small fp32 products of k-contiguous operands (plain store): the small-problem kernels on fp32 MFMAs. The packed
+  // output, which they do not write, sums the same way there (fp32 MFMAs, k in blocks of 128).
+  const bool small = prec == PSGDK_PREC_F32 && A.dt == PSGDK_F32 && B.dt == PSGDK_F32 && A.mode == KC && B.mode == KC &&
+                     M > 32 && splitk == 1 && !kbeg_tri && e.epi == EPI_STORE && e.beta == 0.f && g_force_cfg < 0 &&
+                     g_split && small_f32(M, N, tri, nb) &&
+                     b16_operands_ok(nb, M, tri ? M : N, K, A.p, A.ld, tri ? A.p : B.p, tri ? A.ld : B.ld, 4);
+  if (small && out_mode != PSGDK_OUT_PACKED) {
     B16Out o;
     o.ldc = ldc;
     for (int b = 0; b < nb; ++b) o.C[b] = C[b];
-    return run_b16(nb, M, N, K, A.p, A.ld, tri ? A.p : B.p, tri ? A.ld : B.ld, o, e, tri, out_mode, nullptr, st, 4,
-                   A.mode == MC, (tri ? A.mode : B.mode) == MC);
+    return run_b16(nb, M, N, K, A.p, A.ld, tri ? A.p : B.p, tri ? A.ld : B.ld, o, e, tri, out_mode, ntiles, st, 4);
   }
-  return run_gemm_general(prec, nb, M, N, K, A, B, C, ldc, e, tri, out_mode, kbeg_tri, splitk, kchunk, st);
+  CvArgs a;
+  std::memset(&a, 0, sizeof a);
+  a.M = (int)M; a.N = (int)N; a.K = (int)K;
+  auto opnd = [&](const Opnd& o) {
+    CvOperand c;
+    c.mode = o.mode; c.sign = o.sign; c.bf16 = o.dt == PSGDK_BF16; c.ld = o.ld;
+    c.vec = o.ld < (1 << 21);
+    if (c.bf16) {  // four bf16 in one 8-byte load: 4-byte aligned
+      c.vec = c.vec && o.ld % 2 == 0;
+      for (int b = 0; b < nb; ++b) c.vec = c.vec && (reinterpret_cast<uintptr_t>(o.p[b]) & 3) == 0;
+    }
+    return c;
+  };
+  a.a = opnd(A);
+  a.b = tri ? a.a : opnd(B);
+  a.ldc = ldc; a.ldx = e.ldx;
+  a.alpha = e.alpha; a.beta = e.beta; a.epi = e.epi;
+  a.tri = tri; a.out_mode = out_mode; a.kbeg = kbeg_tri;
+  a.splitk = splitk; a.kchunk = (int)(splitk > 1 ? kchunk : K);
+  a.f32 = prec == PSGDK_PREC_F32 && (!g_split || small);
+  a.order = g_tile_order;
+  a.nb = nb;
+  for (int b = 0; b < nb; ++b) {
+    a.A[b] = A.p[b]; a.B[b] = B.p[b]; a.C[b] = C[b];
+    a.X1[b] = e.X1[b]; a.X2[b] = e.X2[b]; a.s[b] = e.s[b]; a.part[b] = e.part[b];
+  }
+  const int cfg = cv_cfg(prec, M, N, tri, nb, e.epi, !gemm_cv_wide(a),
+                         prec == PSGDK_PREC_F32 && tri && e.epi == EPI_STORE && A.mode == MC);
+  if (ntiles) *ntiles = gemm_cv_tiles(M, N, tri, cfg);
+  if (!g_prof.on) return hip_check(gemm_cv_launch(a, prec, cfg, st), "gemm launch");
+  ProfRec r;
+  r.kernel_id = (prec == PSGDK_PREC_F32 ? 6000 : 8000) + cfg * 10 + e.epi;
+  r.tri = tri;
+  r.nb = nb;
+  if (tri) r.flops = (double)M * (M + 1) * K * nb;                    // SYRK: n(n+1)k
+  else if (kbeg_tri) r.flops = (double)M * (M + 1) * N * nb;         // TRMM: n(n+1)p
+  else r.flops = 2.0 * M * N * K * nb;
+  {  // operands once (a triangle-read operand: its triangle), outputs once, epilogue reads and a beta read of C
+    auto opnd_bytes = [&](const Opnd& o, int64_t mn) {
+      const double el = o.mode == SYM ? (double)K * (K + 1) / 2 : (double)mn * K;
+      return el * (double)esize(o.dt);
+    };
+    const double out = tri ? (out_mode == PSGDK_OUT_MIRROR ? (double)M * M : (double)M * (M + 1) / 2) : (double)M * N;
+    double x = 0;
+    if (e.X1[0]) x += out;
+    if (e.X2[0]) x += out;
+    r.bytes = nb * (opnd_bytes(A, M) + (tri ? 0.0 : opnd_bytes(B, N)) + 4.0 * out * (1 + (e.beta != 0.f) + x / out));
+  }
+  r.a = g_prof.ev();
+  r.b = g_prof.ev();
+  if (!r.a || !r.b) return fail(PSGDK_EHIP, "profiling: hipEventCreate failed");
+  g_last_launch = LaunchShape();
+  PSGDK_HIP(hipEventRecord(r.a, st), "profiling event");
+  PSGDK_TRY(hip_check(gemm_cv_launch(a, prec, cfg, st), "gemm launch"));
+  PSGDK_HIP(hipEventRecord(r.b, st), "profiling event");
+  r.m = M;
+  r.n = tri ? M : N;
+  r.k = K;
+  r.shape = last_launch();
+  g_prof.recs.push_back(r);
+  return PSGDK_OK;
 }
 
 // ------------------------------------------------------------------------------------------------------------
@@ -738,19 +729,6 @@ int precondition(const psgdk_kron2d_t* g, const void* const* X, int xdt, float* 
   for (int b = 0; b < nb; ++b) cur[b] = X[b];
   bool sumsq_done = false;
   float* const* dst1 = k1 != PSGDK_FACTOR_NONE ? tmp : out;
-  if (g->prec == PSGDK_PREC_F32 && curdt == PSGDK_BF16 && g_f32kc && k0 == PSGDK_FACTOR_DENSE &&
-      k1 == PSGDK_FACTOR_DENSE && m > 32) {
-    // bf16 X on the fp32 path: widened into `out` (free until the second product) so that P1 X takes the fp32
-    // twin of the k-contiguous kernel (the general engine, reading the bf16 X, ran 12 products of 768 x 3072 x 768
-    // at 27.5 TFLOP/s)
-    EwArgs a;
-    std::memset(&a, 0, sizeof a);
-    a.nb = nb; a.m = m; a.n = n; a.dt = curdt;
-    for (int b = 0; b < nb; ++b) { a.in[b] = cur[b]; a.out[b] = out[b]; }
-    PSGDK_HIP(noise_launch(a, st), "X to fp32");
-    curdt = PSGDK_F32;
-    for (int b = 0; b < nb; ++b) cur[b] = out[b];
-  }
   // rows: P1 X
   if (k0 == PSGDK_FACTOR_DENSE) {
     Opnd A, B;
@@ -763,9 +741,8 @@ int precondition(const psgdk_kron2d_t* g, const void* const* X, int xdt, float* 
       e.epi = EPI_SUMSQ;
       for (int b = 0; b < nb; ++b) e.part[b] = part[b];
       sumsq_done = true;
-      *npart = gemm_tiles(m, n, 0);
     }
-    PSGDK_TRY(run_gemm(g->prec, nb, m, n, m, A, B, dst1, n, e, 0, 0, 0, 1, 0, st));
+    PSGDK_TRY(run_gemm(g->prec, nb, m, n, m, A, B, dst1, n, e, 0, 0, 0, 1, 0, st, npart));
     curdt = PSGDK_F32;
     for (int b = 0; b < nb; ++b) cur[b] = dst1[b];
   } else if (k0 == PSGDK_FACTOR_DIAG || k1 == PSGDK_FACTOR_NONE) {
@@ -793,9 +770,8 @@ int precondition(const psgdk_kron2d_t* g, const void* const* X, int xdt, float* 
       e.epi = EPI_SUMSQ;
       for (int b = 0; b < nb; ++b) e.part[b] = part[b];
       sumsq_done = true;
-      *npart = gemm_tiles(m, n, 0);
     }
-    PSGDK_TRY(run_gemm(g->prec, nb, m, n, n, A, B, out, n, e, 0, 0, 0, 1, 0, st));
+    PSGDK_TRY(run_gemm(g->prec, nb, m, n, n, A, B, out, n, e, 0, 0, 0, 1, 0, st, npart));
   } else if (k1 == PSGDK_FACTOR_DIAG) {
     EwArgs a;
     std::memset(&a, 0, sizeof a);
@@ -952,8 +928,7 @@ int b16_items(const std::vector<B16Item*>& it, const psgdk_update_opts_t* o, con
           ++k;
         }
       EpiSpec e;
-      PSGDK_TRY(run_b16(k, d, d, kmax, A, kmax, A, kmax, out, e, 1, PSGDK_OUT_MIRROR, nullptr, st, 2, false, false,
-                        0, kp));
+      PSGDK_TRY(run_b16(k, d, d, kmax, A, kmax, A, kmax, out, e, 1, PSGDK_OUT_MIRROR, nullptr, st, 2, 0, kp));
     }
   }
   for (int i0 = 0; i0 < nb;) {
@@ -1473,16 +1448,15 @@ int b16_apply(const psgdk_kron2d_t* g, const psgdk_apply_opts_t* o, void* const*
 }
 
 // ------------------------------------------------------------------------------------------------------------
-// Dense factor steps of the general engine, shared by psgdk_kron2d_update and the per-factor entry points.
+// Dense factor steps on the converting engine, shared by psgdk_kron2d_update and the per-factor entry points.
 
 struct FacWs {
   float *R[MAXB], *RQ[MAXB], *coef[MAXB], *rs[MAXB], *pc[MAXB], *tpart[MAXB], *rtp[MAXB];
-  float *Ta[MAXB], *Tb[MAXB];  // fp32 transposed operands of the k-contiguous kernel (Q^T / (R Q)^T, Qn^T)
   NlbWs nw;
 };
 
 void fac_take(Ws& w, int64_t d, int nb, FacWs& o) {
-  const int tp = gemm_tiles(d, d, 0);
+  const int tp = max_tiles(d, d, 0);
   for (int b = 0; b < nb; ++b) {
     o.R[b] = w.take<float>(d * d);
     o.RQ[b] = w.take<float>(d * d);
@@ -1491,39 +1465,15 @@ void fac_take(Ws& w, int64_t d, int nb, FacWs& o) {
     o.pc[b] = w.take<float>(8);
     o.tpart[b] = w.take<float>(2 * (size_t)tp);
     o.rtp[b] = w.take<float>(rform_pairs(d));
-    o.Ta[b] = w.take<float>(d * d);
-    o.Tb[b] = w.take<float>(d * d);
   }
   nlb_take(w, d, nb, o.nw);
 }
 
-// Whether the fp32 factor products of a d x d group take the k-contiguous kernel's fp32 twin with transposed
-// fp32 copies of their n-contiguous operands (Q, Qn, R Q): fp32 arithmetic, d > 32 (the general engine's
-// 128 x 128 tiles, so that per-tile partials count the same), d a multiple of 4, 16-byte aligned matrices.
-bool fac_kc(int prec, int64_t d, int nb, std::initializer_list<const void* const*> ptrs) {
-  if (prec != PSGDK_PREC_F32 || !g_f32kc || d <= 32 || d % 4 || d * d * 4 >= ((int64_t)1 << 31)) return false;
-  for (auto p : ptrs)
-    for (int b = 0; b < nb; ++b)
-      if (!aligned16(p[b])) return false;
-  return true;
-}
-
-// fp32 transposed copies dst[b] = src[b]^T of d x d matrices
-int transpose_f32(int nb, int64_t d, const float* const* src, float* const* dst, hipStream_t st) {
-  EwArgs a;
-  std::memset(&a, 0, sizeof a);
-  a.nb = nb; a.m = d; a.n = d; a.ld = d; a.i0 = 1;
-  for (int b = 0; b < nb; ++b) { a.in[b] = src[b]; a.out[b] = dst[b]; }
-  return hip_check(to_bf16_launch(a, st), "fp32 transpose");
-}
-
 // ell = nlb_spd(term1, V) + term2; L = max(betaL L + (1 - betaL) ell, ell); Qout = Q - lr/L (term1 Q - term2 Q)
 // (psgd_pro.py:132-135). term1: full symmetric, or its upper triangle when t1_tri. Qout must not alias Q.
-// qn_t (optional): set when Qout^T was also written, into w.Tb (the fp32 k-contiguous route; procrustes_run reads
-// it from there)
 int factor_update_run(int prec, int nb, int64_t d, const float* const* T1, int t1_tri, const float* const* Q,
                       float* const* Qout, float* const* Lv, const float* const* V, float lr, float betaL, float term2,
-                      const FacWs& w, hipStream_t st, bool* qn_t = nullptr) {
+                      const FacWs& w, hipStream_t st) {
   {
     NlbFinal fin;
     std::memset(&fin, 0, sizeof fin);
@@ -1539,18 +1489,6 @@ int factor_update_run(int prec, int nb, int64_t d, const float* const* T1, int t
   EpiSpec e;
   e.epi = EPI_FACTOR; e.ldx = d;
   for (int b = 0; b < nb; ++b) { a.p[b] = T1[b]; bq.p[b] = Q[b]; e.X1[b] = Q[b]; e.s[b] = w.coef[b]; }
-  if (qn_t && !t1_tri && fac_kc(prec, d, nb, {reinterpret_cast<const void* const*>(T1), reinterpret_cast<const void* const*>(Q),
-                                              reinterpret_cast<const void* const*>(Qout), reinterpret_cast<const void* const*>(w.Ta),
-                                              reinterpret_cast<const void* const*>(w.Tb)})) {
-    // Q^T into Ta; Qn = Q - c (term1 Q - term2 Q) with term1 and Q^T k-contiguous, Qn^T into Tb on the way out
-    PSGDK_TRY(transpose_f32(nb, d, Q, w.Ta, st));
-    B16Out o;
-    o.ldc = d; o.ldct = d;
-    const void *Ac[MAXB], *Bc[MAXB];
-    for (int b = 0; b < nb; ++b) { Ac[b] = T1[b]; Bc[b] = w.Ta[b]; o.C[b] = Qout[b]; o.CT[b] = w.Tb[b]; }
-    *qn_t = true;
-    return run_b16(nb, d, d, d, Ac, d, Bc, d, o, e, 0, 0, nullptr, st, 4);
-  }
   return run_gemm(prec, nb, d, d, d, a, bq, Qout, d, e, 0, 0, 0, 1, 0, st);
 }
 
@@ -1561,18 +1499,19 @@ int factor_update_run(int prec, int nb, int64_t d, const float* const* T1, int t
 // M's coefficients, M = a rs R - a^2/2 S (in R's buffer), Qout = Q + M Q.
 int procrustes_r2_tail(int prec, int nb, int64_t d, const float* const* Q, float* const* Qout, const FacWs& w,
                        hipStream_t st) {
+  int nt = 0;
   {
     Opnd a;
     a.mode = KC; a.ld = d;
     EpiSpec e;
     e.epi = EPI_STRACE; e.ldx = d;
     for (int b = 0; b < nb; ++b) { a.p[b] = w.R[b]; e.X1[b] = Q[b]; e.s[b] = w.rs[b]; e.part[b] = w.tpart[b]; }
-    PSGDK_TRY(run_gemm(prec, nb, d, d, d, a, a, w.RQ, d, e, 1, PSGDK_OUT_MIRROR, 0, 1, 0, st));
+    PSGDK_TRY(run_gemm(prec, nb, d, d, d, a, a, w.RQ, d, e, 1, PSGDK_OUT_MIRROR, 0, 1, 0, st, &nt));
   }
   {
     EwArgs a;
     std::memset(&a, 0, sizeof a);
-    a.nb = nb; a.i0 = (int)rform_pairs(d); a.i1 = gemm_tiles(d, d, 1); a.f0 = 0.125f;
+    a.nb = nb; a.i0 = (int)rform_pairs(d); a.i1 = nt; a.f0 = 0.125f;
     for (int b = 0; b < nb; ++b) { a.in2[b] = w.rtp[b]; a.in3[b] = w.tpart[b]; a.sc[b] = w.rs[b]; a.out[b] = w.pc[b]; }
     PSGDK_HIP(proc_scalar_r2_launch(a, st), "procrustes r2 step size");
   }
@@ -1592,9 +1531,8 @@ int procrustes_r2_tail(int prec, int nb, int64_t d, const float* const* Q, float
   return run_gemm(prec, nb, d, d, d, a, bq, Qout, d, e, 0, 0, 0, 1, 0, st);
 }
 
-// q_t: w.Tb already holds Q^T (written by factor_update_run)
 int procrustes_run(int prec, int nb, int64_t d, const float* const* Q, float* const* Qout, const float* const* V,
-                   const FacWs& w, hipStream_t st, bool r2 = false, bool q_t = false) {
+                   const FacWs& w, hipStream_t st, bool r2 = false) {
   {
     EwArgs a;
     std::memset(&a, 0, sizeof a);
@@ -1612,40 +1550,7 @@ int procrustes_run(int prec, int nb, int64_t d, const float* const* Q, float* co
     PSGDK_TRY(run_nlb_full(d, -1, nb, Rc, d, 0, V, fin, w.nw, st));
   }
   if (r2) return procrustes_r2_tail(prec, nb, d, Q, Qout, w, st);
-  if (fac_kc(prec, d, nb, {reinterpret_cast<const void* const*>(Q), reinterpret_cast<const void* const*>(Qout),
-                           reinterpret_cast<const void* const*>(w.R), reinterpret_cast<const void* const*>(w.RQ),
-                           reinterpret_cast<const void* const*>(w.Ta), reinterpret_cast<const void* const*>(w.Tb)})) {
-    // k-contiguous operands: Q^T (Tb), then R Q -> RQ and (R Q)^T (Ta), then R RQ with (R Q)^T
-    if (!q_t) PSGDK_TRY(transpose_f32(nb, d, Q, w.Tb, st));
-    const void *Ac[MAXB], *Bc[MAXB];
-    {
-      B16Out o;
-      o.ldc = d; o.ldct = d;
-      EpiSpec e;
-      e.epi = EPI_RQ; e.ldx = d;
-      for (int b = 0; b < nb; ++b) {
-        Ac[b] = w.R[b]; Bc[b] = w.Tb[b]; o.C[b] = w.RQ[b]; o.CT[b] = w.Ta[b];
-        e.X1[b] = w.R[b]; e.s[b] = w.rs[b]; e.part[b] = w.tpart[b];
-      }
-      PSGDK_TRY(run_b16(nb, d, d, d, Ac, d, Bc, d, o, e, 0, 0, nullptr, st, 4));
-    }
-    {
-      EwArgs a;
-      std::memset(&a, 0, sizeof a);
-      a.nb = nb; a.i0 = gemm_tiles(d, d, 0); a.f0 = 0.125f;
-      for (int b = 0; b < nb; ++b) { a.in2[b] = w.tpart[b]; a.sc[b] = w.rs[b]; a.out[b] = w.pc[b]; }
-      PSGDK_HIP(proc_scalar_launch(a, st), "procrustes step size");
-    }
-    B16Out o;
-    o.ldc = d;
-    EpiSpec e;
-    e.epi = EPI_PROC; e.ldx = d;
-    for (int b = 0; b < nb; ++b) {
-      Ac[b] = w.R[b]; Bc[b] = w.Ta[b]; o.C[b] = Qout[b];
-      e.X1[b] = Q[b]; e.X2[b] = w.RQ[b]; e.s[b] = w.pc[b];
-    }
-    return run_b16(nb, d, d, d, Ac, d, Bc, d, o, e, 0, 0, nullptr, st, 4);
-  }
+  int nt = 0;
   {
     Opnd a, bq;
     a.mode = KC; a.ld = d;
@@ -1653,12 +1558,12 @@ int procrustes_run(int prec, int nb, int64_t d, const float* const* Q, float* co
     EpiSpec e;
     e.epi = EPI_RQ; e.ldx = d;
     for (int b = 0; b < nb; ++b) { a.p[b] = w.R[b]; bq.p[b] = Q[b]; e.X1[b] = w.R[b]; e.s[b] = w.rs[b]; e.part[b] = w.tpart[b]; }
-    PSGDK_TRY(run_gemm(prec, nb, d, d, d, a, bq, w.RQ, d, e, 0, 0, 0, 1, 0, st));
+    PSGDK_TRY(run_gemm(prec, nb, d, d, d, a, bq, w.RQ, d, e, 0, 0, 0, 1, 0, st, &nt));
   }
   {
     EwArgs a;
     std::memset(&a, 0, sizeof a);
-    a.nb = nb; a.i0 = gemm_tiles(d, d, 0); a.f0 = 0.125f;
+    a.nb = nb; a.i0 = nt; a.f0 = 0.125f;
     for (int b = 0; b < nb; ++b) { a.in2[b] = w.tpart[b]; a.sc[b] = w.rs[b]; a.out[b] = w.pc[b]; }
     PSGDK_HIP(proc_scalar_launch(a, st), "procrustes step size");
   }
@@ -1768,39 +1673,31 @@ int psgdk_trmm_ws(int prec, int64_t n, int64_t p, int b_dtype, int nb, const flo
   PSGDK_TRY(check_dims(p, "p"));
   if (!ws_bytes) return fail(PSGDK_EINVAL, "ws_bytes is null");
   if (ldq < n || ldb < p || ldc < p) return fail(PSGDK_ESHAPE, "leading dimension too small");
-  // The k-contiguous kernel with the triangle's k range: bf16 takes bf16 copies of triu(Q) (zeros below the
-  // diagonal) and of B^T; fp32 takes an fp32 copy of triu(Q) and reads B as it is (n-contiguous rows of k).
-  const bool bf = prec == PSGDK_PREC_BF16;
-  const bool fast = (bf ? (n % 8 == 0 && p % 8 == 0) : (b_dtype == PSGDK_F32 && n % 4 == 0 && p % 4 == 0 && n > 32 &&
-                                                        g_f32kc && (ldb * 4) % 16 == 0)) &&
-                    n * n * 4 < ((int64_t)1 << 31) && n * p * 4 < ((int64_t)1 << 31);
+  // bf16: the k-contiguous kernel with the triangle's k range, on bf16 copies of triu(Q) (zeros below the diagonal)
+  // and of B^T; everything else reads Q and B in place (psgdk_trmm)
+  const bool fast = prec == PSGDK_PREC_BF16 && n % 8 == 0 && p % 8 == 0 && n * n * 4 < ((int64_t)1 << 31) &&
+                    n * p * 4 < ((int64_t)1 << 31);
   Ws w(ws);
-  void *Qc[MAXB], *Bt[MAXB];
+  bf16_t *Qc[MAXB], *Bt[MAXB];
   for (int b = 0; b < nb; ++b) {
-    Qc[b] = fast ? (bf ? (void*)w.take<bf16_t>(n * n) : (void*)w.take<float>(n * n)) : nullptr;
-    Bt[b] = fast && bf ? (void*)w.take<bf16_t>(p * n) : nullptr;
+    Qc[b] = fast ? w.take<bf16_t>(n * n) : nullptr;
+    Bt[b] = fast ? w.take<bf16_t>(p * n) : nullptr;
   }
   if (!ws) { *ws_bytes = w.off; return PSGDK_OK; }
   if (*ws_bytes < w.off) return fail(PSGDK_EWORKSPACE, "workspace %zu < %zu bytes", *ws_bytes, w.off);
   PSGDK_TRY(check_ptrs(Q, nb, "Q"));
   PSGDK_TRY(check_ptrs(B, nb, "B"));
   PSGDK_TRY(check_ptrs(C, nb, "C"));
-  bool b_aligned = true;  // the fp32 route reads B in place
-  for (int b = 0; b < nb; ++b) b_aligned = b_aligned && aligned16(B[b]);
-  if (!fast || (!bf && !b_aligned)) return psgdk_trmm(prec, n, p, b_dtype, nb, Q, ldq, B, ldb, C, ldc, stream);
+  if (!fast) return psgdk_trmm(prec, n, p, b_dtype, nb, Q, ldq, B, ldb, C, ldc, stream);
   hipStream_t st = (hipStream_t)stream;
   {  // triu(Q), zeros below the diagonal (never read there)
     EwArgs a;
     std::memset(&a, 0, sizeof a);
     a.nb = nb; a.m = n; a.n = n; a.ld = ldq; a.dt = PSGDK_F32; a.i1 = 1;
-    for (int b = 0; b < nb; ++b) {
-      a.in[b] = Q[b];
-      if (bf) a.out2[b] = Qc[b];
-      else a.out[b] = static_cast<float*>(Qc[b]);
-    }
+    for (int b = 0; b < nb; ++b) { a.in[b] = Q[b]; a.out2[b] = Qc[b]; }
     PSGDK_HIP(to_bf16_launch(a, st), "triu(Q) copy");
   }
-  if (bf) {  // B^T in bf16 (p x n)
+  {  // B^T in bf16 (p x n)
     EwArgs a;
     std::memset(&a, 0, sizeof a);
     a.nb = nb; a.m = p; a.n = n; a.ld = ldb; a.dt = b_dtype; a.i0 = 1;
@@ -1810,10 +1707,9 @@ int psgdk_trmm_ws(int prec, int64_t n, int64_t p, int b_dtype, int nb, const flo
   B16Out o;
   o.ldc = ldc;
   const void *Ac[MAXB], *Bc[MAXB];
-  for (int b = 0; b < nb; ++b) { o.C[b] = C[b]; Ac[b] = Qc[b]; Bc[b] = bf ? (const void*)Bt[b] : B[b]; }
+  for (int b = 0; b < nb; ++b) { o.C[b] = C[b]; Ac[b] = Qc[b]; Bc[b] = Bt[b]; }
   EpiSpec e;
-  if (bf) return run_b16(nb, n, p, n, Ac, n, Bc, n, o, e, 0, 0, nullptr, st, 2, false, false, 1);
-  return run_b16(nb, n, p, n, Ac, n, Bc, ldb, o, e, 0, 0, nullptr, st, 4, false, true, 1);
+  return run_b16(nb, n, p, n, Ac, n, Bc, n, o, e, 0, 0, nullptr, st, 2, 1);
 }
 
 int psgdk_gemm(int prec, int trans_a, int trans_b, int64_t m, int64_t n, int64_t k, float alpha, int a_dtype,
@@ -2087,10 +1983,8 @@ int psgdk_kron2d_update(const psgdk_kron2d_t* g, const psgdk_update_opts_t* o, c
     const float* Qc[MAXB];
     const float* Qnc[MAXB];
     for (int b = 0; b < nb; ++b) { T1c[b] = T1[b]; Qc[b] = g->Q[f][b]; Qnc[b] = Qn[b]; }
-    bool qn_t = false;
-    PSGDK_TRY(factor_update_run(g->prec, nb, d, T1c, term_tri, Qc, Qn, g->L[f], Vs, o->lr, o->betaL, term2, fw, st,
-                                &qn_t));
-    PSGDK_TRY(procrustes_run(g->prec, nb, d, Qnc, g->Q[f], Vk, fw, st, o->r2 != 0, qn_t));
+    PSGDK_TRY(factor_update_run(g->prec, nb, d, T1c, term_tri, Qc, Qn, g->L[f], Vs, o->lr, o->betaL, term2, fw, st));
+    PSGDK_TRY(procrustes_run(g->prec, nb, d, Qnc, g->Q[f], Vk, fw, st, o->r2 != 0));
   }
   // P refresh (psgd_pro_fast.py:191-192)
   int sel[MAXB];
@@ -2163,7 +2057,7 @@ int psgdk_kron2d_apply(const psgdk_kron2d_t* g, const psgdk_apply_opts_t* o, voi
   const int64_t m = g->m, n = g->n, mn = m * n;
   Ws w(ws);
   float *tmp[MAXB], *pre[MAXB], *part[MAXB];
-  const int np_max = std::max(gemm_tiles(m, n, 0), 256);
+  const int np_max = std::max(max_tiles(m, n, 0), 256);
   for (int b = 0; b < nb; ++b) {
     tmp[b] = w.take<float>(mn);
     pre[b] = w.take<float>(mn);
@@ -2378,8 +2272,8 @@ int psgdk_set_option(int option, int value) {
     return PSGDK_OK;
   }
   if (option == 8) {
-    if (value < 0 || value > 1) return fail(PSGDK_EINVAL, "option 8 (fp32 k-contiguous kernel) must be 0 or 1");
-    g_f32kc = value;
+    if (value < 0 || value > 1) return fail(PSGDK_EINVAL, "option 8 (fp32 products by splits) must be 0 or 1");
+    g_split = value;
     return PSGDK_OK;
   }
   if (option == 4) {
@@ -2417,6 +2311,11 @@ int psgdk_set_option(int option, int value) {
     g_ws = value;
     return PSGDK_OK;
   }
+  if (option == 13) {
+    if (value < -1 || value > 3) return fail(PSGDK_EINVAL, "option 13 (converting engine's tile config) must be -1 .. 3");
+    g_cv_cfg = value;
+    return PSGDK_OK;
+  }
   if (option == 6) {
     if (value < 0 || value > 8) return fail(PSGDK_EINVAL, "option 6 (grouped update side streams) must be 0 .. 8");
     g_upd_streams = value;
@@ -2428,8 +2327,8 @@ int psgdk_set_option(int option, int value) {
 int psgdk_get_option(int option, int* value) {
   if (!value) return fail(PSGDK_EINVAL, "value is null");
   const int* opts[] = {&g_tile_order, &g_force_cfg,   &g_nlb_target, &g_vmm_u, &g_vmm_cols,
-                       &g_t1q_pg,     &g_upd_streams, &g_rq16,       &g_f32kc, &g_big_batch, &g_small,
-                       &g_tiny,       &g_ws};
+                       &g_t1q_pg,     &g_upd_streams, &g_rq16,       &g_split, &g_big_batch, &g_small,
+                       &g_tiny,       &g_ws,          &g_cv_cfg};
   if (option < 0 || option >= (int)(sizeof opts / sizeof opts[0])) return fail(PSGDK_EINVAL, "unknown option %d", option);
   *value = *opts[option];
   return PSGDK_OK;

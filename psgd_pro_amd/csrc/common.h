@@ -61,10 +61,11 @@ __device__ __forceinline__ float wave_max(float v) {
   return v;
 }
 
-// Raw buffer resource over [base, base + bytes): loads at offsets >= bytes (clamped to 2^31 - 1) return zero,
-// so a lane with nothing to load passes offset 0x7fffffff instead of branching.
+// Raw buffer resource over [base, base + bytes): loads at offsets >= bytes (clamped to 0 .. 2^31 - 1; a tile wholly
+// past its operand has a negative extent, which as an unsigned record count would let every offset through) return
+// zero, so a lane with nothing to load passes offset 0x7fffffff instead of branching.
 __device__ __forceinline__ __amdgpu_buffer_rsrc_t make_rsrc(const void* base, long long bytes) {
-  const int n = bytes > 0x7fffffffLL ? 0x7fffffff : (int)bytes;
+  const int n = bytes > 0x7fffffffLL ? 0x7fffffff : bytes < 0 ? 0 : (int)bytes;
   return __builtin_amdgcn_make_buffer_rsrc(const_cast<void*>(base), (short)0, n, 0x00020000);
 }
 constexpr int kOob = 0x7fffffff;

@@ -1,4 +1,4 @@
-// MFMA GEMM engine: argument block shared by the host launcher and the kernels.
+// MFMA products: problems per launch and epilogues, shared by the host launchers and the kernels.
 #pragma once
 #include "common.h"
 
@@ -20,30 +20,6 @@ enum Epi : int {
   EPI_STRACE = 6,  // SYRK only: C = (s[0] acc) s[0] (the scale applied twice, so that acc = 0 gives 0 for any
                    // finite s[0]), and partials of sum_ij C_ij X1_ij over the whole symmetric C into part[2 t + 1]
                    // (part[2 t] = 0)                                    (Procrustes r2: S = Rn^T Rn, sum(S * Q))
-};
-
-struct GemmArgs {
-  int M, N, K;
-  int amode, bmode;     // OpMode of A (rows m) and B (rows n), both viewed as X[mn][k]
-  int asign, bsign;     // SYM sign
-  long long lda, ldb, ldc, ldx;
-  float alpha, beta;
-  int epi;
-  int tri;              // 1: upper-triangular tile grid (SYRK: M == N, B is A)
-  int out_mode;         // tri: 0 upper triangle only, 1 mirrored full matrix, 2 packed upper triangle
-  int tiles_m, tiles_n, ntiles;
-  int avec, bvec;       // 16-byte vector loads allowed for A / B (alignment of base and ld)
-  int kbeg_tri;         // A is upper-triangular (SYM, sign 0): start the k loop at the tile's first row
-  int splitk, kchunk;   // split-K (EPI_STORE only): split s covers k in [s kchunk, (s+1) kchunk) and writes its
-                        // partial product to C + s * M * ldc
-  int nb;
-  const void* A[MAXB];
-  const void* B[MAXB];
-  float* C[MAXB];
-  const float* X1[MAXB];
-  const float* X2[MAXB];
-  const float* s[MAXB];
-  float* part[MAXB];
 };
 
 }  // namespace psgdk

@@ -10,7 +10,7 @@
 // reads and row writes). Global loads for tile k+1 are in flight while tile k is
 // multiplied; one barrier per k tile. The (problem, tile) list is dealt out so each XCD gets a contiguous run.
 // Operands: K a multiple of 8, leading dimensions multiples of 8, 16-byte aligned bases, under 2 GiB each (the host
-// routes anything else to the general engine); ragged M, N and K edges read zeros through the buffer extent.
+// routes anything else to the converting engine); ragged M, N and K edges read zeros through the buffer extent.
 #include <type_traits>
 
 #include "gemm_bf16.h"
@@ -19,13 +19,12 @@ namespace psgdk {
 
 namespace {
 
-// Element traits of the k-contiguous operands. A k tile is 8 chunks of 16 bytes (one 128-byte LDS row per m or n,
-// chunks XOR-swizzled by row, swz): 64 bf16 or 32 fp32. CE: elements per chunk; MPF: MFMAs per pair of 16-byte
-// fragments (one v_mfma_f32_16x16x32_bf16, or four v_mfma_f32_16x16x4f32 over the fragment's 4 k values, lane group
-// g holding k = 4 g + s for both operands).
-template <typename T> struct Kc;
-template <> struct Kc<bf16_t> { static constexpr int CE = 8, MPF = 1; using F = bf16x8_t; };
-template <> struct Kc<float> { static constexpr int CE = 4, MPF = 4; using F = f32x4_t; };
+// A k tile is 8 chunks of 16 bytes (one 128-byte LDS row per m or n, chunks XOR-swizzled by row, swz): 64 bf16.
+constexpr int CE = 8;        // elements per chunk
+constexpr int BK = 8 * CE;   // k per tile
+constexpr int KP = BK;       // LDS row pitch
+using F = bf16x8_t;          // one MFMA operand fragment
+using T = bf16_t;
 
 // Row pitch (floats) of a wave's parked epilogue block of hr x wc: unpadded and swizzled for 64 x 64 blocks (see ei
 // in the kernel), padded by 4 otherwise.
@@ -52,9 +51,8 @@ __device__ __forceinline__ int swz32(int row, int c) { return c ^ ((row >> 1) & 
 // past K (K is a multiple of a chunk) gets an offset beyond the buffer extent: it reads zero (or, where the scalar
 // part wraps the 32-bit sum, some element of the same buffer), and either way only feeds outputs that are not
 // stored.
-template <typename T, int ROWS, int NT, bool SW32 = false>
+template <int ROWS, int NT, bool SW32 = false>
 struct Ld {
-  static constexpr int CE = Kc<T>::CE, KP = 8 * CE;
   static constexpr int NV = ROWS * 8 / NT;  // 16-byte vectors per thread
   uint4 r[NV];
 
@@ -89,56 +87,22 @@ struct Ld {
       *reinterpret_cast<uint4*>(lds + row * KP + (SW32 ? swz32(row, kv) : swz(row, kv)) * CE) = r[i];
     }
   }
-
-  // An fp32 operand stored m- or n-contiguous, X[k][mn] with row stride ld (the rows of the buffer are k): thread t
-  // owns the 4 x 4 block of k chunk (t / 4) % 8 and tile rows 4 nb .. + 3, nb = 4 (t / 32) + t % 4. Four 16-byte
-  // loads (k rows: each group of 4 lanes reads 64 contiguous bytes, the 8 lanes of one k chunk in a wave 128) are
-  // transposed in registers into the block's four k-contiguous chunks, stored in the same swizzled layout (at most
-  // 2-way bank conflicts). One block per thread (ROWS = NT / 2); rows past the operand and k past K read zero.
-  __device__ __forceinline__ void load_mc(__amdgpu_buffer_rsrc_t rs, long long ld, int mn0, int rows, int k0, int K,
-                                          int t) {
-    static_assert(std::is_same_v<T, float> && NV == 4 && ROWS * 2 == NT, "m/n-contiguous loader: fp32, one block");
-    const int kc = (t >> 2) & 7, nb = (t >> 5) * 4 + (t & 3);
-    const bool nok = mn0 + nb * 4 < rows;
-    const int soff = (int)(((long long)k0 * ld + mn0) * 4);
-#pragma unroll
-    for (int i = 0; i < 4; ++i) {
-      const int k = kc * 4 + i;
-      const int voff = (int)(((long long)k * ld + nb * 4) * 4);
-      r[i] = __builtin_bit_cast(uint4, __builtin_amdgcn_raw_buffer_load_b128(rs, nok && k0 + k < K ? voff : 0x7fffffff,
-                                                                                soff, 0));
-    }
-  }
-  __device__ __forceinline__ void store_mc(T* lds, int t) const {
-    const int kc = (t >> 2) & 7, nb = (t >> 5) * 4 + (t & 3);
-#pragma unroll
-    for (int j = 0; j < 4; ++j) {
-      const int row = nb * 4 + j;
-      const uint4 x = make_uint4((&r[0].x)[j], (&r[1].x)[j], (&r[2].x)[j], (&r[3].x)[j]);
-      *reinterpret_cast<uint4*>(lds + row * KP + swz(row, kc) * CE) = x;
-    }
-  }
 };
 
 }  // namespace
 
-// WGM x WGN waves, each owning a TM x TN block (TM = BM / WGM, TN = BN / WGN) of 16 x 16 MFMA tiles; T = bf16_t
-// (the bf16 kernel) or float (its fp32 twin for k-contiguous fp32 operands: the same tiles, LDS layout, schedule
-// and epilogues, four fp32 MFMAs per fragment pair).
-// LAY (fp32 only): bit 0 set = A stored m-contiguous, bit 1 = B stored n-contiguous (the buffer's rows are k).
-// PW > 0 (bf16, 256 x 256 tiles on 2 x 4 waves): PW further waves only stage the operands (warp-specialized main
+// WGM x WGN waves, each owning a TM x TN block (TM = BM / WGM, TN = BN / WGN) of 16 x 16 MFMA tiles.
+// PW > 0 (256 x 256 tiles on 2 x 4 waves, 128 x 128 on 2 x 2): PW further waves only stage the operands (warp-specialized main
 // loop; see below); the WGM x WGN waves multiply on 32 x 32 x 16 MFMAs and run the epilogue.
-template <typename T, int BM, int BN, int WGM, int WGN, int EPI, int LAY = 0, int PW = 0>
-__device__ __forceinline__ void gemm_kc_body(const GB16Args& p) {
-  constexpr int CE = Kc<T>::CE, BK = 8 * CE, KP = BK, MPF = Kc<T>::MPF;
-  using F = typename Kc<T>::F;
+template <int BM, int BN, int WGM, int WGN, int EPI, int PW = 0>
+__global__ void __launch_bounds__(64 * (WGM * WGN + PW)) gemm_bf16_kernel(const GB16Args p) {
   constexpr int NT = 64 * WGM * WGN;  // the multiplying waves' threads
   constexpr int TM = BM / WGM, TN = BN / WGN;
   constexpr bool WS = PW > 0;                       // warp-specialized: producer and MFMA waves
   constexpr bool PP = !WS && WGM == 2 && WGN == 4;  // ping-pong main loop (8 waves, two groups of 4)
-  static_assert(!WS || (std::is_same_v<T, bf16_t> && PW == 4 &&
-                        ((BM == 256 && BN == 256 && WGM == 2 && WGN == 4) || (BM == 128 && BN == 128 && WGM == 2 && WGN == 2))),
-                "warp-specialized main loop: bf16, 256 x 256 tiles on 8 MFMA waves or 128 x 128 on 4, 4 producer waves");
+  static_assert(!WS || (PW == 4 && ((BM == 256 && BN == 256 && WGM == 2 && WGN == 4) ||
+                                    (BM == 128 && BN == 128 && WGM == 2 && WGN == 2))),
+                "warp-specialized main loop: 256 x 256 tiles on 8 MFMA waves or 128 x 128 on 4, 4 producer waves");
   constexpr int FM = TM / 16, FN = TN / 16;  // 16x16 tiles per wave along m, n
   extern __shared__ __align__(16) unsigned char smem[];
   T* const As0 = reinterpret_cast<T*>(smem);
@@ -178,18 +142,10 @@ __device__ __forceinline__ void gemm_kc_body(const GB16Args& p) {
   const int r = lane & 15, g = lane >> 4;
 
   f32x4_t acc[FM][FN];
-  // fp32 operands sum k in blocks of 128 (four k tiles) into `part`, folded into `acc` after each block, as the
-  // general fp32 engine does: one fp32 chain over all of K carries several times the rounding error against an
-  // fp64 product (measured 7.6x at K = 3072). The 128-tile configuration has the registers for the second set.
-  constexpr bool BLK = std::is_same_v<T, float>;
-  static_assert(!BLK || !PP, "blocked fp32 summation needs the 128-tile configuration");
-  constexpr int KC_TILES = 128 / BK;
-  f32x4_t part[FM][FN];
 #pragma unroll
   for (int i = 0; i < FM; ++i)
 #pragma unroll
-    for (int j = 0; j < FN; ++j) acc[i][j] = part[i][j] = f32x4_t{0.f, 0.f, 0.f, 0.f};
-  auto& dst = BLK ? part : acc;  // the MFMA accumulators of the main loop
+    for (int j = 0; j < FN; ++j) acc[i][j] = f32x4_t{0.f, 0.f, 0.f, 0.f};
   // WS: FM32 x FN32 tiles of 32 x 32 per wave (element m of lane l at row 8 (m / 4) + 4 (l / 32) + m % 4, column
   // l % 32)
   constexpr int FM32 = WS ? TM / 32 : 1, FN32 = WS ? TN / 32 : 1;
@@ -207,22 +163,9 @@ __device__ __forceinline__ void gemm_kc_body(const GB16Args& p) {
   // k tile holding m0; kb is the k origin of the first one
   const int kfirst = p.kbeg ? m0 / BK : 0, kb = kfirst * BK;
   const int nk = (K + BK - 1) / BK - kfirst;
-  // fp32 operands may be stored m- / n-contiguous (amc, bmc: the buffer's rows are k)
-  constexpr bool amc = (LAY & 1) != 0, bmc = (LAY & 2) != 0;  // a SYRK (B = A) has both bits or neither
-  static_assert(LAY == 0 || std::is_same_v<T, float>, "m/n-contiguous operands: fp32 only");
-  const __amdgpu_buffer_rsrc_t rsA =
-      make_rsrc(Ap, (long long)(amc ? K : p.M) * lda * (long long)sizeof(T));
-  const __amdgpu_buffer_rsrc_t rsB =
-      make_rsrc(Bp, (long long)(bmc ? K : (p.tri ? p.M : p.N)) * ldb * (long long)sizeof(T));
-  // acc += a b over one pair of 16-byte fragments (32 k of bf16, or 16 k of fp32 in four steps)
-  auto mma = [](f32x4_t& c, const F& a, const F& bb) {
-    if constexpr (MPF == 1) {
-      c = __builtin_amdgcn_mfma_f32_16x16x32_bf16(a, bb, c, 0, 0, 0);
-    } else {
-#pragma unroll
-      for (int s = 0; s < MPF; ++s) c = __builtin_amdgcn_mfma_f32_16x16x4f32(a[s], bb[s], c, 0, 0, 0);
-    }
-  };
+  const __amdgpu_buffer_rsrc_t rsA = make_rsrc(Ap, (long long)p.M * lda * (long long)sizeof(T));
+  const __amdgpu_buffer_rsrc_t rsB = make_rsrc(Bp, (long long)(p.tri ? p.M : p.N) * ldb * (long long)sizeof(T));
+  auto mma = [](f32x4_t& c, const F& a, const F& bb) { c = __builtin_amdgcn_mfma_f32_16x16x32_bf16(a, bb, c, 0, 0, 0); };
   const int rowsB = p.tri ? p.M : p.N;
   // 2 steps of 4 chunks per k tile from LDS (B fragments held, A fragments streamed one row ahead)
   auto mma_tile = [&](const T* As, const T* Bs) {
@@ -241,7 +184,7 @@ __device__ __forceinline__ void gemm_kc_body(const GB16Args& p) {
         if (i + 1 < FM)
           a_nxt = *reinterpret_cast<const F*>(As + (wm * TM + (i + 1) * 16 + r) * KP + ko);
 #pragma unroll
-        for (int j = 0; j < FN; ++j) mma(dst[i][j], a_cur, bfr[j]);
+        for (int j = 0; j < FN; ++j) mma(acc[i][j], a_cur, bfr[j]);
         a_cur = a_nxt;
       }
     }
@@ -281,7 +224,7 @@ __device__ __forceinline__ void gemm_kc_body(const GB16Args& p) {
       if (q + LA < NQ && q == FM / 2) __builtin_amdgcn_sched_group_barrier(0x100, FN + 1, 0);
       else if (q + LA < NQ) __builtin_amdgcn_sched_group_barrier(0x100, 1, 0);
       else if (q == FM / 2) __builtin_amdgcn_sched_group_barrier(0x100, FN, 0);
-      __builtin_amdgcn_sched_group_barrier(0x008, FN * MPF, 0);
+      __builtin_amdgcn_sched_group_barrier(0x008, FN, 0);
     }
   };
   if constexpr (WS) {
@@ -298,8 +241,8 @@ __device__ __forceinline__ void gemm_kc_body(const GB16Args& p) {
       const int t = tid - NT;
       const int voffA = (int)(((long long)(t >> 3) * lda + (t & 7) * CE) * (long long)sizeof(T));
       const int voffB = (int)(((long long)(t >> 3) * ldb + (t & 7) * CE) * (long long)sizeof(T));
-      Ld<T, BM, NTP, true> la0, la1;
-      Ld<T, BN, NTP, true> lb0, lb1;
+      Ld<BM, NTP, true> la0, la1;
+      Ld<BN, NTP, true> lb0, lb1;
       la0.load_pinned(rsA, voffA, lda, m0, p.M, kb, K, t);
       lb0.load_pinned(rsB, voffB, ldb, n0, rowsB, kb, K, t);
       la1.load_pinned(rsA, voffA, lda, m0, p.M, kb + BK, K, t);
@@ -359,19 +302,15 @@ __device__ __forceinline__ void gemm_kc_body(const GB16Args& p) {
   } else if constexpr (!PP) {
     const int voffA = (int)(((long long)(tid >> 3) * lda + (tid & 7) * CE) * (long long)sizeof(T));
     const int voffB = (int)(((long long)(tid >> 3) * ldb + (tid & 7) * CE) * (long long)sizeof(T));
-    Ld<T, BM, NT> la;
-    Ld<T, BN, NT> lb;
+    Ld<BM, NT> la;
+    Ld<BN, NT> lb;
     auto load = [&](int k0) {
-      if constexpr (amc) la.load_mc(rsA, lda, m0, p.M, k0, K, tid);
-      else la.load(rsA, voffA, lda, m0, p.M, k0, K, tid);
-      if constexpr (bmc) lb.load_mc(rsB, ldb, n0, rowsB, k0, K, tid);
-      else lb.load(rsB, voffB, ldb, n0, rowsB, k0, K, tid);
+      la.load(rsA, voffA, lda, m0, p.M, k0, K, tid);
+      lb.load(rsB, voffB, ldb, n0, rowsB, k0, K, tid);
     };
     auto store = [&](T* as, T* bs) {
-      if constexpr (amc) la.store_mc(as, tid);
-      else la.store(as, tid);
-      if constexpr (bmc) lb.store_mc(bs, tid);
-      else lb.store(bs, tid);
+      la.store(as, tid);
+      lb.store(bs, tid);
     };
     load(kb);
     store(As0, Bs0);
@@ -381,17 +320,6 @@ __device__ __forceinline__ void gemm_kc_body(const GB16Args& p) {
       const bool more = kt + 1 < nk;
       if (more) load(kb + (kt + 1) * BK);
       mma_tile(As0 + cur * BM * KP, Bs0 + cur * BN * KP);
-      if constexpr (BLK) {
-        if ((kt + 1) % KC_TILES == 0 || !more) {
-#pragma unroll
-          for (int i = 0; i < FM; ++i)
-#pragma unroll
-            for (int j = 0; j < FN; ++j) {
-              acc[i][j] += part[i][j];
-              part[i][j] = f32x4_t{0.f, 0.f, 0.f, 0.f};
-            }
-        }
-      }
       if (more) store(As0 + (cur ^ 1) * BM * KP, Bs0 + (cur ^ 1) * BN * KP);
       __syncthreads();
     }
@@ -410,8 +338,8 @@ __device__ __forceinline__ void gemm_kc_body(const GB16Args& p) {
     static_assert(BM == BN && (NT / 2) * 4 == (BM / 2) * 8, "ping-pong loader: one group loads half the rows");
     const int voffA = (int)(((long long)(t >> 3) * lda + (t & 7) * CE) * (long long)sizeof(T));
     const int voffB = (int)(((long long)(t >> 3) * ldb + (t & 7) * CE) * (long long)sizeof(T));
-    Ld<T, BM / 2, NT / 2> la;
-    Ld<T, BN / 2, NT / 2> lb;
+    Ld<BM / 2, NT / 2> la;
+    Ld<BN / 2, NT / 2> lb;
     la.load(rsA, voffA, lda, m0, p.M, kb, K, t);
     lb.load(rsB, voffB, ldb, n0, rowsB, kb, K, t);
     la.store(As0, t);
@@ -462,7 +390,6 @@ __device__ __forceinline__ void gemm_kc_body(const GB16Args& p) {
   float* __restrict__ C = p.C[b];
   bf16_t* __restrict__ Cb = p.Cb[b];
   bf16_t* __restrict__ CTb = p.CTb[b];
-  float* __restrict__ CTf = p.CT[b];
   const float* __restrict__ X1 = p.X1[b];
   const float* __restrict__ X2 = p.X2[b];
   float s0 = 0.f, s1 = 0.f;
@@ -471,13 +398,13 @@ __device__ __forceinline__ void gemm_kc_body(const GB16Args& p) {
     s0 = p.s[b][0];
   if constexpr (EPI == EPI_FACTOR || EPI == EPI_PROC || EPI == EPI_PROCB) s1 = p.s[b][1];
   const bool mirror = p.tri && p.out_mode == 1;
-  const bool colpass = CTb != nullptr || CTf != nullptr || mirror || EPI == EPI_RQ || EPI == EPI_STRACE;
+  const bool colpass = CTb != nullptr || mirror || EPI == EPI_RQ || EPI == EPI_STRACE;
   auto al = [](const void* q, int bytes) { return (reinterpret_cast<uintptr_t>(q) & (bytes - 1)) == 0; };
   const bool fast = m0 + BM <= p.M && n0 + BN <= p.N && (!p.tri || ti < tj) &&
                     (!C || ((p.ldc & 3) == 0 && al(C, 16))) && (!Cb || ((p.ldcb & 3) == 0 && al(Cb, 8))) &&
-                    (!CTb || ((p.ldct & 3) == 0 && al(CTb, 8))) && (!CTf || ((p.ldct & 3) == 0 && al(CTf, 16))) &&
+                    (!CTb || ((p.ldct & 3) == 0 && al(CTb, 8))) &&
                     (p.ldx & 3) == 0 &&
-                    (!X1 || al(X1, EPI == EPI_RQ && !std::is_same_v<T, float> ? 8 : 16)) && (!X2 || al(X2, 16));
+                    (!X1 || al(X1, EPI == EPI_RQ ? 8 : 16)) && (!X2 || al(X2, 16));
   float t1 = 0.f, t2 = 0.f;
   // one half of each wave's rows; h is a template constant so that the accumulator indices stay static (a loop
   // over h is too large to be unrolled, and a dynamic index would move the accumulators to scratch)
@@ -714,17 +641,7 @@ __device__ __forceinline__ void gemm_kc_body(const GB16Args& p) {
           ok[e] = FAST || (row + e < p.M && col < p.N && !(p.tri && row + e > col));
         }
         const bool all = ok[0] && ok[1] && ok[2] && ok[3];
-        if constexpr (EPI == EPI_RQ && std::is_same_v<T, float>) {  // X1: R in fp32, read at (col, row..row+3)
-          const float* x = X1 + (long long)col * p.ldx + row;
-          if constexpr (FAST) {
-            const float4 t = *reinterpret_cast<const float4*>(x);
-            t2 += s0 * (t.x * v[0] + t.y * v[1] + t.z * v[2] + t.w * v[3]);
-          } else {
-#pragma unroll
-            for (int e = 0; e < 4; ++e)
-              if (ok[e]) t2 += s0 * x[e] * v[e];
-          }
-        } else if constexpr (EPI == EPI_RQ) {  // X1: R in bf16, read at (col, row..row+3)
+        if constexpr (EPI == EPI_RQ) {  // X1: R in bf16, read at (col, row..row+3)
           const bf16_t* x = reinterpret_cast<const bf16_t*>(X1) + (long long)col * p.ldx + row;
           if constexpr (FAST) {
             const uint2 t = *reinterpret_cast<const uint2*>(x);
@@ -746,13 +663,6 @@ __device__ __forceinline__ void gemm_kc_body(const GB16Args& p) {
             for (int e = 0; e < 4; ++e)
               if (ok[e] && row + e < col) t2 += v[e] * x[e];
           }
-        }
-        if (CTf) {
-          float* dst = CTf + (long long)col * p.ldct + row;
-          if (FAST || (all && (p.ldct & 3) == 0)) *reinterpret_cast<float4*>(dst) = make_float4(v[0], v[1], v[2], v[3]);
-          else
-#pragma unroll
-            for (int e = 0; e < 4; ++e) if (ok[e]) dst[e] = v[e];
         }
         if (CTb) {
           bf16_t* dst = CTb + (long long)col * p.ldct + row;
@@ -837,32 +747,19 @@ __device__ __forceinline__ void gemm_kc_body(const GB16Args& p) {
   }
 }
 
-template <int BM, int BN, int WGM, int WGN, int EPI, int PW = 0>
-__global__ void __launch_bounds__(64 * (WGM * WGN + PW)) gemm_bf16_kernel(const GB16Args p) {
-  gemm_kc_body<bf16_t, BM, BN, WGM, WGN, EPI, 0, PW>(p);
-}
-
-// two workgroups per CU (two waves per SIMD): the register budget of every layout
-template <int BM, int BN, int WGM, int WGN, int EPI, int LAY>
-__global__ void __launch_bounds__(64 * WGM * WGN, 2) gemm_f32kc_kernel(const GB16Args p) {
-  gemm_kc_body<float, BM, BN, WGM, WGN, EPI, LAY>(p);
-}
-
 int gemm_bf16_tiles(long long M, long long N, int tri, int cfg) {
   const int T = cfg == 1 || cfg == 4 ? 128 : 256;
   const long long tm = (M + T - 1) / T, tn = (N + T - 1) / T;
   return (int)(tri ? tm * (tm + 1) / 2 : tm * tn);
 }
 
-template <typename T, int BM, int BN, int WGM, int WGN, int EPI, int LAY = 0, int PW = 0>
+template <int BM, int BN, int WGM, int WGN, int EPI, int PW = 0>
 static hipError_t launch_b16(GB16Args& a, hipStream_t st) {
   constexpr int NW = WGM * WGN;
   constexpr int smem_main = 2 * (BM + BN) * 128,
                 smem_epi = NW * (BM / WGM / 2) * epi_pitch(BM / WGM / 2, BN / WGN) * 4;
   constexpr int smem = smem_main > smem_epi ? smem_main : smem_epi;
-  void (*fn)(GB16Args) = nullptr;
-  if constexpr (std::is_same_v<T, bf16_t>) fn = gemm_bf16_kernel<BM, BN, WGM, WGN, EPI, PW>;
-  else fn = gemm_f32kc_kernel<BM, BN, WGM, WGN, EPI, LAY>;
+  void (*fn)(GB16Args) = gemm_bf16_kernel<BM, BN, WGM, WGN, EPI, PW>;
   // once per instantiation (a function-local static is initialised once, also under concurrent first calls)
   static const hipError_t attr =
       hipFuncSetAttribute(reinterpret_cast<const void*>(fn), hipFuncAttributeMaxDynamicSharedMemorySize, smem);
@@ -876,23 +773,19 @@ static hipError_t launch_b16(GB16Args& a, hipStream_t st) {
   return e;
 }
 
-template <typename T, int BM, int BN, int WGM, int WGN, int LAY = 0, int PW = 0>
+template <int BM, int BN, int WGM, int WGN, int PW = 0>
 static hipError_t launch_epi(GB16Args& a, hipStream_t st) {
-  constexpr bool B16 = std::is_same_v<T, bf16_t>;
   switch (a.epi) {
-    case EPI_FACTOR: return launch_b16<T, BM, BN, WGM, WGN, EPI_FACTOR, LAY, PW>(a, st);
-    case EPI_PROC: return launch_b16<T, BM, BN, WGM, WGN, EPI_PROC, LAY, PW>(a, st);
-    case EPI_SCALE: return launch_b16<T, BM, BN, WGM, WGN, EPI_SCALE, LAY, PW>(a, st);
-    case EPI_SUMSQ: return launch_b16<T, BM, BN, WGM, WGN, EPI_SUMSQ, LAY, PW>(a, st);
-    case EPI_STRACE: return launch_b16<T, BM, BN, WGM, WGN, EPI_STRACE, LAY, PW>(a, st);
-    case EPI_STORE: return launch_b16<T, BM, BN, WGM, WGN, EPI_STORE, LAY, PW>(a, st);
-    case EPI_RQ: return launch_b16<T, BM, BN, WGM, WGN, EPI_RQ, LAY, PW>(a, st);  // R read as T
-    default: break;
+    case EPI_FACTOR: return launch_b16<BM, BN, WGM, WGN, EPI_FACTOR, PW>(a, st);
+    case EPI_PROC: return launch_b16<BM, BN, WGM, WGN, EPI_PROC, PW>(a, st);
+    case EPI_SCALE: return launch_b16<BM, BN, WGM, WGN, EPI_SCALE, PW>(a, st);
+    case EPI_SUMSQ: return launch_b16<BM, BN, WGM, WGN, EPI_SUMSQ, PW>(a, st);
+    case EPI_STRACE: return launch_b16<BM, BN, WGM, WGN, EPI_STRACE, PW>(a, st);
+    case EPI_STORE: return launch_b16<BM, BN, WGM, WGN, EPI_STORE, PW>(a, st);
+    case EPI_RQ: return launch_b16<BM, BN, WGM, WGN, EPI_RQ, PW>(a, st);
+    case EPI_PROCB: return launch_b16<BM, BN, WGM, WGN, EPI_PROCB, PW>(a, st);
+    default: return hipErrorInvalidValue;
   }
-  if constexpr (B16) {  // reads a bf16 X operand
-    if (a.epi == EPI_PROCB) return launch_b16<T, BM, BN, WGM, WGN, EPI_PROCB, LAY, PW>(a, st);
-  }
-  return hipErrorInvalidValue;
 }
 
 // cfg 0: 256 x 256 tiles, 8 waves (2 per SIMD) of 128 x 64; cfg 1: 128 x 128 tiles, 4 waves of 64 x 64;
@@ -900,23 +793,11 @@ static hipError_t launch_epi(GB16Args& a, hipStream_t st) {
 // 128 x 64 on 32 x 32 x 16 MFMAs plus 4 producer waves (warp-specialized main loop); cfg 4: the same on 128 x 128
 // tiles, 4 MFMA waves of 64 x 64
 hipError_t gemm_bf16_launch(GB16Args& a, int cfg, hipStream_t st) {
-  if (cfg == 1) return launch_epi<bf16_t, 128, 128, 2, 2>(a, st);
-  if (cfg == 4) return launch_epi<bf16_t, 128, 128, 2, 2, 0, 4>(a, st);
-  if (cfg == 2) return launch_epi<bf16_t, 256, 256, 2, 2>(a, st);
-  if (cfg == 3) return launch_epi<bf16_t, 256, 256, 2, 4, 0, 4>(a, st);
-  return launch_epi<bf16_t, 256, 256, 2, 4>(a, st);
-}
-
-// fp32: the 128-tile configuration only (its waves hold the blocked-summation accumulators)
-hipError_t gemm_f32kc_launch(GB16Args& a, int cfg, hipStream_t st) {
-  (void)cfg;
-  if (a.tri && a.amc != a.bmc) return hipErrorInvalidValue;  // a SYRK reads one operand
-  switch ((a.amc ? 1 : 0) | (a.bmc ? 2 : 0)) {
-    case 1: return launch_epi<float, 128, 128, 2, 2, 1>(a, st);
-    case 2: return launch_epi<float, 128, 128, 2, 2, 2>(a, st);
-    case 3: return launch_epi<float, 128, 128, 2, 2, 3>(a, st);
-    default: return launch_epi<float, 128, 128, 2, 2, 0>(a, st);
-  }
+  if (cfg == 1) return launch_epi<128, 128, 2, 2>(a, st);
+  if (cfg == 4) return launch_epi<128, 128, 2, 2, 4>(a, st);
+  if (cfg == 2) return launch_epi<256, 256, 2, 2>(a, st);
+  if (cfg == 3) return launch_epi<256, 256, 2, 4, 4>(a, st);
+  return launch_epi<256, 256, 2, 4>(a, st);
 }
 
 }  // namespace psgdk

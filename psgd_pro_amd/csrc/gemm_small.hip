@@ -10,8 +10,7 @@
 // fragment read fall on 16 distinct bank groups; the 32 lanes that store one row still fill its 32 slots).
 // fp32 operands feed four v_mfma_f32_16x16x4f32 per 16-byte fragment pair (lane group g holds k = 4 g + s of both
 // operands) and sum k in blocks of 128 (one chunk) into a second accumulator set, as the other fp32 paths do.
-// Epilogue straight from the accumulators: C (fp32) and / or Cb (bf16) at (row, col), CTb (bf16) / CT (fp32) at
-// (col, row); a SYRK writes row <= col, and with out_mode 1 also (col, row) for row < col.
+// Epilogue straight from the accumulators: C (fp32) and / or Cb (bf16) at (row, col), CTb (bf16) at (col, row); a SYRK writes row <= col, and with out_mode 1 also (col, row) for row < col.
 #include <cstring>
 
 #include "gemm_bf16.h"
@@ -171,7 +170,6 @@ __global__ void __launch_bounds__(256) gemm_small_kernel(const GB16Args p) {
   float* __restrict__ C = p.C[b];
   bf16_t* __restrict__ Cb = p.Cb[b];
   bf16_t* __restrict__ CTb = p.CTb[b];
-  float* __restrict__ CT = p.CT[b];
   const bool mirror = p.tri && p.out_mode == 1;
 #pragma unroll
   for (int i = 0; i < 2; ++i)
@@ -185,7 +183,6 @@ __global__ void __launch_bounds__(256) gemm_small_kernel(const GB16Args p) {
         if (C) C[(long long)row * p.ldc + col] = v;
         if (Cb) Cb[(long long)row * p.ldcb + col] = f32_to_bf16(v);
         if (CTb) CTb[(long long)col * p.ldct + row] = f32_to_bf16(v);
-        if (CT) CT[(long long)col * p.ldct + row] = v;
         if (mirror && row < col) {
           if (C) C[(long long)col * p.ldc + row] = v;
           if (Cb) Cb[(long long)col * p.ldcb + row] = f32_to_bf16(v);
@@ -220,7 +217,6 @@ struct TinyArgs {
   float* C[TY_MAXB];
   bf16_t* Cb[TY_MAXB];
   bf16_t* CTb[TY_MAXB];
-  float* CT[TY_MAXB];
 };
 
 struct TyBatch {
@@ -349,7 +345,6 @@ __global__ void __launch_bounds__(256) gemm_tiny_kernel(const TinyArgs p) {
   float* __restrict__ C = p.C[b];
   bf16_t* __restrict__ Cb = p.Cb[b];
   bf16_t* __restrict__ CTb = p.CTb[b];
-  float* __restrict__ CT = p.CT[b];
   const bool mirror = p.tri && p.out_mode == 1;
 #pragma unroll
   for (int q = 0; q < 4; ++q) {
@@ -359,7 +354,6 @@ __global__ void __launch_bounds__(256) gemm_tiny_kernel(const TinyArgs p) {
     if (C) C[(long long)row * p.ldc + col] = v;
     if (Cb) Cb[(long long)row * p.ldcb + col] = f32_to_bf16(v);
     if (CTb) CTb[(long long)col * p.ldct + row] = f32_to_bf16(v);
-    if (CT) CT[(long long)col * p.ldct + row] = v;
     if (mirror && row < col) {
       if (C) C[(long long)col * p.ldc + row] = v;
       if (Cb) Cb[(long long)col * p.ldcb + row] = f32_to_bf16(v);
@@ -373,7 +367,7 @@ int gemm_tiny_tiles(long long M, long long N, int tri) {
 }
 
 hipError_t gemm_tiny_launch(const GB16Args& a, int esz, hipStream_t st) {
-  if (a.epi != EPI_STORE || a.kbeg || a.amc || a.bmc) return hipErrorInvalidValue;
+  if (a.epi != EPI_STORE || a.kbeg) return hipErrorInvalidValue;
   TinyArgs t;
   std::memset(&t, 0, sizeof t);
   t.M = a.M; t.N = a.N; t.K = a.K; t.tri = a.tri; t.out_mode = a.out_mode;
@@ -386,7 +380,7 @@ hipError_t gemm_tiny_launch(const GB16Args& a, int esz, hipStream_t st) {
     const int nb = a.nb - b0 < TY_MAXB ? a.nb - b0 : TY_MAXB;
     for (int b = 0; b < nb; ++b) {
       t.A[b] = a.A[b0 + b]; t.B[b] = a.B[b0 + b];
-      t.C[b] = a.C[b0 + b]; t.Cb[b] = a.Cb[b0 + b]; t.CTb[b] = a.CTb[b0 + b]; t.CT[b] = a.CT[b0 + b];
+      t.C[b] = a.C[b0 + b]; t.Cb[b] = a.Cb[b0 + b]; t.CTb[b] = a.CTb[b0 + b];
     }
     hipLaunchKernelGGL(fn, dim3(t.ntiles * nb), dim3(256), 0, st, t);
     const hipError_t e = hipGetLastError();
@@ -412,7 +406,7 @@ hipError_t gemm_small_launch(GB16Args& a, int esz, hipStream_t st) {
                           hipFuncAttributeMaxDynamicSharedMemorySize, smem);
   if (attr_b != hipSuccess) return attr_b;
   if (attr_f != hipSuccess) return attr_f;
-  if (a.epi != EPI_STORE || a.kbeg || a.amc || a.bmc) return hipErrorInvalidValue;
+  if (a.epi != EPI_STORE || a.kbeg) return hipErrorInvalidValue;
   a.tiles_m = (a.M + SM_T - 1) / SM_T;
   a.tiles_n = (a.N + SM_T - 1) / SM_T;
   a.ntiles = a.tri ? a.tiles_m * (a.tiles_m + 1) / 2 : a.tiles_m * a.tiles_n;

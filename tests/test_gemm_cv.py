@@ -1,0 +1,96 @@
+"""The converting MFMA engine (csrc/gemm_cv.hip): every tile configuration at the edges of its tiles, in both precisions
+and every layout it reads, against float64."""
+import pytest
+import torch
+
+from psgd_pro_amd import _lib as L
+from psgd_pro_amd import ops as K
+
+pytestmark = pytest.mark.gpu
+DEV = "cuda"
+
+
+@pytest.fixture(params=[-1, 0, 1, 2, 3])
+def engine(request):
+    """The engine alone (option 10 = 0: no small-problem kernels), in one tile configuration (option 13)."""
+    hip = L.lib()
+    L.check(hip.psgdk_set_option(13, request.param))
+    L.check(hip.psgdk_set_option(10, 0))
+    yield hip
+    L.check(hip.psgdk_set_option(13, -1))
+    L.check(hip.psgdk_set_option(10, 128))
+
+
+def _rnd(rows, cols, seed):
+    # a view one column into a wider matrix: rows that no 16-byte access is aligned to
+    x = torch.randn(rows, cols + 3, generator=torch.Generator().manual_seed(seed))
+    return x.to(DEV)[:, 1:1 + cols]
+
+
+def _check(C, A, B, bf16, what):
+    """|C - A B| <= c |A| |B| elementwise. fp32: the split drops under 2^-23 of each product, and a product takes part in
+    at most 6 roundings per 16 k of its 128-k block (a truncation counting two) and one per block, each 2^-24 of sums
+    that |A| |B| bounds. bf16: two operand
+    roundings of 2^-8 besides. (The last term: results below the smallest normal.)"""
+    A, B = A.double().cpu(), B.double().cpu()
+    u = 2.0 ** -24
+    c = u * (2 + 2 * 6 * 8 + A.shape[1] / 64 + 4) + (2.0 ** -7 + 2.0 ** -16 if bf16 else 0.0)
+    bad = (C.double().cpu() - A @ B).abs() > c * (A.abs() @ B.abs()) + 2.0 ** -126
+    assert not bad.any(), (what, int(bad.sum()))
+
+
+@pytest.mark.parametrize("m,n,k", [(1, 1, 1), (31, 63, 33), (64, 64, 64), (65, 129, 127), (129, 257, 130),
+                                   (200, 500, 321)])
+@pytest.mark.parametrize("bf16", [False, True])
+def test_converting_engine(engine, m, n, k, bf16):
+    for ta in (False, True):
+        for tb in (False, True):
+            A, B = _rnd(*((k, m) if ta else (m, k)), seed=m + k), _rnd(*((n, k) if tb else (k, n)), seed=n + k)
+            for dt in (torch.float32, torch.bfloat16):
+                a, b = A.to(dt), B.to(dt)
+                C = K.gemm(a, b, ta, tb, bf16)
+                _check(C, a.T if ta else a, b.T if tb else b, bf16, (ta, tb, dt))
+    A, S = _rnd(m, k, 1), _rnd(m, m, 2)
+    _check(K.symm(S, A, 1, bf16), torch.triu(S) + torch.triu(S, 1).T, A, bf16, "symm")
+    _check(K.symm_right(A.T, S, -1, bf16), A.T, torch.triu(S, 1) - torch.triu(S, 1).T, bf16, "symm_right")
+    _check(K.trmm(S, A, bf16), torch.triu(S), A, bf16, "trmm")
+    for trans in (False, True):
+        x = A.T if trans else A
+        full = K.syrk(A, trans, L.OUT_MIRROR, bf16)
+        assert torch.equal(full, full.T)
+        _check(full, x, x.T, bf16, "syrk")
+        i, j = torch.triu_indices(len(x), len(x))
+        assert torch.equal(K.syrk(A, trans, L.OUT_PACKED, bf16), full[i, j])
+        assert torch.equal(torch.triu(K.syrk(A, trans, L.OUT_UPPER, bf16)), torch.triu(full))
+    if bf16:
+        return
+    # rows holding an infinity, a NaN, a value over the bfloat16 range or under its normals: as on fp32 MFMAs
+    A, B = _rnd(m, k, 3).clone(), _rnd(k, n, 4)
+    for i, v in enumerate((float("inf"), float("nan"), 3.4e38, 1e-41)):
+        A[i * 9 % m, i % k] = v
+    C = K.gemm(A, B, False, False, False)
+    L.check(engine.psgdk_set_option(8, 0))
+    R = K.gemm(A, B, False, False, False)
+    L.check(engine.psgdk_set_option(8, 1))
+    fin = torch.isfinite(R)
+    assert torch.equal(fin, torch.isfinite(C)) and torch.equal(torch.isnan(R), torch.isnan(C))
+    assert torch.equal(R[torch.isinf(R)], C[torch.isinf(R)])
+    ok = fin.all(1)
+    _check(C[ok], A[ok], B, False, "finite rows")
+
+
+@pytest.mark.parametrize("cfg", [-1, 1, 3])
+def test_gram_diagonal_keeps_its_small_squares(cfg):
+    """X^T X for X near the identity: the small squares beside a diagonal entry's large one are not lost to its
+    alignment, which would lower every entry by their sum."""
+    n = 192
+    X = (torch.eye(n) + 2.0 ** -13 * torch.randn(n, n, generator=torch.Generator().manual_seed(5))).to(DEV)
+    L.check(L.lib().psgdk_set_option(13, cfg))
+    try:
+        C = K.syrk(X, True, L.OUT_MIRROR, False)
+    finally:
+        L.check(L.lib().psgdk_set_option(13, -1))
+    d = C.diagonal().double() - X.double().square().sum(0)
+    # one rounding of at most 2^-24 per entry and either sign (1 <= C_ii < 2), so a mean of n of them within 4 standard
+    # deviations 2^-24 / sqrt(3 n); the seven squares lost would make it -7 * 2^-26
+    assert d.mean().abs().item() < 4 * 2.0 ** -24 / (3 * n) ** 0.5, d.mean()
