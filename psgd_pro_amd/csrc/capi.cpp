@@ -448,8 +448,8 @@ int run_gemm(int prec, int nb, int64_t M, int64_t N, int64_t K, const Opnd& A, c
 }
 
 // ------------------------------------------------------------------------------------------------------------
-// Norm lower bound pipeline (see nlb.hip). full = the matrix is stored in full (read by contiguous loads);
-// otherwise only its upper triangle is read.
+// Norm lower bound pipeline (see nlb.hip). run_nlb reads the upper triangle only, run_nlb_full a matrix
+// stored in full.
 // tile pairs of rform (64 x 64 tiles, I <= J): its trace partials
 int64_t rform_pairs(int64_t d) {
   const int64_t T = (d + 63) / 64;
@@ -458,17 +458,17 @@ int64_t rform_pairs(int64_t d) {
 
 struct NlbWs {
   float *vb0[MAXB], *vb1[MAXB], *part[MAXB], *ss0[MAXB], *ss1[MAXB];
-  float *rpart[MAXB], *cpart[MAXB], *tmax[MAXB], *dmax[MAXB], *rn2[MAXB], *scal[MAXB];
+  float *rpart[MAXB], *cpart[MAXB], *tmax[MAXB], *rstat[MAXB], *rn2[MAXB], *scal[MAXB];
   int splits;
   int64_t kchunk;
   int64_t part_cols;  // capacity of part[b] in columns of 32 rows
 };
 
+// Split of the V A products read from the triangle: one workgroup (32 x 64 tile, one k range) per CU, k ranges of at
+// least 128 (n 2048: 8 ranges of 256, 18 us per product; 32 ranges of 64 on 1024 workgroups took 30).
 void nlb_plan(int64_t n, int nb, int& splits, int64_t& kchunk) {
-  const int tiles = (int)((n + 127) / 128);
-  int s = (512 + tiles * nb - 1) / (tiles * nb);
-  const int maxs = (int)std::max<int64_t>(1, (n + 63) / 64);
-  s = std::max(1, std::min(s, maxs));
+  const int64_t tiles = (n + 63) / 64 * nb;
+  const int64_t s = std::max<int64_t>(1, std::min((256 + tiles - 1) / tiles, n / 128));
   kchunk = ((n + s - 1) / s + 63) / 64 * 64;
   splits = (int)((n + kchunk - 1) / kchunk);
 }
@@ -498,7 +498,7 @@ void nlb_take(Ws& w, int64_t n, int nb, NlbWs& o) {
     o.rpart[b] = w.take<float>((size_t)T * T * 64);
     o.cpart[b] = w.take<float>((size_t)T * 64);
     o.tmax[b] = w.take<float>(ntri);
-    o.dmax[b] = w.take<float>(ntri);
+    o.rstat[b] = w.take<float>(2 * n);
     o.rn2[b] = w.take<float>(n);
     o.scal[b] = w.take<float>(NLB_NSCAL);
   }
@@ -514,38 +514,43 @@ NlbArgs nlb_args(int64_t n, int sign, int nb, const float* const* A, int64_t lda
   a.ssc = 64;
   for (int b = 0; b < nb; ++b) {
     a.A[b] = A[b];
-    a.rpart[b] = w.rpart[b]; a.cpart[b] = w.cpart[b]; a.tmax[b] = w.tmax[b]; a.dmax[b] = w.dmax[b];
+    a.rpart[b] = w.rpart[b]; a.cpart[b] = w.cpart[b]; a.tmax[b] = w.tmax[b]; a.rstat[b] = w.rstat[b];
     a.rn2[b] = w.rn2[b]; a.scal[b] = w.scal[b]; a.part[b] = w.part[b];
   }
   return a;
 }
 
 // One V A_sym product into the split partials.
-int nlb_vmm(int64_t n, int sign, int nb, const float* const* A, int64_t lda, bool full, float* const* Vin,
-            const NlbWs& w, hipStream_t st) {
+int nlb_vmm(int64_t n, int sign, int nb, const float* const* A, int64_t lda, float* const* Vin, const NlbWs& w,
+            hipStream_t st) {
   Opnd oa, ob;
   oa.mode = KC; oa.ld = n;
   for (int b = 0; b < nb; ++b) { oa.p[b] = Vin[b]; ob.p[b] = A[b]; }
-  ob.ld = lda;
-  if (full) { ob.mode = MC; } else { ob.mode = SYM; ob.sign = sign; }
+  ob.ld = lda; ob.mode = SYM; ob.sign = sign;
   EpiSpec e;
   float* C[MAXB];
   for (int b = 0; b < nb; ++b) C[b] = w.part[b];
   return run_gemm(PSGDK_PREC_F32, nb, NLB_K, n, n, oa, ob, C, n, e, 0, 0, 0, w.splits, w.kchunk, st);
 }
 
-int run_nlb(int64_t n, int sign, int nb, const float* const* A, int64_t lda, bool full, const float* const* V,
-            const NlbFinal& fin, const NlbWs& w, hipStream_t st) {
-  NlbArgs a = nlb_args(n, sign, nb, A, lda, w);
+// Row statistics of matrices read from their upper triangle, then (a.Vin set) V0.
+int nlb_tri_start(NlbArgs a, hipStream_t st) {
   PSGDK_HIP(nlb_rownorm_launch(a, st), "tri_rownorm");
+  for (int b = 0; b < a.nb; ++b) { a.rpart[b] = a.rstat[b]; a.cpart[b] = a.rstat[b] + a.n; }
+  return hip_check(nlb_full_launch(a, 4, 0, 0, st), "nlb_init");
+}
+
+int run_nlb(int64_t n, int sign, int nb, const float* const* A, int64_t lda, const float* const* V, const NlbFinal& fin,
+            const NlbWs& w, hipStream_t st) {
+  NlbArgs a = nlb_args(n, sign, nb, A, lda, w);
   for (int b = 0; b < nb; ++b) { a.Vin[b] = V[b]; a.Vout[b] = w.vb0[b]; }
-  PSGDK_HIP(nlb_init_launch(a, st), "nlb_init");
+  PSGDK_TRY(nlb_tri_start(a, st));
   float* const* vb[2] = {w.vb0, w.vb1};
   float* const* ss[2] = {w.ss0, w.ss1};
   // V1 = V0 A / nf; V2 = (V1/|V1|) A / nf; V3 = V2 A / nf; V4 = (V3/|V3|) A / nf
   int cur = 0;
   for (int it = 0; it < 4; ++it) {
-    PSGDK_TRY(nlb_vmm(n, sign, nb, A, lda, full, vb[cur], w, st));
+    PSGDK_TRY(nlb_vmm(n, sign, nb, A, lda, vb[cur], w, st));
     const int normalize = it & 1;
     for (int b = 0; b < nb; ++b) {
       a.Vout[b] = vb[cur ^ 1][b];
@@ -1479,7 +1484,7 @@ int factor_update_run(int prec, int nb, int64_t d, const float* const* T1, int t
     std::memset(&fin, 0, sizeof fin);
     fin.mode = NLB_FINAL_FACTOR; fin.lr = lr; fin.beta = betaL;
     for (int b = 0; b < nb; ++b) { fin.L[b] = Lv[b]; fin.coef[b] = w.coef[b]; fin.term2[b] = term2; }
-    if (t1_tri) PSGDK_TRY(run_nlb(d, 1, nb, T1, d, false, V, fin, w.nw, st));
+    if (t1_tri) PSGDK_TRY(run_nlb(d, 1, nb, T1, d, V, fin, w.nw, st));
     else PSGDK_TRY(run_nlb_full(d, 1, nb, reinterpret_cast<const void* const*>(T1), d, 0, V, fin, w.nw, st));
   }
   Opnd a, bq;
@@ -1762,9 +1767,7 @@ int psgdk_tri_rownorm2(int64_t n, int sign, int nb, const float* const* A, int64
   NlbArgs a = nlb_args(n, sign, nb, A, lda, nw);
   for (int b = 0; b < nb; ++b) { a.rn2[b] = rn2[b]; a.amax_out[b] = amax[b]; a.Vin[b] = nullptr; }
   hipStream_t st = (hipStream_t)stream;
-  PSGDK_HIP(nlb_rownorm_launch(a, st), "tri_rownorm");
-  PSGDK_HIP(nlb_init_launch(a, st), "rownorm reduce");
-  return PSGDK_OK;
+  return nlb_tri_start(a, st);
 }
 
 int psgdk_tri_vmm(int64_t n, int sign, int nb, const float* const* V, const float* const* A, int64_t lda,
@@ -1819,7 +1822,7 @@ int psgdk_norm_lower_bound(int64_t n, int sign, int nb, const float* const* A, i
   NlbFinal fin;
   std::memset(&fin, 0, sizeof fin);
   fin.mode = NLB_FINAL_NONE;
-  PSGDK_TRY(run_nlb(n, sign, nb, A, lda, false, V, fin, nw, st));
+  PSGDK_TRY(run_nlb(n, sign, nb, A, lda, V, fin, nw, st));
   for (int b = 0; b < nb; ++b)
     PSGDK_HIP(hipMemcpyAsync(out[b], nw.scal[b] + NLB_BOUND, sizeof(float), hipMemcpyDeviceToDevice, st), "copy bound");
   return PSGDK_OK;

@@ -40,7 +40,7 @@ struct NlbArgs {
   float* rpart[MAXB];       // T x T x 64 row-norm partials
   float* cpart[MAXB];       // T x 64 diagonal-tile column partials
   float* tmax[MAXB];        // per stored tile max |A_ij|
-  float* dmax[MAXB];        // per stored tile max diagonal
+  float* rstat[MAXB];       // 2 n: per row max |A_ij| (of its tile row), then the diagonal
   float* rn2[MAXB];         // n squared row norms
   float* scal[MAXB];        // NLB_NSCAL scalars
   float* amax_out[MAXB];    // optional: max |A_ij| of the stored triangle (init)
@@ -72,10 +72,10 @@ struct GramArgs {
 hipError_t gram_launch(const GramArgs& a, int stage, hipStream_t st);
 
 hipError_t nlb_rownorm_launch(const NlbArgs& a, hipStream_t st);
-hipError_t nlb_init_launch(const NlbArgs& a, hipStream_t st);
 hipError_t nlb_reduce_launch(const NlbArgs& a, int normalize_in, hipStream_t st);
 hipError_t nlb_final_launch(const NlbArgs& a, const NlbFinal& f, hipStream_t st);
 // fully stored matrices: stage 0 row norms (rn2, rpart = row max |A|, cpart = diagonal), 1 init, 2 one V A product,
+// 4 init from the upper triangle only (fp32; without Vin the row statistics' results alone),
 // 3 the stage-0 outputs of a skew matrix from the per-(row, 64-column block) partials its producer left in part
 hipError_t nlb_full_launch(const NlbArgs& a, int stage, int a_bf16, int normalize, hipStream_t st);
 hipError_t debug_mfma_launch(const float* A, const float* B, float* C, int prec, hipStream_t st);

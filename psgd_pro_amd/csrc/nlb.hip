@@ -4,9 +4,10 @@
 // V0 = a_j + sgn(<a_j, V_r>) V_r (a_j = row j of A/nf, j = the largest row), V1 = V0 A/nf, V2 = (V1/|V1|) A/nf,
 // V3 = V2 A/nf, V4 = (V3/|V3|) A/nf. Stages (each a grouped launch over up to MAXB matrices):
 //   tri_rownorm : one pass over the stored upper triangle in 64x64 tiles: per-tile row and column sums of squares
-//                 (deterministic partial slots, no float atomics), per-tile max |A_ij| and max diagonal
-//   nlb_init    : one workgroup per matrix: squared row norms, argmax (first maximum), nf, V0
-//   V A products: the GEMM engine (M = 32, B read from the triangle), split over k, partials in ws
+//                 (deterministic partial slots, no float atomics) and per-tile max |A_ij|
+//   tri_rowstats: a workgroup per 64 rows: squared row norms (partials in a fixed order), row maxima, the diagonal
+//   nlb_init    : a workgroup per (matrix, row of V): argmax (first maximum), nf, V0 (nlb_init_full_kernel)
+//   V A products: the converting engine (M = 32, B read from the triangle), split over k, partials in ws
 //   nlb_reduce  : sums the k-split partials in a fixed order, scales the rows by 1/nf and by the input row
 //                 normalisation 1/(|V_in,r| + smallest normal) (exact: the product is linear in each row of V),
 //                 and writes per-(row, column block) sums of squares of the result
@@ -19,7 +20,7 @@ constexpr int RT = 64;  // row-norm tile side
 
 // grid: nb * T(T+1)/2 workgroups of 256 threads; T = ceil(n / 64).
 // rpart[b][(X * T + Y) * 64 + i] = contribution to squared row norm 64 X + i from the stored tile pair {X, Y}.
-// tmax[b][t] = max |A_ij| over stored tile t, dmax[b][t] = max diagonal element over tile t (-inf if none).
+// tmax[b][t] = max |A_ij| over stored tile t.
 __global__ void __launch_bounds__(256) tri_rownorm_kernel(const NlbArgs p) {
   __shared__ float sq[RT][RT + 1];
   __shared__ float red[16];
@@ -33,7 +34,7 @@ __global__ void __launch_bounds__(256) tri_rownorm_kernel(const NlbArgs p) {
   const int n = p.n, tid = threadIdx.x;
   const int lr = tid >> 2, lc0 = (tid & 3) * 16;
   const int gi = I * RT + lr;
-  float rs = 0.f, am = 0.f, dm = -INFINITY;
+  float rs = 0.f, am = 0.f;
   // the 16 loads go out together: each reads a valid address (element 0 in place of one outside the stored
   // triangle) and the value is selected afterwards (a load behind a per-element branch waited for each in turn)
   float a16[16];
@@ -48,10 +49,7 @@ __global__ void __launch_bounds__(256) tri_rownorm_kernel(const NlbArgs p) {
     const int gj = J * RT + lc0 + c;
     const float v0 = a16[c];
     float v = gi < n && gj < n && gi <= gj ? v0 : 0.f;
-    if (gi == gj && gi < n) {
-      dm = fmaxf(dm, v);
-      if (p.sign < 0) v = 0.f;  // skew: the diagonal is zero by definition
-    }
+    if (gi == gj && p.sign < 0) v = 0.f;  // skew: the diagonal is zero by definition
     const float s = v * v;
     sq[lr][lc0 + c] = (gi < gj) ? s : 0.f;  // strictly-upper elements also count for the column's row norm
     rs += s;
@@ -72,117 +70,62 @@ __global__ void __launch_bounds__(256) tri_rownorm_kernel(const NlbArgs p) {
     p.cpart[b][(long long)I * RT + tid] = cs;  // diagonal tile: its column sums get a slot of their own
   }
   am = block_max(am, red);
-  dm = block_max(dm, red);
-  if (tid == 0) {
-    p.tmax[b][t] = am;
-    p.dmax[b][t] = dm;
-  }
+  if (tid == 0) p.tmax[b][t] = am;
 }
 
-// One workgroup (1024 threads) per matrix.
-__global__ void __launch_bounds__(1024) nlb_init_kernel(const NlbArgs p) {
+// The statistics nlb_init_full_kernel reads, from tri_rownorm's partials: rn2[i] (partner blocks in quarters, each summed
+// in order, then the four), rstat[i] = the largest |A_ij| over the stored tiles of row i's tile row (its maximum over all
+// rows is max |A|), rstat[n + i] = A_ii. One workgroup per 64 rows. (As part of a one-workgroup init kernel these sums,
+// n ceil(n / 64) dependent loads by one workgroup, and V0 took 70 us at n 2048; 4.5 us here and 9 us there now.)
+// grid: nb * T workgroups of 256 threads.
+__global__ void __launch_bounds__(256) tri_rowstats_kernel(const NlbArgs p) {
+  __shared__ float ps[4][RT];
   __shared__ float red[16];
-  __shared__ float sval[16];
-  __shared__ int sidx[16];
-  __shared__ float snf;
-  __shared__ int sj;
-  const int b = blockIdx.x, tid = threadIdx.x, nt = blockDim.x;
-  const int n = p.n, T = p.T, ntri = T * (T + 1) / 2;
-  const float* __restrict__ A = p.A[b];
-  const long long ld = p.lda;
-  const float* __restrict__ rp = p.rpart[b];
-  const float* __restrict__ cp = p.cpart[b];
-  float* __restrict__ rn2 = p.rn2[b];
-  // squared row norms (fixed summation order over the partner blocks) and their argmax (first maximum)
-  float best = -1.f;
-  int bi = 0x7fffffff;
-  for (int i = tid; i < n; i += nt) {
-    const int X = i / RT, li = i % RT;
-    float s = 0.f;
-    for (int Y = 0; Y < T; ++Y) s += rp[((long long)X * T + Y) * RT + li];
-    s += cp[(long long)X * RT + li];
-    rn2[i] = s;
-    if (s > best) { best = s; bi = i; }  // i increases: first maximum per thread
-  }
-  // block argmax: max value, then smallest index among equals
-  for (int o = 32; o > 0; o >>= 1) {
-    const float ov = __shfl_xor(best, o, 64);
-    const int oi = __shfl_xor(bi, o, 64);
-    if (ov > best || (ov == best && oi < bi)) { best = ov; bi = oi; }
-  }
-  if ((tid & 63) == 0) { sval[tid >> 6] = best; sidx[tid >> 6] = bi; }
-  float am = 0.f, dm = -INFINITY;
-  for (int t = tid; t < ntri; t += nt) { am = fmaxf(am, p.tmax[b][t]); dm = fmaxf(dm, p.dmax[b][t]); }
-  __syncthreads();
-  if (tid == 0) {
-    float bv = sval[0];
-    int bj = sidx[0];
-    for (int w = 1; w < nt / 64; ++w)
-      if (sval[w] > bv || (sval[w] == bv && sidx[w] < bj)) { bv = sval[w]; bj = sidx[w]; }
-    sj = bj < n ? bj : 0;
-  }
-  am = block_max(am, red);
-  dm = block_max(dm, red);
-  if (tid == 0) {
-    const float nf = (p.sign > 0 ? dm : am) + kSmallestNormal;
-    snf = nf;
-    p.scal[b][NLB_NF] = nf;
-    p.scal[b][NLB_J] = (float)sj;
-    if (p.amax_out[b]) p.amax_out[b][0] = am;
-  }
-  __syncthreads();
-  if (p.Vin[b] == nullptr) return;  // row norms only
-  const int j = sj;
-  // a_j[k] = A_sym[j][k] / nf from the triangle; V0[r] = a_j + sgn(<a_j, V_r>) V_r
-  const float* __restrict__ Vin = p.Vin[b];
-  float* __restrict__ V0 = p.Vout[b];
-  auto aj = [&](int k) -> float {
-    float v;
-    if (k > j) v = A[(long long)j * ld + k];
-    else if (k < j) v = (float)p.sign * A[(long long)k * ld + j];
-    else v = p.sign < 0 ? 0.f : A[(long long)j * ld + j];
-    return v / snf;
-  };
-  const int wave = tid >> 6, lane = tid & 63, nw = nt >> 6;
-  for (int r = wave; r < NLB_K; r += nw) {
-    float d = 0.f;
-    for (int k = lane; k < n; k += 64) d += aj(k) * Vin[(long long)r * n + k];
-    d = wave_sum(d);
-    const float sg = d > 0.f ? 1.f : (d < 0.f ? -1.f : 0.f);
-    for (int k = lane; k < n; k += 64) V0[(long long)r * n + k] = aj(k) + sg * Vin[(long long)r * n + k];
+  const int n = p.n, T = p.T, b = blockIdx.x / T, X = blockIdx.x % T;
+  const int tid = threadIdx.x, r = tid & 63, q = tid >> 6, i = X * RT + r;
+  const float* __restrict__ rp = p.rpart[b] + (long long)X * T * RT + r;
+  float s = 0.f, m = 0.f;
+#pragma unroll 8
+  for (int Y = q * T / 4; Y < (q + 1) * T / 4; ++Y) s += rp[(long long)Y * RT];
+  ps[q][r] = s;
+  const float* __restrict__ tm = p.tmax[b] + (long long)X * T - (long long)X * (X - 1) / 2;
+  for (int t = tid; t < T - X; t += 256) m = fmaxf(m, tm[t]);
+  m = block_max(m, red);
+  if (q == 0 && i < n) {
+    p.rn2[b][i] = (((ps[0][r] + ps[1][r]) + ps[2][r]) + ps[3][r]) + p.cpart[b][i];
+    p.rstat[b][i] = m;
+    p.rstat[b][n + i] = p.A[b][(long long)i * p.lda + i];
   }
 }
 
-// grid: nb * ceil(n / 64) workgroups of 256 threads (4 waves x 8 rows, 64 columns).
-// out[r][c] = rowscale_r / nf * sum_s part[s][r][c]; ss[r][cb] = sum over the block's 64 columns of out^2.
+// out[r][c] = rowscale_r / nf * sum_s part[s][r][c] (s in order); ss[r][cb] = sum over the block's 64 columns of out^2.
+// One wave per row and 64 columns, all of its loads independent (eight rows per wave, each summing its input row's
+// partials and its splits one load after the other, took 75 us at n 2048 and 32 splits; 4 us now, with 8 splits).
+// grid: nb * ceil(n / 64) * 8 workgroups of 256 threads (4 rows x 64 columns).
 __global__ void __launch_bounds__(256) nlb_reduce_kernel(const NlbArgs p, int normalize_in) {
   const int nbk = (p.n + 63) / 64;
-  const int b = blockIdx.x / nbk, cb = blockIdx.x % nbk;
-  const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
+  const int b = blockIdx.x / (nbk * 8), cb = blockIdx.x / 8 % nbk;
+  const int lane = threadIdx.x & 63, r = blockIdx.x % 8 * 4 + (threadIdx.x >> 6);
   const int n = p.n, c = cb * 64 + lane;
-  const float nf = p.scal[b][NLB_NF];
-  const float* __restrict__ part = p.part[b];
-  const float* __restrict__ ssin = p.ssin[b];
-  float* __restrict__ out = p.Vout[b];
-  float* __restrict__ ss = p.ssout[b];
-  for (int rr = 0; rr < 8; ++rr) {
-    const int r = wave * 8 + rr;
-    float sc = 1.f / nf;
-    if (normalize_in) {
-      float s = 0.f;
-      for (int q = 0; q < nbk; ++q) s += ssin[r * nbk + q];
-      sc = sc / (sqrtf(s) + kSmallestNormal);
-    }
-    float v = 0.f;
-    if (c < n) {
-      float acc = 0.f;
-      for (int s = 0; s < p.splits; ++s) acc += part[((long long)s * NLB_K + r) * n + c];
-      v = acc * sc;
-      out[(long long)r * n + c] = v;
-    }
-    const float t = wave_sum(v * v);
-    if (lane == 0) ss[r * nbk + cb] = t;
+  const float* __restrict__ part = p.part[b] + (long long)r * n + min(c, n - 1);
+  float sc = 1.f / p.scal[b][NLB_NF];
+  if (normalize_in) {
+    float s = 0.f;
+    for (int q = lane; q < nbk; q += 64) s += p.ssin[b][r * nbk + q];
+    sc = sc / (sqrtf(wave_sum(s)) + kSmallestNormal);
   }
+  float acc = 0.f;
+  for (int s0 = 0; s0 < p.splits; s0 += 8) {
+    float x[8];
+#pragma unroll
+    for (int e = 0; e < 8; ++e) x[e] = part[(long long)min(s0 + e, p.splits - 1) * NLB_K * n];
+#pragma unroll
+    for (int e = 0; e < 8; ++e) acc += s0 + e < p.splits ? x[e] : 0.f;
+  }
+  const float v = c < n ? acc * sc : 0.f;
+  if (c < n) p.Vout[b][(long long)r * n + c] = v;
+  const float t = wave_sum(v * v);
+  if (lane == 0) p.ssout[b][r * nbk + cb] = t;
 }
 
 // One workgroup (64 threads) per matrix: bound = nf * max_r |V4_r|, then the consumer's scalars.
@@ -221,15 +164,12 @@ __global__ void __launch_bounds__(64) nlb_final_kernel(const NlbArgs p, NlbFinal
 hipError_t nlb_rownorm_launch(const NlbArgs& a, hipStream_t st) {
   const int ntri = a.T * (a.T + 1) / 2;
   hipLaunchKernelGGL(tri_rownorm_kernel, dim3(ntri * a.nb), dim3(256), 0, st, a);
-  return hipGetLastError();
-}
-hipError_t nlb_init_launch(const NlbArgs& a, hipStream_t st) {
-  hipLaunchKernelGGL(nlb_init_kernel, dim3(a.nb), dim3(1024), 0, st, a);
+  hipLaunchKernelGGL(tri_rowstats_kernel, dim3(a.T * a.nb), dim3(256), 0, st, a);
   return hipGetLastError();
 }
 hipError_t nlb_reduce_launch(const NlbArgs& a, int normalize_in, hipStream_t st) {
   const int nbk = (a.n + 63) / 64;
-  hipLaunchKernelGGL(nlb_reduce_kernel, dim3(nbk * a.nb), dim3(256), 0, st, a, normalize_in);
+  hipLaunchKernelGGL(nlb_reduce_kernel, dim3(nbk * a.nb * 8), dim3(256), 0, st, a, normalize_in);
   return hipGetLastError();
 }
 hipError_t nlb_final_launch(const NlbArgs& a, const NlbFinal& f, hipStream_t st) {
@@ -357,8 +297,9 @@ __device__ __forceinline__ void store4(float* dst, const float (&x)[4]) {
 // (skew) + smallest normal, then V0[r] = a_j + sgn(<a_j, V_r>) V_r with a_j = row j of A / nf (psgd_pro.py:25-33,
 // :49-57). Workgroup r = 0 also publishes nf and j. The scans read 4 (statistics) or 8 (rows) elements per thread
 // and step with the loads of several steps in flight; the rows take the element path unless n % 8 == 0, A's row
-// stride is a multiple of 16 bytes and the bases are 16-byte aligned.
-template <typename T>
+// stride is a multiple of 16 bytes and the bases are 16-byte aligned. TRI: only A's upper triangle is read (row j's part
+// left of the diagonal from column j); without a start V the row statistics' results alone are published.
+template <typename T, bool TRI>
 __global__ void __launch_bounds__(256) nlb_init_full_kernel(const NlbArgs p) {
   __shared__ float red[4];
   __shared__ float sval[4];
@@ -372,7 +313,8 @@ __global__ void __launch_bounds__(256) nlb_init_full_kernel(const NlbArgs p) {
   const float* __restrict__ diag = p.cpart[b];
   float best = -1.f, am = 0.f, dm = -INFINITY;
   int bi = 0x7fffffff;
-  if ((n & 3) == 0) {  // workspace arrays: 256-byte aligned bases
+  // workspace arrays: 256-byte aligned bases (rn2 may be the caller's)
+  if ((n & 3) == 0 && (!TRI || (reinterpret_cast<uintptr_t>(rn2) & 15) == 0)) {
     const int n4 = n >> 2;
 #pragma unroll 4
     for (int i = tid; i < n4; i += 256) {
@@ -413,8 +355,10 @@ __global__ void __launch_bounds__(256) nlb_init_full_kernel(const NlbArgs p) {
     if (r == 0) {
       p.scal[b][NLB_NF] = nf;
       p.scal[b][NLB_J] = (float)sj;
+      if (TRI && p.amax_out[b]) p.amax_out[b][0] = am;
     }
   }
+  if (TRI && !p.Vin[b]) return;
   __syncthreads();
   const T* __restrict__ arow = reinterpret_cast<const T*>(p.A[b]) + (long long)sj * p.lda;
   const int j = sj;
@@ -423,10 +367,15 @@ __global__ void __launch_bounds__(256) nlb_init_full_kernel(const NlbArgs p) {
   T* __restrict__ v0 = reinterpret_cast<T*>(p.Vout[b]);
   // element k of row r of V0: row-major, or in 16-column blocks (vblk)
   auto vat = [&](int k) { return p.vblk ? ((long long)(k >> 4) * NLB_K + r) * 16 + (k & 15) : (long long)r * n + k; };
-  const bool vec = (n & 7) == 0 && (p.lda * (long long)sizeof(T)) % 16 == 0 &&
+  const bool vec = !TRI && (n & 7) == 0 && (p.lda * (long long)sizeof(T)) % 16 == 0 &&
                    (reinterpret_cast<uintptr_t>(p.A[b]) & 15) == 0 && (reinterpret_cast<uintptr_t>(p.Vin[b]) & 15) == 0 &&
                    (reinterpret_cast<uintptr_t>(p.Vout[b]) & 15) == 0;
   auto aval = [&](float a, int k) { return (p.sign < 0 && k == j ? 0.f : a) / nf; };
+  auto aelem = [&](int k) {
+    if (!TRI) return to_f32<T>(arow[k]);
+    const float a = to_f32<T>(reinterpret_cast<const T*>(p.A[b])[k < j ? (long long)k * p.lda + j : (long long)j * p.lda + k]);
+    return k < j && p.sign < 0 ? -a : a;
+  };
   float d = 0.f;
   if (vec) {
 #pragma unroll 2
@@ -438,7 +387,8 @@ __global__ void __launch_bounds__(256) nlb_init_full_kernel(const NlbArgs p) {
       for (int e = 0; e < 8; ++e) d += aval(a[e], 8 * c + e) * v[e];
     }
   } else {
-    for (int k = tid; k < n; k += 256) d += aval(to_f32<T>(arow[k]), k) * vr[k];
+#pragma unroll 4
+    for (int k = tid; k < n; k += 256) d += aval(aelem(k), k) * vr[k];
   }
   d = block_sum(d, red);
   const float sg = d > 0.f ? 1.f : (d < 0.f ? -1.f : 0.f);
@@ -453,7 +403,8 @@ __global__ void __launch_bounds__(256) nlb_init_full_kernel(const NlbArgs p) {
       store8(v0 + vat(8 * c), a);  // 8 columns inside one 16-column block
     }
   } else {
-    for (int k = tid; k < n; k += 256) v0[vat(k)] = from_f32<T>(aval(to_f32<T>(arow[k]), k) + sg * vr[k]);
+#pragma unroll 4
+    for (int k = tid; k < n; k += 256) v0[vat(k)] = from_f32<T>(aval(aelem(k), k) + sg * vr[k]);
   }
 }
 
@@ -1239,8 +1190,11 @@ hipError_t nlb_full_launch(const NlbArgs& a, int stage, int a_bf16, int normaliz
     if (a_bf16) hipLaunchKernelGGL(rownorm_full_kernel<bf16_t>, dim3(nrb * a.nb), dim3(256), 0, st, a);
     else hipLaunchKernelGGL(rownorm_full_kernel<float>, dim3(nrb * a.nb), dim3(256), 0, st, a);
   } else if (stage == 1) {
-    if (a_bf16) hipLaunchKernelGGL(nlb_init_full_kernel<bf16_t>, dim3(a.nb * NLB_K), dim3(256), 0, st, a);
-    else hipLaunchKernelGGL(nlb_init_full_kernel<float>, dim3(a.nb * NLB_K), dim3(256), 0, st, a);
+    const dim3 grid(a.nb * NLB_K);
+    if (a_bf16) hipLaunchKernelGGL((nlb_init_full_kernel<bf16_t, false>), grid, dim3(256), 0, st, a);
+    else hipLaunchKernelGGL((nlb_init_full_kernel<float, false>), grid, dim3(256), 0, st, a);
+  } else if (stage == 4) {
+    hipLaunchKernelGGL((nlb_init_full_kernel<float, true>), dim3(a.nb * (a.Vin[0] ? NLB_K : 1)), dim3(256), 0, st, a);
   } else if (a.vmm_cols) {
     const dim3 grid(((a.n + VMC - 1) / VMC) * a.nb);
     if (a.vmm_cols == 3) {  // bf16, square, n a multiple of 128 (an even number of 64-tiles)
