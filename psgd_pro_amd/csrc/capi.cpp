@@ -487,7 +487,7 @@ void nlb_full_plan(int64_t n, int nb, int64_t part_cols, int& ksplit, int& kslic
 
 void nlb_take(Ws& w, int64_t n, int nb, NlbWs& o) {
   nlb_plan(n, nb, o.splits, o.kchunk);
-  const int64_t T = (n + 63) / 64, nbk = T, ntri = T * (T + 1) / 2;
+  const int64_t T = (n + 63) / 64, nbk = (n + 15) / 16, ntri = T * (T + 1) / 2;
   o.part_cols = std::max<int64_t>(o.splits, 8) * n;
   for (int b = 0; b < nb; ++b) {
     o.vb0[b] = w.take<float>(NLB_K * n);
@@ -521,8 +521,8 @@ NlbArgs nlb_args(int64_t n, int sign, int nb, const float* const* A, int64_t lda
 }
 
 // One V A_sym product into the split partials.
-int nlb_vmm(int64_t n, int sign, int nb, const float* const* A, int64_t lda, float* const* Vin, const NlbWs& w,
-            hipStream_t st) {
+int nlb_vmm(int64_t n, int sign, int nb, const float* const* A, int64_t lda, const float* const* Vin,
+            const NlbWs& w, hipStream_t st) {
   Opnd oa, ob;
   oa.mode = KC; oa.ld = n;
   for (int b = 0; b < nb; ++b) { oa.p[b] = Vin[b]; ob.p[b] = A[b]; }
@@ -540,31 +540,6 @@ int nlb_tri_start(NlbArgs a, hipStream_t st) {
   return hip_check(nlb_full_launch(a, 4, 0, 0, st), "nlb_init");
 }
 
-int run_nlb(int64_t n, int sign, int nb, const float* const* A, int64_t lda, const float* const* V, const NlbFinal& fin,
-            const NlbWs& w, hipStream_t st) {
-  NlbArgs a = nlb_args(n, sign, nb, A, lda, w);
-  for (int b = 0; b < nb; ++b) { a.Vin[b] = V[b]; a.Vout[b] = w.vb0[b]; }
-  PSGDK_TRY(nlb_tri_start(a, st));
-  float* const* vb[2] = {w.vb0, w.vb1};
-  float* const* ss[2] = {w.ss0, w.ss1};
-  // V1 = V0 A / nf; V2 = (V1/|V1|) A / nf; V3 = V2 A / nf; V4 = (V3/|V3|) A / nf
-  int cur = 0;
-  for (int it = 0; it < 4; ++it) {
-    PSGDK_TRY(nlb_vmm(n, sign, nb, A, lda, vb[cur], w, st));
-    const int normalize = it & 1;
-    for (int b = 0; b < nb; ++b) {
-      a.Vout[b] = vb[cur ^ 1][b];
-      a.ssin[b] = ss[0][b];
-      a.ssout[b] = ss[normalize][b];
-    }
-    PSGDK_HIP(nlb_reduce_launch(a, normalize, st), "nlb_reduce");
-    cur ^= 1;
-  }
-  for (int b = 0; b < nb; ++b) a.ssin[b] = ss[1][b];
-  PSGDK_HIP(nlb_final_launch(a, fin, st), "nlb_final");
-  return PSGDK_OK;
-}
-
 // Norm lower bound of fully stored matrices (fp32 or bf16): row norms, init, 4 V A products with folded scaling,
 // final. 7 launches.
 // The column-block V A kernel needs the 16-byte operand layout (n and the row stride multiples of 16 bytes,
@@ -575,6 +550,49 @@ bool vmm_cols_ok(int64_t n, int nb, const void* const* A, int64_t lda, int esz, 
   for (int b = 0; b < nb; ++b)
     if (!aligned16(A[b]) || !aligned16(w.vb0[b]) || !aligned16(w.vb1[b])) return false;
   return true;
+}
+
+// The four products of a bound, V1 = V0 A / nf; V2 = (V1/|V1|) A / nf; V3 = V2 A / nf; V4 = (V3/|V3|) A / nf, each by
+// product(a, normalize) into a.Vout and a.ssout, then the bound. V0 is in w.vb0.
+template <typename P>
+int nlb_iterate(NlbArgs a, const NlbFinal& fin, const NlbWs& w, hipStream_t st, P product) {
+  float* const* vb[2] = {w.vb0, w.vb1};
+  float* const* ss[2] = {w.ss0, w.ss1};
+  int cur = 0;
+  for (int it = 0; it < 4; ++it) {
+    const int normalize = it & 1;
+    for (int b = 0; b < a.nb; ++b) {
+      a.Vin[b] = vb[cur][b];
+      a.Vout[b] = vb[cur ^ 1][b];
+      a.ssin[b] = ss[0][b];
+      a.ssout[b] = ss[normalize][b];
+    }
+    PSGDK_TRY(product(a, normalize));
+    cur ^= 1;
+  }
+  for (int b = 0; b < a.nb; ++b) a.ssin[b] = ss[1][b];
+  return hip_check(nlb_final_launch(a, fin, st), "nlb_final");
+}
+
+// Bounds of matrices read from their upper triangle only: the 16-column kernel where it can read them, else split-K
+// products on the converting engine.
+int run_nlb(int64_t n, int sign, int nb, const float* const* A, int64_t lda, const float* const* V, const NlbFinal& fin,
+            const NlbWs& w, hipStream_t st) {
+  NlbArgs a = nlb_args(n, sign, nb, A, lda, w);
+  for (int b = 0; b < nb; ++b) { a.Vin[b] = V[b]; a.Vout[b] = w.vb0[b]; }
+  PSGDK_TRY(nlb_tri_start(a, st));
+  const void* Av[MAXB];
+  for (int b = 0; b < nb; ++b) Av[b] = A[b];
+  if (vmm_cols_ok(n, nb, Av, lda, 4, w)) {
+    a.vmm_cols = 4; a.tri = 1; a.ssc = 16;
+    return nlb_iterate(a, fin, w, st, [&](const NlbArgs& p, int normalize) {
+      return hip_check(nlb_full_launch(p, 2, 0, normalize, st), "V A");
+    });
+  }
+  return nlb_iterate(a, fin, w, st, [&](const NlbArgs& p, int normalize) {
+    PSGDK_TRY(nlb_vmm(n, sign, nb, A, lda, p.Vin, w, st));
+    return hip_check(nlb_reduce_launch(p, normalize, st), "nlb_reduce");
+  });
 }
 
 // stats_in_part: the producer of the (skew) matrices left per-(row, column block) row statistics in w.part
@@ -592,30 +610,20 @@ int run_nlb_full(int64_t n, int sign, int nb, const void* const* A, int64_t lda,
   // workgroups; smaller sets ran faster on the row kernel (measured crossovers), and option 4 = 3 forces it.
   const bool tri_ok = a.vmm_cols == 2 && a_bf16 && n % 128 == 0;
   if (tri_ok && (g_vmm_cols == 3 || (g_vmm_cols == -1 && nb >= 16 && (int64_t)nb * (n / 64) >= 512))) a.vmm_cols = 3;
+  // launches of the row kernel that would fill at most half of the CUs: 16 columns per workgroup instead of 64 (whole
+  // bounds, us, 64 -> 16 columns: fp32 n 1024 80 -> 51, two of 4096 (128 workgroups) 248 -> 219, twelve of 768 (144)
+  // 101 -> 120; bf16 1024 50 -> 39, two of 4096 132 -> 125, twelve of 768 72 -> 82)
+  else if (a.vmm_cols == 2 && g_vmm_cols == -1 && (int64_t)nb * ((n + 63) / 64) <= 128) a.vmm_cols = 4;
   a.vblk = a.vmm_cols == 3;  // the upper-tile kernel's V layout, from the init kernel on
-  a.ssc = a.vmm_cols ? 64 : 128;
+  a.ssc = a.vmm_cols == 4 ? 16 : a.vmm_cols ? 64 : 128;
   if (a.vmm_cols && a.vmm_u == 8) a.vmm_u = 4;
   if (stats_in_part) PSGDK_HIP(nlb_full_launch(a, 3, a_bf16, 0, st), "row norms from partials");
   else PSGDK_HIP(nlb_full_launch(a, 0, a_bf16, 0, st), "row norms");
   for (int b = 0; b < nb; ++b) { a.Vin[b] = V[b]; a.Vout[b] = w.vb0[b]; }
   PSGDK_HIP(nlb_full_launch(a, 1, a_bf16, 0, st), "nlb init");
-  float* const* vb[2] = {w.vb0, w.vb1};
-  float* const* ss[2] = {w.ss0, w.ss1};
-  int cur = 0;
-  for (int it = 0; it < 4; ++it) {
-    const int normalize = it & 1;
-    for (int b = 0; b < nb; ++b) {
-      a.Vin[b] = vb[cur][b];
-      a.Vout[b] = vb[cur ^ 1][b];
-      a.ssin[b] = ss[0][b];
-      a.ssout[b] = ss[normalize][b];
-    }
-    PSGDK_HIP(nlb_full_launch(a, 2, a_bf16, normalize, st), "V A");
-    cur ^= 1;
-  }
-  for (int b = 0; b < nb; ++b) a.ssin[b] = ss[1][b];
-  PSGDK_HIP(nlb_final_launch(a, fin, st), "nlb_final");
-  return PSGDK_OK;
+  return nlb_iterate(a, fin, w, st, [&](const NlbArgs& p, int normalize) {
+    return hip_check(nlb_full_launch(p, 2, a_bf16, normalize, st), "V A");
+  });
 }
 
 // The SPD bound of term1 = Pc Pc^T (d x d) from its factor Pc (d x k bf16 rows; Pr = Pc^T, k x d rows), without

@@ -19,8 +19,9 @@ struct NlbArgs {
   int vmm_cols;             // full path: 1 = one workgroup per 64 output columns over the whole k range (no
                             // partials, ssc = 64); 2 = the same with A staged through LDS in row-contiguous
                             // runs; 3 = square bf16 matrices read from their upper 64-tiles in
-                            // tournament-paired rounds (ssc = 64); 0 = split-K products plus a reduce kernel
-                            // (ssc = 128)
+                            // tournament-paired rounds (ssc = 64); 4 = one workgroup per 16 columns (ssc = 16);
+                            // 0 = split-K products plus a reduce kernel (ssc = 128)
+  int tri;                  // vmm_cols 4: A is read from its upper triangle (fp32)
   int kdim;                 // column kernel: k extent of a rectangular product (0: n)
   int vblk;                 // init and upper-tile kernels: V (32 x n) stored in 16-column blocks, element (r, c)
                             // at ((c / 16) 32 + r) 16 + c % 16, so that a wave's MFMA fragment of 32 rows x 16 k

@@ -7,7 +7,8 @@
 //                 (deterministic partial slots, no float atomics) and per-tile max |A_ij|
 //   tri_rowstats: a workgroup per 64 rows: squared row norms (partials in a fixed order), row maxima, the diagonal
 //   nlb_init    : a workgroup per (matrix, row of V): argmax (first maximum), nf, V0 (nlb_init_full_kernel)
-//   V A products: the converting engine (M = 32, B read from the triangle), split over k, partials in ws
+//   V A products: vmm_strip_kernel; for operands it cannot read, the converting engine (M = 32, B read from the
+//                 triangle), split over k, partials in ws, and
 //   nlb_reduce  : sums the k-split partials in a fixed order, scales the rows by 1/nf and by the input row
 //                 normalisation 1/(|V_in,r| + smallest normal) (exact: the product is linear in each row of V),
 //                 and writes per-(row, column block) sums of squares of the result
@@ -128,18 +129,18 @@ __global__ void __launch_bounds__(256) nlb_reduce_kernel(const NlbArgs p, int no
   if (lane == 0) p.ssout[b][r * nbk + cb] = t;
 }
 
-// One workgroup (64 threads) per matrix: bound = nf * max_r |V4_r|, then the consumer's scalars.
-__global__ void __launch_bounds__(64) nlb_final_kernel(const NlbArgs p, NlbFinal f) {
+// One workgroup per matrix, 16 threads per row of V: bound = nf * max_r |V4_r|, then the consumer's scalars. (One
+// thread per row read its ceil(n / ssc) partials one after the other: 22 us at n 3072.)
+__global__ void __launch_bounds__(16 * NLB_K) nlb_final_kernel(const NlbArgs p, NlbFinal f) {
+  __shared__ float red[16];
   const int b = blockIdx.x, lane = threadIdx.x;
   const int nbk = (p.n + p.ssc - 1) / p.ssc;
-  const float* __restrict__ ss = p.ssin[b];
-  float m = 0.f;
-  if (lane < NLB_K) {
-    float s = 0.f;
-    for (int q = 0; q < nbk; ++q) s += ss[lane * nbk + q];
-    m = sqrtf(s);
-  }
-  m = wave_max(m);
+  const float* __restrict__ ss = p.ssin[b] + (lane >> 4) * nbk;
+  float s = 0.f;
+#pragma unroll 4
+  for (int q = lane & 15; q < nbk; q += 16) s += ss[q];
+  for (int o = 1; o < 16; o <<= 1) s += __shfl_xor(s, o, 64);
+  const float m = block_max(fmaxf(sqrtf(s), 0.f), red);  // a row of NaN counts as zero
   if (lane == 0) {
     const float nf = p.scal[b][NLB_NF];
     const float bound = nf * m;
@@ -173,7 +174,7 @@ hipError_t nlb_reduce_launch(const NlbArgs& a, int normalize_in, hipStream_t st)
   return hipGetLastError();
 }
 hipError_t nlb_final_launch(const NlbArgs& a, const NlbFinal& f, hipStream_t st) {
-  hipLaunchKernelGGL(nlb_final_kernel, dim3(a.nb), dim3(64), 0, st, a, f);
+  hipLaunchKernelGGL(nlb_final_kernel, dim3(a.nb), dim3(16 * NLB_K), 0, st, a, f);
   return hipGetLastError();
 }
 
@@ -943,6 +944,150 @@ __global__ void __launch_bounds__(256) vmm_rows_kernel(const NlbArgs p, int norm
   }
 }
 
+// The product of vmm_rows_kernel on narrow column blocks: one workgroup of 8 waves per 16 output columns, for launches
+// whose 64-column blocks would leave CUs idle (n 1024: 64 workgroups instead of 16; every workgroup reads all of V, 32
+// rows against its 16 of A, from L2). The k range goes through LDS in chunks of 2 KB per row; wave w multiplies the k
+// eighth w of a chunk (4 MFMA steps, V fragments straight from global memory); the next chunk's loads are in flight
+// meanwhile. The waves' partial blocks are summed through LDS in the order w = 0..7.
+// TRI (fp32): A is read from its upper triangle. Column c's k below the block's first column c0 are stored in rows k:
+// chunks of 512 rows x 16 columns, [k][c] in LDS (rows of 20 floats: the 64 lanes of a fragment read hit 64 banks),
+// negated for skew matrices; from c0 on they are stored in row c, and the 16 x 16 block at the diagonal is completed in
+// LDS from its upper half. (A_sym^T is what is multiplied, as by the kernels that read rows in full.)
+// Latency-bound at these sizes: about 8 us per product of n 2048 fp32 from full storage (21 on 64-column blocks), 13 from
+// the triangle (18 and a 4 us reduce by split-K products).
+// Same operand contract as vmm_cols_kernel. grid: nb * ceil(n / 16).
+constexpr int VS_C = 16, VS_LD = 20;  // columns per workgroup; row pitch (floats) of a [k][c] chunk
+
+template <typename T, bool TRI>
+__global__ void __launch_bounds__(512, 4) vmm_strip_kernel(const NlbArgs p, int normalize) {
+  constexpr int CE = 16 / sizeof(T), CK = 2048 / sizeof(T);  // elements per 16-byte piece; k per chunk
+  constexpr int KS = 4 * CE;                                 // k per MFMA step
+  static_assert(!TRI || sizeof(T) == 4, "triangles are fp32");
+  __shared__ __attribute__((aligned(16))) unsigned char sm[TRI ? CK * VS_LD * 4 : VS_C * 2048];
+  __shared__ float rsl[NLB_K];
+  const int n = p.n, nbk = (n + VS_C - 1) / VS_C;
+  const int b = blockIdx.x / nbk, cb = blockIdx.x % nbk, c0 = cb * VS_C;
+  const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+  const int r16 = lane & 15, g = lane >> 4;
+  const T* __restrict__ V = reinterpret_cast<const T*>(p.Vin[b]);
+  const __amdgpu_buffer_rsrc_t rv = make_rsrc(V, (long long)NLB_K * n * sizeof(T));
+  const __amdgpu_buffer_rsrc_t ra = make_rsrc(p.A[b], (long long)n * p.lda * sizeof(T));
+  const int lda = (int)p.lda;
+  uint4 st[4], vn[4][2];
+  // chunk of k kc .. kc + CK - 1, none at or past kend: A's rows c0 .. (piece tid % 128 of rows tid / 128 + 4 i), or
+  // (cols) rows kc .. (piece tid % 4 of rows tid / 4 + 128 i)
+  auto load = [&](int kc, int kend, bool cols) {
+#pragma unroll
+    for (int i = 0; i < 4; ++i) {
+      const int row = cols ? kc + (tid >> 2) + 128 * i : c0 + (tid >> 7) + 4 * i;
+      const int col = cols ? c0 + (tid & 3) * CE : kc + (tid & 127) * CE;
+      const bool in = cols ? row < kend && col < n : row < n && col < kend;
+      st[i] = __builtin_bit_cast(
+          uint4, __builtin_amdgcn_raw_buffer_load_b128(ra, in ? (row * lda + col) * (int)sizeof(T) : kOob, 0, 0));
+    }
+#pragma unroll
+    for (int s = 0; s < 4; ++s) {
+      const int k = kc + wave * (CK / 8) + s * KS + g * CE;
+#pragma unroll
+      for (int i = 0; i < 2; ++i)
+        vn[s][i] = __builtin_bit_cast(uint4, __builtin_amdgcn_raw_buffer_load_b128(
+                                                 rv, k < kend ? ((i * 16 + r16) * n + k) * (int)sizeof(T) : kOob, 0, 0));
+    }
+  };
+  f32x4_t acc[2] = {};
+  const int split = TRI ? c0 : 0;  // k below it are read from rows k
+  bool cols = split > 0;
+  int kc = 0;
+  load(0, cols ? split : n, cols);
+  {  // row scales: 16 threads per row
+    const int r = tid >> 4, q0 = tid & 15;
+    float sc = 1.f / p.scal[b][NLB_NF];
+    if (normalize) {
+      float s = 0.f;
+      for (int q = q0; q < nbk; q += 16) s += p.ssin[b][r * nbk + q];
+      for (int o = 1; o < 16; o <<= 1) s += __shfl_xor(s, o, 64);
+      sc = sc / (sqrtf(s) + kSmallestNormal);
+    }
+    if (q0 == 0) rsl[r] = sc;
+  }
+  while (true) {
+    uint4 vc[4][2];
+#pragma unroll
+    for (int s = 0; s < 4; ++s)
+#pragma unroll
+      for (int i = 0; i < 2; ++i) vc[s][i] = vn[s][i];
+#pragma unroll
+    for (int i = 0; i < 4; ++i) {
+      const int row = (tid >> 7) + 4 * i;
+      if (cols) *reinterpret_cast<uint4*>(sm + (((tid >> 2) + 128 * i) * VS_LD + (tid & 3) * 4) * 4) = st[i];
+      else *reinterpret_cast<uint4*>(sm + row * 2048 + ((tid & 127) ^ row) * 16) = st[i];
+    }
+    __syncthreads();
+    const bool now_cols = cols, diag = TRI && !cols && kc == split;
+    kc += CK;
+    if (cols && kc >= split) { cols = false; kc = split; }
+    const bool more = kc < n;
+    if (more) load(kc, cols ? split : n, cols);
+    if constexpr (TRI) {
+      if (diag) {  // the 16 x 16 block of rows c0 .. at k = c0 ..: its lower half from its upper one
+        float* const D = reinterpret_cast<float*>(sm);
+        auto at = [&](int i, int j) -> float& { return D[i * 512 + ((j >> 2) ^ i) * 4 + (j & 3)]; };
+        const int i = tid >> 4, j = tid & 15;
+        if (tid < 256) {
+          if (j < i) at(i, j) = p.sign < 0 ? -at(j, i) : at(j, i);
+          else if (j == i && p.sign < 0) at(i, i) = 0.f;
+        }
+        __syncthreads();
+      }
+    }
+#pragma unroll
+    for (int s = 0; s < 4; ++s) {
+      const int piece = wave * 16 + s * 4 + g;  // 16-byte piece of the row this lane's fragment reads
+      uint4 af;
+      if (TRI && now_cols) {
+        const float* const q = reinterpret_cast<const float*>(sm) + piece * 4 * VS_LD + r16;
+        const uint32_t flip = p.sign < 0 ? 0x80000000u : 0u;
+        af = make_uint4(__float_as_uint(q[0]) ^ flip, __float_as_uint(q[VS_LD]) ^ flip,
+                        __float_as_uint(q[2 * VS_LD]) ^ flip, __float_as_uint(q[3 * VS_LD]) ^ flip);
+      } else {
+        af = *reinterpret_cast<const uint4*>(sm + r16 * 2048 + (piece ^ r16) * 16);
+      }
+      if constexpr (sizeof(T) == 2) {
+#pragma unroll
+        for (int i = 0; i < 2; ++i)
+          acc[i] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(__builtin_bit_cast(bf16x8_t, vc[s][i]),
+                                                           __builtin_bit_cast(bf16x8_t, af), acc[i], 0, 0, 0);
+      } else {
+#pragma unroll
+        for (int s4 = 0; s4 < 4; ++s4)
+#pragma unroll
+          for (int i = 0; i < 2; ++i)
+            acc[i] = __builtin_amdgcn_mfma_f32_16x16x4f32(__uint_as_float((&vc[s][i].x)[s4]),
+                                                          __uint_as_float((&af.x)[s4]), acc[i], 0, 0, 0);
+      }
+    }
+    __syncthreads();
+    if (!more) break;
+  }
+  // lane holds rows 16 i + 4 g + e of column r16; thread t of the sum: row t / 16, column t % 16
+  float (*red)[NLB_K][VS_LD] = reinterpret_cast<float (*)[NLB_K][VS_LD]>(sm);
+  static_assert(8 * NLB_K * VS_LD * 4 <= sizeof sm, "the partial blocks fit in the staging buffer");
+#pragma unroll
+  for (int i = 0; i < 2; ++i)
+#pragma unroll
+    for (int e = 0; e < 4; ++e) red[wave][16 * i + 4 * g + e][r16] = acc[i][e];
+  __syncthreads();
+  const int row = tid >> 4, c = tid & 15;
+  float w = red[0][row][c];
+#pragma unroll
+  for (int q = 1; q < 8; ++q) w += red[q][row][c];
+  w = c0 + c < n ? w * rsl[row] : 0.f;
+  if (c0 + c < n) reinterpret_cast<T*>(p.Vout[b])[(long long)row * n + c0 + c] = from_f32<T>(w);
+  float sq = w * w;
+  for (int o = 1; o < 16; o <<= 1) sq += __shfl_xor(sq, o, 64);
+  if (c == 0) p.ssout[b][row * nbk + cb] = sq;
+}
+
 // ---------------------------------------------------------------------------------------------------------------
 // Norm bound of term1 = P P^T from its factor P (d x k, k < d / 2 on the bf16 update's Pg route). With H = P^T P:
 // ||row i of P P^T||^2 = P_i H P_i^T = sum_c (P H)_ic P_ic, (P P^T)_ii = ||P_i||^2, row j of P P^T = P P_j^T.
@@ -1197,7 +1342,12 @@ hipError_t nlb_full_launch(const NlbArgs& a, int stage, int a_bf16, int normaliz
     hipLaunchKernelGGL((nlb_init_full_kernel<float, true>), dim3(a.nb * (a.Vin[0] ? NLB_K : 1)), dim3(256), 0, st, a);
   } else if (a.vmm_cols) {
     const dim3 grid(((a.n + VMC - 1) / VMC) * a.nb);
-    if (a.vmm_cols == 3) {  // bf16, square, n a multiple of 128 (an even number of 64-tiles)
+    if (a.vmm_cols == 4) {
+      const dim3 gs(((a.n + VS_C - 1) / VS_C) * a.nb);
+      if (a.tri) hipLaunchKernelGGL((vmm_strip_kernel<float, true>), gs, dim3(512), 0, st, a, normalize);
+      else if (a_bf16) hipLaunchKernelGGL((vmm_strip_kernel<bf16_t, false>), gs, dim3(512), 0, st, a, normalize);
+      else hipLaunchKernelGGL((vmm_strip_kernel<float, false>), gs, dim3(512), 0, st, a, normalize);
+    } else if (a.vmm_cols == 3) {  // bf16, square, n a multiple of 128 (an even number of 64-tiles)
       const int T = a.n / VMC;
       hipLaunchKernelGGL(vmm_tri_kernel, dim3(8 * ((a.nb + 7) / 8) * T), dim3(256), 0, st, a, normalize);
     } else if (a.vmm_cols == 2) {
