@@ -301,10 +301,10 @@ int run_b16(int nb, int64_t M, int64_t N, int64_t K, const void* const* A, int64
   const int cfg = b16_cfg(M, N, K, tri, nb, e.epi);
   // a plain store whose 128-tiles would leave most of the chip idle: the small-problem kernel (64-tiles, k in
   // 512-byte chunks, two in flight). Measured crossovers against the pipelined kernels (launch of nb problems, in
-  // 128-tiles): bf16 GEMMs about 130, bf16 SYRKs (whose triangle the 64-tiles follow more closely) about 200.
+  // 128-tiles): about 130 for products and for SYRKs (one SYRK, k = n, small against pipelined: n 1792, 105 tiles, 19.4
+  // us against 22.0; n 2048, 136 tiles, 32.0 against 24.2; n 2304, k 768, 171 tiles, 16.5 against 15.1).
   const int64_t t128 = (int64_t)gemm_bf16_tiles(M, N, tri, 1) * nb;
-  const int64_t small_max = tri ? 3 * (int64_t)g_small / 2 : g_small;
-  const bool small = esz == 4 || (e.epi == EPI_STORE && !kbeg && !kper && g_force_cfg < 0 && t128 < small_max);
+  const bool small = esz == 4 || (e.epi == EPI_STORE && !kbeg && !kper && g_force_cfg < 0 && t128 < g_small);
   // ... and one whose 64-tiles would still fill only a fraction of the CUs: the tiny-product kernel
   const bool tiny = small && (int64_t)gemm_small_tiles(M, N, tri) * nb < g_tiny;
   if (ntiles)
