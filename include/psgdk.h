@@ -334,8 +334,9 @@ int psgdk_profile_stop(psgdk_prof_record_t* out, int max_records, int* n_records
  * waves; other values are refused); option 2 = workgroups
  * per split-K V A product of the norm lower bound (default 1024); option 3 = MFMA steps per load batch of the V A
  * kernels (2, 4 or 8; default 4; the column-block kernel takes 2 or 4); option 4 = the V A kernel of full-storage
- * norm bounds (-1 by shape: 3 for bf16 launches of at least 16 matrices and 512 workgroups, workgroups of 16 columns for launches
- * of at most 128 64-column blocks, else 2; 0 split-K products plus a reduce kernel, 1 one workgroup
+ * norm bounds (-1 by shape: 3 for bf16 launches of at least 16 matrices and 512 workgroups, one launch for the whole bound up to n 128 (256 in
+ * bf16 or where fp32 rows are not 16-byte aligned), workgroups of 16 columns for launches of at most 128 64-column blocks
+ * and unaligned fp32 rows, else 2; 0 split-K products plus a reduce kernel, 1 one workgroup
  * per 64 output columns over the whole k range, 2 the same with A staged through LDS in row-contiguous runs, 3 bf16
  * matrices of an even number of 64-tiles read from their upper tiles only, in tournament-paired rounds (else as 2);
  * shapes the column kernels cannot read take the split-K kernel); option 5 = how the bf16 update

@@ -574,16 +574,19 @@ int nlb_iterate(NlbArgs a, const NlbFinal& fin, const NlbWs& w, hipStream_t st, 
   return hip_check(nlb_final_launch(a, fin, st), "nlb_final");
 }
 
-// Bounds of matrices read from their upper triangle only: the 16-column kernel where it can read them, else split-K
-// products on the converting engine.
+// The 16-column V A kernel reads any fp32 matrix of less than 2 GiB (and bf16 ones in the layout above).
+bool strip_ok(int64_t n, int64_t lda, int a_bf16) {
+  return !a_bf16 && n * lda < ((int64_t)1 << 29) && NLB_K * n < ((int64_t)1 << 29);
+}
+
+// Bounds of matrices read from their upper triangle only: the 16-column kernel below 2 GiB, else split-K products on the
+// converting engine.
 int run_nlb(int64_t n, int sign, int nb, const float* const* A, int64_t lda, const float* const* V, const NlbFinal& fin,
             const NlbWs& w, hipStream_t st) {
   NlbArgs a = nlb_args(n, sign, nb, A, lda, w);
   for (int b = 0; b < nb; ++b) { a.Vin[b] = V[b]; a.Vout[b] = w.vb0[b]; }
   PSGDK_TRY(nlb_tri_start(a, st));
-  const void* Av[MAXB];
-  for (int b = 0; b < nb; ++b) Av[b] = A[b];
-  if (vmm_cols_ok(n, nb, Av, lda, 4, w)) {
+  if (strip_ok(n, lda, 0)) {
     a.vmm_cols = 4; a.tri = 1; a.ssc = 16;
     return nlb_iterate(a, fin, w, st, [&](const NlbArgs& p, int normalize) {
       return hip_check(nlb_full_launch(p, 2, 0, normalize, st), "V A");
@@ -602,9 +605,19 @@ int run_nlb_full(int64_t n, int sign, int nb, const void* const* A, int64_t lda,
   const float* Af[MAXB];
   for (int b = 0; b < nb; ++b) Af[b] = reinterpret_cast<const float*>(A[b]);
   NlbArgs a = nlb_args(n, sign, nb, Af, lda, w);
+  // small matrices: the whole bound in one launch. Up to 256 where the products are bf16 or the column kernels below
+  // cannot read the rows, else up to 128: one workgroup's fp32 MFMAs take longer than seven launches beyond (whole
+  // bounds, us, seven to eleven launches -> one: fp32 n 10 33 -> 20, 128 39 -> 32, 256 40 -> 75, 250 89 -> 61; bf16 64
+  // 34 -> 17, 256 36 -> 31).
+  const bool wide = vmm_cols_ok(n, nb, A, lda, a_bf16 ? 2 : 4, w);
+  if (g_vmm_cols == -1 && (!a_bf16 || wide) && n <= (a_bf16 || !wide ? NLB_SMALL_N : NLB_SMALL_N / 2) &&
+      n * lda < ((int64_t)1 << 29)) {
+    for (int b = 0; b < nb; ++b) a.Vin[b] = V[b];
+    return hip_check(nlb_small_launch(a, fin, a_bf16, st), "small norm bound");
+  }
   nlb_full_plan(n, nb, w.part_cols, a.ksplit, a.kslice);
   a.vmm_u = g_vmm_u;
-  a.vmm_cols = g_vmm_cols != 0 && vmm_cols_ok(n, nb, A, lda, a_bf16 ? 2 : 4, w) ? (g_vmm_cols != 1 ? 2 : 1) : 0;
+  a.vmm_cols = g_vmm_cols != 0 && wide ? (g_vmm_cols != 1 ? 2 : 1) : 0;
   // bf16 matrices of an even number of 64-tiles: the kernel that reads the upper tiles only. It keeps a matrix on
   // one XCD, so by shape (option 4 = -1) it takes launches of at least 16 matrices (two per XCD or more) and 512
   // workgroups; smaller sets ran faster on the row kernel (measured crossovers), and option 4 = 3 forces it.
@@ -613,7 +626,8 @@ int run_nlb_full(int64_t n, int sign, int nb, const void* const* A, int64_t lda,
   // launches of the row kernel that would fill at most half of the CUs: 16 columns per workgroup instead of 64 (whole
   // bounds, us, 64 -> 16 columns: fp32 n 1024 80 -> 51, two of 4096 (128 workgroups) 248 -> 219, twelve of 768 (144)
   // 101 -> 120; bf16 1024 50 -> 39, two of 4096 132 -> 125, twelve of 768 72 -> 82)
-  else if (a.vmm_cols == 2 && g_vmm_cols == -1 && (int64_t)nb * ((n + 63) / 64) <= 128) a.vmm_cols = 4;
+  // and all fp32 matrices whose rows the 64-column kernels cannot read (two of 1531: 131 us by split-K products -> 88)
+  else if (g_vmm_cols == -1 && (a.vmm_cols ? (int64_t)nb * ((n + 63) / 64) <= 128 : strip_ok(n, lda, a_bf16))) a.vmm_cols = 4;
   a.vblk = a.vmm_cols == 3;  // the upper-tile kernel's V layout, from the init kernel on
   a.ssc = a.vmm_cols == 4 ? 16 : a.vmm_cols ? 64 : 128;
   if (a.vmm_cols && a.vmm_u == 8) a.vmm_u = 4;

@@ -70,6 +70,19 @@ __device__ __forceinline__ __amdgpu_buffer_rsrc_t make_rsrc(const void* base, lo
 }
 constexpr int kOob = 0x7fffffff;
 
+// x of the lane that DPP control C names (a move inside a row of 16 lanes; no LDS traffic, unlike a shuffle)
+template <int C>
+__device__ __forceinline__ float dpp(float x) {
+  return __int_as_float(__builtin_amdgcn_update_dpp(0, __float_as_int(x), C, 0xf, 0xf, false));
+}
+// sum over each row of 16 lanes, every lane getting its row's: quads, then the two quads of each half, then the halves
+__device__ __forceinline__ float row16_sum(float s) {
+  s += dpp<0xB1>(s);
+  s += dpp<0x4E>(s);
+  s += dpp<0x141>(s);
+  return s + dpp<0x140>(s);
+}
+
 // Block-wide reductions for blockDim.x a multiple of 64 (<= 1024). `red` holds >= 16 floats of LDS.
 __device__ __forceinline__ float block_sum(float v, float* red) {
   v = wave_sum(v);

@@ -53,11 +53,6 @@ static int ew_blocks(long long total) {
 }
 
 // ---------------------------------------------------------------------------------------------------------------
-// x of the lane that DPP control C names (a move inside a row of 16 lanes; no LDS traffic, unlike a shuffle)
-template <int C>
-__device__ __forceinline__ float dpp(float x) {
-  return __int_as_float(__builtin_amdgcn_update_dpp(0, __float_as_int(x), C, 0xf, 0xf, false));
-}
 // Sum and max over each row of 16 lanes, every lane getting the row's result: quad_perm(1,0,3,2) and (2,3,0,1) make
 // quad results, row_half_mirror combines the two quads of each half, row_mirror the two halves.
 __device__ __forceinline__ void row16_sum_max(float& s, float& m) {

@@ -6,6 +6,7 @@
 namespace psgdk {
 
 constexpr int NLB_K = 32;  // rows of the random start V
+constexpr int NLB_SMALL_N = 256;  // the largest side of a one-launch bound (nlb_small_launch)
 
 // per-matrix device scalars (scal[b][...])
 enum : int { NLB_NF = 0, NLB_J = 1, NLB_BOUND = 2, NLB_NSCAL = 4 };
@@ -79,6 +80,8 @@ hipError_t nlb_final_launch(const NlbArgs& a, const NlbFinal& f, hipStream_t st)
 // 4 init from the upper triangle only (fp32; without Vin the row statistics' results alone),
 // 3 the stage-0 outputs of a skew matrix from the per-(row, 64-column block) partials its producer left in part
 hipError_t nlb_full_launch(const NlbArgs& a, int stage, int a_bf16, int normalize, hipStream_t st);
+// the whole bound (a.Vin the start) of fully stored matrices of at most NLB_SMALL_N, bf16 in the 16-byte layout
+hipError_t nlb_small_launch(const NlbArgs& a, const NlbFinal& f, int a_bf16, hipStream_t st);
 hipError_t debug_mfma_launch(const float* A, const float* B, float* C, int prec, hipStream_t st);
 
 }  // namespace psgdk

@@ -7,7 +7,7 @@
 //                 (deterministic partial slots, no float atomics) and per-tile max |A_ij|
 //   tri_rowstats: a workgroup per 64 rows: squared row norms (partials in a fixed order), row maxima, the diagonal
 //   nlb_init    : a workgroup per (matrix, row of V): argmax (first maximum), nf, V0 (nlb_init_full_kernel)
-//   V A products: vmm_strip_kernel; for operands it cannot read, the converting engine (M = 32, B read from the
+//   V A products: vmm_strip_kernel; for matrices of 2 GiB and more, the converting engine (M = 32, B read from the
 //                 triangle), split over k, partials in ws, and
 //   nlb_reduce  : sums the k-split partials in a fixed order, scales the rows by 1/nf and by the input row
 //                 normalisation 1/(|V_in,r| + smallest normal) (exact: the product is linear in each row of V),
@@ -129,8 +129,26 @@ __global__ void __launch_bounds__(256) nlb_reduce_kernel(const NlbArgs p, int no
   if (lane == 0) p.ssout[b][r * nbk + cb] = t;
 }
 
-// One workgroup per matrix, 16 threads per row of V: bound = nf * max_r |V4_r|, then the consumer's scalars. (One
-// thread per row read its ceil(n / ssc) partials one after the other: 22 us at n 3072.)
+// The bound nf m of matrix b (m = max_r |V4_r|) and the consumer's scalars. One thread.
+__device__ __forceinline__ void nlb_finish(const NlbArgs& p, const NlbFinal& f, int b, float nf, float m) {
+  const float bound = nf * m;
+  p.scal[b][NLB_BOUND] = bound;
+  if (f.mode == NLB_FINAL_FACTOR) {
+    // psgd_pro.py:132-135: ell = bound + term2; L = max(beta L + (1 - beta) ell, ell); coef = lr / L, term2
+    const float ell = bound + f.term2[b];
+    float* L = f.L[b];
+    const float Ln = fmaxf(f.beta * L[0] + (1.f - f.beta) * ell, ell);
+    L[0] = Ln;
+    f.coef[b][0] = f.lr / Ln;
+    f.coef[b][1] = f.term2[b];
+  } else if (f.mode == NLB_FINAL_SCALE) {
+    // psgd_pro.py:88: R / (bound + smallest normal)
+    f.coef[b][0] = 1.f / (bound + kSmallestNormal);
+  }
+}
+
+// One workgroup per matrix, 16 threads per row of V. (One thread per row read its ceil(n / ssc) partials one after the
+// other: 22 us at n 3072.)
 __global__ void __launch_bounds__(16 * NLB_K) nlb_final_kernel(const NlbArgs p, NlbFinal f) {
   __shared__ float red[16];
   const int b = blockIdx.x, lane = threadIdx.x;
@@ -141,23 +159,7 @@ __global__ void __launch_bounds__(16 * NLB_K) nlb_final_kernel(const NlbArgs p, 
   for (int q = lane & 15; q < nbk; q += 16) s += ss[q];
   for (int o = 1; o < 16; o <<= 1) s += __shfl_xor(s, o, 64);
   const float m = block_max(fmaxf(sqrtf(s), 0.f), red);  // a row of NaN counts as zero
-  if (lane == 0) {
-    const float nf = p.scal[b][NLB_NF];
-    const float bound = nf * m;
-    p.scal[b][NLB_BOUND] = bound;
-    if (f.mode == NLB_FINAL_FACTOR) {
-      // psgd_pro.py:132-135: ell = bound + term2; L = max(beta L + (1 - beta) ell, ell); coef = lr / L, term2
-      const float ell = bound + f.term2[b];
-      float* L = f.L[b];
-      const float Ln = fmaxf(f.beta * L[0] + (1.f - f.beta) * ell, ell);
-      L[0] = Ln;
-      f.coef[b][0] = f.lr / Ln;
-      f.coef[b][1] = f.term2[b];
-    } else if (f.mode == NLB_FINAL_SCALE) {
-      // psgd_pro.py:88: R / (bound + smallest normal)
-      f.coef[b][0] = 1.f / (bound + kSmallestNormal);
-    }
-  }
+  if (lane == 0) nlb_finish(p, f, b, p.scal[b][NLB_NF], m);
 }
 
 // ---------------------------------------------------------------------------------------------------------------
@@ -955,10 +957,12 @@ __global__ void __launch_bounds__(256) vmm_rows_kernel(const NlbArgs p, int norm
 // LDS from its upper half. (A_sym^T is what is multiplied, as by the kernels that read rows in full.)
 // Latency-bound at these sizes: about 8 us per product of n 2048 fp32 from full storage (21 on 64-column blocks), 13 from
 // the triangle (18 and a 4 us reduce by split-K products).
-// Same operand contract as vmm_cols_kernel. grid: nb * ceil(n / 16).
+// bf16 needs the operand layout of vmm_cols_kernel; fp32 rows may start at any 4-byte boundary (16-byte loads checked by
+// the dword; ODD, n no multiple of 4: values past a row's end cleared on the way, which cost 8 us of a 2048 bound).
+// grid: nb * ceil(n / 16).
 constexpr int VS_C = 16, VS_LD = 20;  // columns per workgroup; row pitch (floats) of a [k][c] chunk
 
-template <typename T, bool TRI>
+template <typename T, bool TRI, bool ODD>
 __global__ void __launch_bounds__(512, 4) vmm_strip_kernel(const NlbArgs p, int normalize) {
   constexpr int CE = 16 / sizeof(T), CK = 2048 / sizeof(T);  // elements per 16-byte piece; k per chunk
   constexpr int KS = 4 * CE;                                 // k per MFMA step
@@ -971,7 +975,7 @@ __global__ void __launch_bounds__(512, 4) vmm_strip_kernel(const NlbArgs p, int 
   const int r16 = lane & 15, g = lane >> 4;
   const T* __restrict__ V = reinterpret_cast<const T*>(p.Vin[b]);
   const __amdgpu_buffer_rsrc_t rv = make_rsrc(V, (long long)NLB_K * n * sizeof(T));
-  const __amdgpu_buffer_rsrc_t ra = make_rsrc(p.A[b], (long long)n * p.lda * sizeof(T));
+  const __amdgpu_buffer_rsrc_t ra = make_rsrc(p.A[b], ((n - 1) * p.lda + n) * (long long)sizeof(T));
   const int lda = (int)p.lda;
   uint4 st[4], vn[4][2];
   // chunk of k kc .. kc + CK - 1, none at or past kend: A's rows c0 .. (piece tid % 128 of rows tid / 128 + 4 i), or
@@ -1011,17 +1015,32 @@ __global__ void __launch_bounds__(512, 4) vmm_strip_kernel(const NlbArgs p, int 
     if (q0 == 0) rsl[r] = sc;
   }
   while (true) {
+    // (fp32: the piece that straddles a row's end is followed by the next row)
+    const int keep = n & 3;
+    auto cut = [&](uint4& u, int k) {
+      const bool end = ODD && k == n - keep;
+      u.x = end && keep < 1 ? 0 : u.x;
+      u.y = end && keep < 2 ? 0 : u.y;
+      u.z = end && keep < 3 ? 0 : u.z;
+      u.w = end ? 0 : u.w;
+    };
+    int t = tid;
+    if constexpr (TRI && ODD) asm volatile("" : "+v"(t));  // its addresses recomputed per chunk: few registers
+#pragma unroll
+    for (int i = 0; i < 4; ++i) {
+      const int row = (t >> 7) + 4 * i;
+      if (!cols) cut(st[i], kc + (t & 127) * CE);
+      if (cols) *reinterpret_cast<uint4*>(sm + (((t >> 2) + 128 * i) * VS_LD + (t & 3) * 4) * 4) = st[i];
+      else *reinterpret_cast<uint4*>(sm + row * 2048 + ((t & 127) ^ row) * 16) = st[i];
+    }
     uint4 vc[4][2];
 #pragma unroll
     for (int s = 0; s < 4; ++s)
 #pragma unroll
-      for (int i = 0; i < 2; ++i) vc[s][i] = vn[s][i];
-#pragma unroll
-    for (int i = 0; i < 4; ++i) {
-      const int row = (tid >> 7) + 4 * i;
-      if (cols) *reinterpret_cast<uint4*>(sm + (((tid >> 2) + 128 * i) * VS_LD + (tid & 3) * 4) * 4) = st[i];
-      else *reinterpret_cast<uint4*>(sm + row * 2048 + ((tid & 127) ^ row) * 16) = st[i];
-    }
+      for (int i = 0; i < 2; ++i) {
+        vc[s][i] = vn[s][i];
+        cut(vc[s][i], kc + wave * (CK / 8) + s * KS + g * CE);
+      }
     __syncthreads();
     const bool now_cols = cols, diag = TRI && !cols && kc == split;
     kc += CK;
@@ -1327,6 +1346,186 @@ __global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(5))) v
   }
 }
 
+// A whole bound of a small fully stored matrix (n <= VB_N) in one launch, one workgroup per matrix: row statistics, start,
+// four V A products and the final scalars, V in LDS throughout. Wave w owns the 16 rows (as output columns) 16 w .. and
+// reads their MFMA fragments from global memory, all of a pass's loads issued together, once for the statistics and once
+// per product; fp32 rows may start at any 4-byte boundary (dword-checked 16-byte loads, values past the row cleared),
+// bf16 needs the layout of vmm_cols_kernel. V is rounded to A's type between products, as in the kernels above.
+// Bound by launches, not work, at these sizes: seven to eleven launches become one (a whole bound of
+// bf16 n 64: 34 us, now 17; fp32 n 10: 33, now 20).
+constexpr int VB_N = NLB_SMALL_N, VB_LD = VB_N + 4;
+
+template <typename T>
+__global__ void __launch_bounds__(1024) nlb_small_kernel(const NlbArgs p, NlbFinal f) {
+  constexpr int CE = 16 / sizeof(T), KS = 4 * CE, NS = VB_N / KS;  // elements per piece, k per step, steps
+  constexpr bool BF = sizeof(T) == 2;
+  __shared__ __attribute__((aligned(16))) float V[NLB_K][VB_LD];  // bf16: 2-byte elements in the same rows
+  __shared__ float aj[VB_N], ssw[16][NLB_K], rsl[NLB_K], red[16];
+  __shared__ float smax[16];
+  __shared__ int sidx[16];
+  const int b = blockIdx.x, n = p.n, tid = threadIdx.x, lane = tid & 63;
+  const int w = __builtin_amdgcn_readfirstlane(tid >> 6), r16 = lane & 15, g = lane >> 4;
+  const int c = 16 * w + r16, lda = (int)p.lda;  // this lane's row of A
+  const T* __restrict__ A = reinterpret_cast<const T*>(p.A[b]);
+  const __amdgpu_buffer_rsrc_t ra = make_rsrc(A, ((long long)(n - 1) * lda + n) * sizeof(T));
+  const int off = c < n ? (c * lda + g * CE) * (int)sizeof(T) : kOob;
+  auto load = [&](uint4 (&x)[NS]) {
+#pragma unroll
+    for (int s = 0; s < NS; ++s) {
+      const int k = s * KS + g * CE;
+      x[s] = __builtin_bit_cast(uint4, __builtin_amdgcn_raw_buffer_load_b128(ra, k < n ? off : kOob, s * 64, 0));
+    }
+#pragma unroll
+    for (int s = 0; s < NS; ++s)
+      if constexpr (!BF) {
+        const int k = s * KS + g * CE;
+        x[s].y = k + 1 < n ? x[s].y : 0;
+        x[s].z = k + 2 < n ? x[s].z : 0;
+        x[s].w = k + 3 < n ? x[s].w : 0;
+      }
+  };
+  auto val = [&](const uint4& u, int e) {
+    const uint32_t d = (&u.x)[BF ? e >> 1 : e];
+    return BF ? __uint_as_float(e & 1 ? d & 0xffff0000u : d << 16) : __uint_as_float(d);
+  };
+  // row statistics: squared norm, max |.|, diagonal (skew: counts as zero)
+  float s2 = 0.f, am = 0.f, dm = -INFINITY;
+  {
+    uint4 x[NS];
+    load(x);
+    const int own = p.sign < 0 ? c - g * CE : -1;  // skew: the k, in this lane's pieces, that counts as zero
+#pragma unroll
+    for (int s = 0; s < NS; ++s) {
+      __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+      for (int e = 0; e < CE; ++e) {
+        const float v = s * KS + e == own ? 0.f : val(x[s], e);
+        s2 += v * v;
+        am = fmaxf(am, fabsf(v));
+      }
+    }
+    if (c < n) dm = to_f32<T>(A[(long long)c * lda + c]);
+  }
+  s2 += __shfl_xor(s2, 16, 64);
+  s2 += __shfl_xor(s2, 32, 64);
+  float best = c < n ? s2 : -1.f;
+  int bi = c;
+  for (int o = 1; o < 16; o <<= 1) {
+    const float ov = __shfl_xor(best, o, 64);
+    const int oi = __shfl_xor(bi, o, 64);
+    if (ov > best || (ov == best && oi < bi)) { best = ov; bi = oi; }
+  }
+  if (lane == 0) { smax[w] = best; sidx[w] = bi; }
+  am = block_max(am, red);
+  dm = block_max(dm, red);
+  float bv = -1.f;
+  int j = 0x7fffffff;
+  for (int q = 0; q < 16; ++q)
+    if (smax[q] > bv) { bv = smax[q]; j = sidx[q]; }  // waves in row order: the first maximum
+  j = j < n ? j : 0;
+  const float nf = (p.sign > 0 ? dm : am) + kSmallestNormal;
+  for (int k = tid; k < VB_N; k += 1024)
+    aj[k] = k < n ? (p.sign < 0 && k == j ? 0.f : to_f32<T>(A[(long long)j * lda + k])) / nf : 0.f;
+  __syncthreads();
+  auto vput = [&](int r, int k, float v) {
+    if constexpr (BF) reinterpret_cast<bf16_t*>(V[r])[k] = f32_to_bf16(v);
+    else V[r][k] = v;
+  };
+  // V0[r] = a_j + sgn(<a_j, V_r>) V_r, zero past n
+  for (int r = w; r < NLB_K; r += 16) {
+    const float* __restrict__ vr = p.Vin[b] + (long long)r * n;
+    float v[VB_N / 64], d = 0.f;
+#pragma unroll
+    for (int q = 0; q < VB_N / 64; ++q) {
+      const int k = 64 * q + lane;
+      v[q] = vr[k < n ? k : 0];
+      d += aj[k] * v[q];
+    }
+    d = wave_sum(d);
+    const float sg = d > 0.f ? 1.f : (d < 0.f ? -1.f : 0.f);
+#pragma unroll
+    for (int q = 0; q < VB_N / 64; ++q) {
+      const int k = 64 * q + lane;
+      vput(r, k, k < n ? aj[k] + sg * v[q] : 0.f);
+    }
+  }
+  float m = 0.f;
+#pragma unroll 1
+  for (int it = 0; it < 4; ++it) {
+    uint4 x[NS];
+    load(x);
+    __syncthreads();  // V and, from the second product on, ssw
+    if (tid < NLB_K) {
+      float sc = 1.f / nf;
+      if (it & 1) {
+        float t = 0.f;
+        for (int q = 0; q < 16; ++q) t += ssw[q][tid];
+        sc = sc / (sqrtf(t) + kSmallestNormal);
+      }
+      rsl[tid] = sc;
+    }
+    f32x4_t acc[2] = {};
+    if (16 * w < n) {
+#pragma unroll
+      for (int s = 0; s < NS; ++s) {
+        if (s * KS >= n) break;
+        if (s % 2 == 0) __builtin_amdgcn_sched_barrier(0);  // few of V's fragments at a time: 128 registers
+        uint4 vf[2];
+#pragma unroll
+        for (int i = 0; i < 2; ++i)
+          vf[i] = *reinterpret_cast<const uint4*>(reinterpret_cast<const T*>(V[i * 16 + r16]) + s * KS + g * CE);
+        if constexpr (BF) {
+#pragma unroll
+          for (int i = 0; i < 2; ++i)
+            acc[i] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(__builtin_bit_cast(bf16x8_t, vf[i]),
+                                                             __builtin_bit_cast(bf16x8_t, x[s]), acc[i], 0, 0, 0);
+        } else {
+#pragma unroll
+          for (int e = 0; e < 4; ++e)
+#pragma unroll
+            for (int i = 0; i < 2; ++i)
+              acc[i] = __builtin_amdgcn_mfma_f32_16x16x4f32(__uint_as_float((&vf[i].x)[e]), __uint_as_float((&x[s].x)[e]),
+                                                            acc[i], 0, 0, 0);
+        }
+      }
+    }
+    __syncthreads();  // V's and ssw's readers are done, rsl is written
+    // lane holds rows 16 i + 4 g + e of column c
+    if (16 * w < n) {
+#pragma unroll
+      for (int i = 0; i < 2; ++i)
+#pragma unroll
+        for (int e = 0; e < 4; ++e) {
+          const int r = 16 * i + 4 * g + e;
+          const float v = c < n ? acc[i][e] * rsl[r] : 0.f;
+          vput(r, c, v);
+          const float sq = row16_sum(v * v);
+          if (r16 == 0) ssw[w][r] = sq;
+        }
+    } else if (lane < NLB_K) {
+      ssw[w][lane] = 0.f;
+    }
+  }
+  __syncthreads();
+  if (tid < 64) {
+    float t = 0.f;
+    if (tid < NLB_K)
+      for (int q = 0; q < 16; ++q) t += ssw[q][tid];
+    m = wave_max(fmaxf(sqrtf(t), 0.f));  // a row of NaN counts as zero
+    if (tid == 0) {
+      p.scal[b][NLB_NF] = nf;
+      p.scal[b][NLB_J] = (float)j;
+      nlb_finish(p, f, b, nf, m);
+    }
+  }
+}
+hipError_t nlb_small_launch(const NlbArgs& a, const NlbFinal& f, int a_bf16, hipStream_t st) {
+  if (a.n > VB_N) return hipErrorInvalidValue;
+  if (a_bf16) hipLaunchKernelGGL(nlb_small_kernel<bf16_t>, dim3(a.nb), dim3(1024), 0, st, a, f);
+  else hipLaunchKernelGGL(nlb_small_kernel<float>, dim3(a.nb), dim3(1024), 0, st, a, f);
+  return hipGetLastError();
+}
+
 hipError_t nlb_full_launch(const NlbArgs& a, int stage, int a_bf16, int normalize, hipStream_t st) {
   if (stage == 3) {
     hipLaunchKernelGGL(rowstats_reduce_kernel, dim3(((a.n + 63) / 64) * a.nb), dim3(256), 0, st, a);
@@ -1344,9 +1543,12 @@ hipError_t nlb_full_launch(const NlbArgs& a, int stage, int a_bf16, int normaliz
     const dim3 grid(((a.n + VMC - 1) / VMC) * a.nb);
     if (a.vmm_cols == 4) {
       const dim3 gs(((a.n + VS_C - 1) / VS_C) * a.nb);
-      if (a.tri) hipLaunchKernelGGL((vmm_strip_kernel<float, true>), gs, dim3(512), 0, st, a, normalize);
-      else if (a_bf16) hipLaunchKernelGGL((vmm_strip_kernel<bf16_t, false>), gs, dim3(512), 0, st, a, normalize);
-      else hipLaunchKernelGGL((vmm_strip_kernel<float, false>), gs, dim3(512), 0, st, a, normalize);
+      const bool odd = (a.n & 3) != 0;
+      if (a_bf16) hipLaunchKernelGGL((vmm_strip_kernel<bf16_t, false, false>), gs, dim3(512), 0, st, a, normalize);
+      else if (a.tri && odd) hipLaunchKernelGGL((vmm_strip_kernel<float, true, true>), gs, dim3(512), 0, st, a, normalize);
+      else if (a.tri) hipLaunchKernelGGL((vmm_strip_kernel<float, true, false>), gs, dim3(512), 0, st, a, normalize);
+      else if (odd) hipLaunchKernelGGL((vmm_strip_kernel<float, false, true>), gs, dim3(512), 0, st, a, normalize);
+      else hipLaunchKernelGGL((vmm_strip_kernel<float, false, false>), gs, dim3(512), 0, st, a, normalize);
     } else if (a.vmm_cols == 3) {  // bf16, square, n a multiple of 128 (an even number of 64-tiles)
       const int T = a.n / VMC;
       hipLaunchKernelGGL(vmm_tri_kernel, dim3(8 * ((a.nb + 7) / 8) * T), dim3(256), 0, st, a, normalize);

@@ -1,5 +1,6 @@
-"""Norm bounds whose V A products run on 16-column workgroups (csrc/nlb.hip, vmm_strip_kernel): matrices read from their
-upper triangle, and launches of few fully stored ones, at the edges of the kernel's column blocks and k chunks."""
+"""Norm bounds of one launch (csrc/nlb.hip, nlb_small_kernel) and those whose V A products run on 16-column workgroups
+(vmm_strip_kernel): matrices read from their upper triangle, launches of few fully stored ones and rows at odd addresses,
+at the edges of the kernels' sides, column blocks and k chunks."""
 import pytest
 import torch
 
@@ -17,11 +18,11 @@ def _bound(fn, mats, Vs, sign, *extra):
     return [float(o) for o in outs]
 
 
-# k chunks hold 512 fp32 or 1024 bf16; n 4 and 8 are less than one column block, 509 has no 16-byte rows (the split-K
-# route), 516 and 1032 end a chunk after 4 and 8, 1040 is a whole number of blocks
-@pytest.mark.parametrize("n", [4, 8, 16, 509, 512, 516, 1032, 1040])
+# One launch: up to 128 (fp32), 256 (bf16, and fp32 rows that are not 16-byte aligned). Strips: k chunks hold 512 fp32 or
+# 1024 bf16; 257, 509 and 1030 end in a partial piece, 516 and 1032 end a chunk after 4 and 8.
+@pytest.mark.parametrize("n", [1, 3, 16, 127, 128, 129, 132, 254, 256, 257, 264, 509, 512, 516, 1030, 1032, 1040])
 @pytest.mark.parametrize("sign", [1, -1])
-def test_bound_by_column_strips(n, sign):
+def test_bounds_at_the_edges(n, sign):
     """Against float64: fp32 sums of n products and five roundings per pass leave far less than 1e-5 of the norms here
     (sqrt(n) 2^-24 is 2e-6); bf16 storage rounds each of the iteration's vectors by up to 2^-8 (rel 2e-2)."""
     g = torch.Generator().manual_seed(n)
@@ -33,13 +34,13 @@ def test_bound_by_column_strips(n, sign):
         Vs.append(torch.randn(32, n, generator=g))
     lib, dv = L.lib(), [v.to(DEV) for v in Vs]
     ref = [float(norm_lower_bound(M.double(), V.double(), skew=sign < 0)) for M, V in zip(mats, Vs)]
-    wide = []  # a row stride over n, and NaN wherever only the other triangle's reader may look
+    nan, wide, up = float("nan"), [], []  # a row stride over n; NaN wherever the bound must not look
     for M in mats:
-        W = torch.full((n, n + 4), float("nan"), device=DEV)
-        W[:, :n] = torch.where(torch.ones(n, n).triu().bool(), M, torch.tensor(float("nan"))).to(DEV)
-        wide.append(W)
-    tri = _bound(lib.psgdk_norm_lower_bound, wide, dv, sign)
-    full = _bound(lib.psgdk_norm_lower_bound_full, [M.to(DEV) for M in mats], dv, sign, 0)
+        wide.append(torch.full((n, n + 4), nan, device=DEV))
+        wide[-1][:, :n] = M.to(DEV)
+        up.append(torch.where(torch.ones(n, n + 4, device=DEV).triu().bool(), wide[-1], nan))
+    tri = _bound(lib.psgdk_norm_lower_bound, up, dv, sign)
+    full = _bound(lib.psgdk_norm_lower_bound_full, wide, dv, sign, 0)
     b16 = [M.to(DEV).bfloat16() for M in mats]
     low = _bound(lib.psgdk_norm_lower_bound_full, b16, dv, sign, 1)
     for r, t, f, q in zip(ref, tri, full, low):
