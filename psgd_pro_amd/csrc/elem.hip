@@ -774,24 +774,31 @@ __device__ __forceinline__ float clamp_keep_nan(float x, float amp) { return x <
 __global__ void __launch_bounds__(EW_THREADS) clip_update_kernel(const EwArgs a, int blocks_per) {
   __shared__ float red[16];
   const int b = blockIdx.x / blocks_per;
-  const float* part = a.in3[b];
-  float s = 0.f;
-  for (int t = threadIdx.x; t < a.i0; t += blockDim.x) s += part[2 * t];
-  s = block_sum(s, red);
   const long long total = a.m * a.n;
-  const float avg = sqrtf(s / (float)total);
-  const bool scale = avg > a.f0;
-  const float sc = a.f0 / avg;
   long long beg, end;
   const float* pre = a.in2[b];
   void* prm = const_cast<void*>(a.in[b]);
   float* gout = reinterpret_cast<float*>(a.out2[b]);
-  if ((total & 7) == 0 && al16(pre) && al16(prm) && (!gout || al16(gout))) {
+  const bool vec = (total & 7) == 0 && al16(pre) && al16(prm) && (!gout || al16(gout));
+  // the thread's first elements are requested before the partial sums are added up (they are all of its elements in
+  // launches of many workgroups, whose loads waited for the sum and its barriers: 28.3 M elements, bf16
+  // parameters, within the step, 86 us; 67 now)
+  float g[8], w[8];
+  if (vec) {
     ew_range8(total, blocks_per, beg, end);
-    for (long long v = beg + threadIdx.x; v < end; v += EW_THREADS) {
-      float g[8], w[8];
-      ew_load8(pre + 8 * v, g);
-      ew_load8_dt(prm, a.dt, 8 * v, w);
+    const long long v = beg + threadIdx.x < end ? beg + threadIdx.x : 0;
+    ew_load8(pre + 8 * v, g);
+    ew_load8_dt(prm, a.dt, 8 * v, w);
+  }
+  const float* part = a.in3[b];
+  float s = 0.f;
+  for (int t = threadIdx.x; t < a.i0; t += blockDim.x) s += part[2 * t];
+  s = block_sum(s, red);
+  const float avg = sqrtf(s / (float)total);
+  const bool scale = avg > a.f0;
+  const float sc = a.f0 / avg;
+  if (vec) {
+    for (long long v = beg + threadIdx.x; v < end;) {
 #pragma unroll
       for (int e = 0; e < 8; ++e) {
         if (scale) g[e] *= sc;
@@ -801,6 +808,11 @@ __global__ void __launch_bounds__(EW_THREADS) clip_update_kernel(const EwArgs a,
       if (gout) ew_store8(gout + 8 * v, g);
       if (a.dt) ew_store8(reinterpret_cast<bf16_t*>(prm) + 8 * v, w);
       else ew_store8(reinterpret_cast<float*>(prm) + 8 * v, w);
+      v += EW_THREADS;
+      if (v < end) {
+        ew_load8(pre + 8 * v, g);
+        ew_load8_dt(prm, a.dt, 8 * v, w);
+      }
     }
     return;
   }
