@@ -333,8 +333,9 @@ __global__ void __launch_bounds__(WN == 4 || KG == 2 ? 512 : 256, 2) gemm_cv_ker
   };
   auto zero = [&]() INL { each_acc([&](int i, int j, int e) INL { acc[i][j][e] = blk[i][j][e] = sm[i][j][e] = 0.f; }); };
   auto fold = [&](bool neg) INL {
+    const float sg = neg ? -1.f : 1.f;
     each_acc([&](int i, int j, int e) INL {
-      acc[i][j][e] += neg ? -blk[i][j][e] : blk[i][j][e];
+      acc[i][j][e] = fmaf(sg, blk[i][j][e], acc[i][j][e]);  // an exact product: one rounding, as of the sum
       blk[i][j][e] = 0.f;
     });
   };
