@@ -743,6 +743,16 @@ int64_t dense_max(const psgdk_kron2d_t* g) {
   return d;
 }
 
+// The diagonal factor of a group of vectors (the other side 1, no factor there), or -1. Up to 16384 elements, which one
+// workgroup reads in about the time of a launch, their update and application take one launch each (the small ViT's
+// six groups of vectors: 30 launches fewer, its step 1852 us -> 1724; longer ones keep a workgroup per 2048 elements).
+int vector_factor(const psgdk_kron2d_t* g) {
+  if (g->m * g->n > 16384) return -1;
+  for (int f = 0; f < 2; ++f)
+    if (g->kind[f] == PSGDK_FACTOR_DIAG && g->kind[1 - f] == PSGDK_FACTOR_NONE) return f;
+  return -1;
+}
+
 // out = P1 X P2 over the factor kinds (dense: GEMM with P; diagonal: scaling by q * q; none: identity).
 // tmp: m x n scratch. With part non-null, sum-of-squares partials of out are written there and their count to
 // *npart.
@@ -1953,6 +1963,17 @@ int psgdk_kron2d_update(const psgdk_kron2d_t* g, const psgdk_update_opts_t* o, c
   PSGDK_TRY(check_ptrs(noise, nb, "noise"));
   if (dmx) PSGDK_TRY(check_ptrs(V, nb, "V"));
   hipStream_t st = (hipStream_t)stream;
+  const int vf = vector_factor(g);
+  if (vf >= 0) {
+    EwArgs a;
+    std::memset(&a, 0, sizeof a);
+    a.nb = nb; a.m = mn; a.dt = g->g_dtype; a.f0 = o->lr; a.f1 = o->betaL; a.f2 = o->damping; a.f3 = o->grad_eps;
+    for (int b = 0; b < nb; ++b) {
+      a.in[b] = g->G[b]; a.in2[b] = reinterpret_cast<const float*>(noise[b]);
+      a.out[b] = g->Q[vf][b]; a.out2[b] = g->P[vf][b]; a.sc[b] = g->L[vf][b];
+    }
+    return hip_check(vec_update_launch(a, st), "vector update");
+  }
 
   // X = G + (damping + eps |G|) N   (psgd_pro.py:121-123)
   {
@@ -2092,6 +2113,19 @@ int psgdk_kron2d_apply(const psgdk_kron2d_t* g, const psgdk_apply_opts_t* o, voi
   if (*ws_bytes < w.off) return fail(PSGDK_EWORKSPACE, "workspace %zu < %zu bytes", *ws_bytes, w.off);
   PSGDK_TRY(check_ptrs(params, nb, "params"));
   hipStream_t st = (hipStream_t)stream;
+  const int vf = vector_factor(g);
+  if (vf >= 0) {
+    EwArgs a;
+    std::memset(&a, 0, sizeof a);
+    a.nb = nb; a.m = mn; a.dt = g->p_dtype; a.i1 = g->g_dtype;
+    a.f0 = o->max_avg_amp; a.f1 = o->max_element_amp; a.f2 = o->lr_params;
+    for (int b = 0; b < nb; ++b) {
+      a.in[b] = params[b]; a.in2[b] = g->P[vf][b]; a.out[b] = pre_out ? pre_out[b] : nullptr;
+      a.aux[b] = reinterpret_cast<float*>(const_cast<void*>(g->G[b]));
+      a.out2[b] = clipped_out ? clipped_out[b] : nullptr;
+    }
+    return hip_check(vec_apply_launch(a, st), "vector application");
+  }
   for (int b = 0; b < nb; ++b)
     if (pre_out && pre_out[b]) pre[b] = pre_out[b];
   int np = 0;

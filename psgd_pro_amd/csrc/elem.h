@@ -30,6 +30,9 @@ struct EwArgs {
 // (psgd_pro.py:121-123);
 // in3 (optional): a row scale applied to X (a diagonal P1 of P1 X P2)
 hipError_t noise_launch(const EwArgs& a, hipStream_t st);
+// the whole update and the whole application of vectors (one diagonal factor, the other side 1)
+hipError_t vec_update_launch(const EwArgs& a, hipStream_t st);
+hipError_t vec_apply_launch(const EwArgs& a, hipStream_t st);
 // out2 = bf16 (X diag(in3))^T with X as noise_launch (a diagonal P2 folded into the transposed operand of P1 X P2)
 hipError_t noise_t_launch(const EwArgs& a, hipStream_t st);
 // out[i] = sum_j X[i][j]^2 of a bf16 m x n matrix (a diagonal factor's term1 from the bf16 Pg or Pg^T)

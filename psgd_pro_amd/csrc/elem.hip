@@ -838,6 +838,84 @@ hipError_t clip_update_launch(const EwArgs& a, hipStream_t st) {
 }
 
 // ---------------------------------------------------------------------------------------------------------------
+// A vector's whole update: one diagonal factor of m elements, the other side 1, so Pg = X P elementwise, term1 = Pg^2 and
+// term2 = 1. in = G and in2 = N (dtype dt), out = q (in place), out2 = P (read, then q * q), sc = L; f0 = lr, f1 = beta,
+// f2, f3 = damping and eps of X = G + (f2 + f3 |G|) N. One workgroup per vector; term1 is computed again for the second
+// pass rather than kept. (Four launches of a few microseconds each, bound by the host: noise, scaling, term1 and update.)
+__global__ void __launch_bounds__(1024) vec_update_kernel(const EwArgs a) {
+  __shared__ float red[16];
+  __shared__ float s_c;
+  const int b = blockIdx.x;
+  const void* N = a.in2[b];
+  float* q = a.out[b];
+  float* P = reinterpret_cast<float*>(a.out2[b]);
+  auto term1 = [&](long long i) {
+    const float g = ldv(a.in[b], a.dt, i);
+    const float pg = (g + (a.f2 + a.f3 * fabsf(g)) * ldv(N, a.dt, i)) * P[i];
+    return pg * pg;
+  };
+  float mx = -INFINITY;
+  for (long long i = threadIdx.x; i < a.m; i += blockDim.x) mx = fmaxf(mx, term1(i));
+  mx = block_max(mx, red);
+  if (threadIdx.x == 0) {
+    const float ell = mx + 1.f;
+    float* L = a.sc[b];
+    const float Ln = fmaxf(a.f1 * L[0] + (1.f - a.f1) * ell, ell);
+    L[0] = Ln;
+    s_c = a.f0 / Ln;
+  }
+  __syncthreads();
+  const float c = s_c;
+  for (long long i = threadIdx.x; i < a.m; i += blockDim.x) {
+    const float v = q[i] * (1.f - c * (term1(i) - 1.f));
+    q[i] = v;
+    P[i] = v * v;
+  }
+}
+hipError_t vec_update_launch(const EwArgs& a, hipStream_t st) {
+  hipLaunchKernelGGL(vec_update_kernel, dim3(a.nb), dim3(1024), 0, st, a);
+  return hipGetLastError();
+}
+
+// A vector's whole application: pre = G P (in2 = P, into out where given), its RMS, then clip_update_kernel's arithmetic.
+// in = param (dtype dt), aux = G (dtype i1), out2 = clipped (optional); f0 .. f2 as there. One workgroup per vector.
+__global__ void __launch_bounds__(1024) vec_apply_kernel(const EwArgs a) {
+  __shared__ float red[16];
+  const int b = blockIdx.x;
+  const float* P = a.in2[b];
+  auto pre = [&](long long i) { return ldv(a.aux[b], a.i1, i) * P[i]; };
+  float s = 0.f;
+  for (long long i = threadIdx.x; i < a.m; i += blockDim.x) {
+    const float v = pre(i);
+    if (a.out[b]) a.out[b][i] = v;
+    s += v * v;
+  }
+  s = block_sum(s, red);
+  const float avg = sqrtf(s / (float)a.m);
+  const bool scale = avg > a.f0;
+  const float sc = a.f0 / avg;
+  void* prm = const_cast<void*>(a.in[b]);
+  float* gout = reinterpret_cast<float*>(a.out2[b]);
+  for (long long i = threadIdx.x; i < a.m; i += blockDim.x) {
+    float g = pre(i);
+    if (scale) g *= sc;
+    g = clamp_keep_nan(g, a.f1);
+    if (gout) gout[i] = g;
+    if (a.dt) {
+      bf16_t* p = reinterpret_cast<bf16_t*>(prm);
+      p[i] = f32_to_bf16(bf16_to_f32(p[i]) - a.f2 * g);
+    } else {
+      float* p = reinterpret_cast<float*>(prm);
+      p[i] = p[i] - a.f2 * g;
+    }
+  }
+}
+hipError_t vec_apply_launch(const EwArgs& a, hipStream_t st) {
+  hipLaunchKernelGGL(vec_apply_kernel, dim3(a.nb), dim3(1024), 0, st, a);
+  return hipGetLastError();
+}
+
+// ---------------------------------------------------------------------------------------------------------------
 // out[b][blk] = max |in[b][i]| over the block's range (i0 = blocks per problem).
 __global__ void __launch_bounds__(EW_THREADS) absmax_kernel(const EwArgs a, int blocks_per) {
   __shared__ float red[16];
