@@ -301,7 +301,8 @@ __device__ __forceinline__ void store4(float* dst, const float (&x)[4]) {
 // :49-57). Workgroup r = 0 also publishes nf and j. The scans read 4 (statistics) or 8 (rows) elements per thread
 // and step with the loads of several steps in flight; the rows take the element path unless n % 8 == 0, A's row
 // stride is a multiple of 16 bytes and the bases are 16-byte aligned. TRI: only A's upper triangle is read (row j's part
-// left of the diagonal from column j); without a start V the row statistics' results alone are published.
+// left of the diagonal from column j); without a start V (of any matrix) one workgroup per matrix publishes the row
+// statistics' results alone.
 template <typename T, bool TRI>
 __global__ void __launch_bounds__(256) nlb_init_full_kernel(const NlbArgs p) {
   __shared__ float red[4];
@@ -309,7 +310,8 @@ __global__ void __launch_bounds__(256) nlb_init_full_kernel(const NlbArgs p) {
   __shared__ int sidx[4];
   __shared__ float snf;
   __shared__ int sj;
-  const int b = blockIdx.x / NLB_K, r = blockIdx.x % NLB_K;
+  const int rows = !TRI || p.Vin[0] ? NLB_K : 1;  // workgroups per matrix
+  const int b = blockIdx.x / rows, r = blockIdx.x % rows;
   const int tid = threadIdx.x, n = p.n;
   const float* __restrict__ rn2 = p.rn2[b];
   const float* __restrict__ rmax = p.rpart[b];

@@ -1,11 +1,12 @@
 """Norm bounds of one launch (csrc/nlb.hip, nlb_small_kernel) and those whose V A products run on 16-column workgroups
 (vmm_strip_kernel): matrices read from their upper triangle, launches of few fully stored ones and rows at odd addresses,
-at the edges of the kernels' sides, column blocks and k chunks."""
+at the edges of the kernels' sides, column blocks and k chunks; and the row norms of groups of triangles."""
 import pytest
 import torch
 
 from oracle.psgd_oracle import norm_lower_bound
 from psgd_pro_amd import _lib as L
+from tests.metrics import rel_err_norm
 
 pytestmark = pytest.mark.gpu
 DEV = "cuda"
@@ -46,3 +47,21 @@ def test_bounds_at_the_edges(n, sign):
     for r, t, f, q in zip(ref, tri, full, low):
         assert t == pytest.approx(r, rel=1e-5) and f == pytest.approx(r, rel=1e-5)
         assert q == pytest.approx(r, rel=2e-2)
+
+
+@pytest.mark.parametrize("nb", [3, 16])
+@pytest.mark.parametrize("n", [130, 129])
+def test_row_norms_of_several_matrices(nb, n):
+    """psgdk_tri_rownorm2 on a group: every matrix's squared row norms and largest element are its own (scales a factor of
+    two apart), and every output is written. rn2: n squares summed in fp32, 1e-6 as for one matrix."""
+    g = torch.Generator().manual_seed(n + nb)
+    X = [torch.randn(n, n, generator=g) * 2.0 ** b for b in range(nb)]
+    mats = [(x + x.T) for x in X]
+    up = [torch.where(torch.ones(n, n).triu().bool(), m, torch.tensor(float("nan"))).to(DEV) for m in mats]
+    rn2 = [torch.full((n,), float("nan"), device=DEV) for _ in mats]
+    amax = [torch.full((), float("nan"), device=DEV) for _ in mats]
+    L.call_ws(L.lib().psgdk_tri_rownorm2, n, 1, nb, L.ptrs(up), n, L.ptrs(rn2), L.ptrs(amax), ws=L.Workspace(),
+              device=up[0].device, stream=L.stream_of(up[0]))
+    for m, r, a in zip(mats, rn2, amax):
+        assert float(a) == float(m.abs().max())
+        assert rel_err_norm(r, m.double().square().sum(1)) < 1e-6
