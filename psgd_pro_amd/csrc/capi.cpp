@@ -143,8 +143,11 @@ struct EpiSpec {
 int run_gemm(int prec, int nb, int64_t M, int64_t N, int64_t K, const Opnd& A, const Opnd& B, float* const* C,
              int64_t ldc, const EpiSpec& e, int tri, int out_mode, int kbeg_tri, int splitk, int64_t kchunk,
              hipStream_t st, int* ntiles = nullptr);
-// The most partials an epilogue of run_gemm writes for an M x N product
-int max_tiles(int64_t M, int64_t N, int tri) { return gemm_cv_tiles(M, N, tri, 1); }
+// The most partials an epilogue of run_gemm writes for an M x N product, under any tile configuration (option 13 may
+// change between a size query and the call): 64 x 64 tiles, or the 32 x 64 ones that sums of squares also take
+int max_tiles(int64_t M, int64_t N, int tri) {
+  return std::max(gemm_cv_tiles(M, N, tri, 1), tri ? 0 : gemm_cv_tiles(M, N, 0, 2));
+}
 
 // ------------------------------------------------------------------------------------------------------------
 // bf16 k-contiguous GEMM (gemm_bf16.hip). A: M x K rows, B: N x K rows (bf16, k contiguous); C = acc A B^T.

@@ -1,10 +1,13 @@
 """The converting MFMA engine (csrc/gemm_cv.hip): every tile configuration at the edges of its tiles, in both precisions
 and every layout it reads, against float64."""
+import ctypes
+
 import pytest
 import torch
 
 from psgd_pro_amd import _lib as L
 from psgd_pro_amd import ops as K
+from tests.metrics import rel_err_norm
 
 pytestmark = pytest.mark.gpu
 DEV = "cuda"
@@ -94,3 +97,36 @@ def test_gram_diagonal_keeps_its_small_squares(cfg):
     # one rounding of at most 2^-24 per entry and either sign (1 <= C_ii < 2), so a mean of n of them within 4 standard
     # deviations 2^-24 / sqrt(3 n); the seven squares lost would make it -7 * 2^-26
     assert d.mean().abs().item() < 4 * 2.0 ** -24 / (3 * n) ** 0.5, d.mean()
+
+
+@pytest.mark.parametrize("m,n", [(1032, 1032), (24, 390), (129, 257)])
+def test_application_in_every_configuration(engine, m, n):
+    """P1 G P2, its sum of squares and the clipped update of two fp32 weights, from a workspace of exactly the queried size
+    between guard bytes that stay as they are. Two products of up to 1032 terms, 2e-7 each, and six element-wise roundings
+    of 2^-24: 1e-6 normwise leaves a factor of two."""
+    g = torch.Generator().manual_seed(m + n)
+    P = [[(lambda x: x @ x.T)(torch.randn(d, d, generator=g) / d ** 0.5 + torch.eye(d)) for d in (m, n)] for _ in range(2)]
+    G = [torch.randn(m, n, generator=g) for _ in range(2)]
+    W = [torch.randn(m, n, generator=g) for _ in range(2)]
+    k = L.Kron2d()
+    k.nb, k.prec, k.m, k.n, k.g_dtype, k.p_dtype = 2, L.PREC_F32, m, n, L.F32, L.F32
+    k.kind[0] = k.kind[1] = L.FACTOR_DENSE
+    dP, dG, dW = [[p.to(DEV) for p in ps] for ps in P], [x.to(DEV) for x in G], [x.to(DEV) for x in W]
+    for b in range(2):
+        k.G[b] = dG[b].data_ptr()
+        for f in range(2):
+            k.P[f][b] = k.Q[f][b] = k.L[f][b] = dP[b][f].data_ptr()
+    pre = [torch.full((m, n), float("nan"), device=DEV) for _ in range(2)]
+    o = L.ApplyOpts(1e-3, 0.5, 1.0, 0)
+    args = (k, o, L.ptrs(dW), L.ptrs(pre), None)
+    sz, st = ctypes.c_size_t(0), L.stream_of(dG[0])
+    L.check(engine.psgdk_kron2d_apply(*args, None, ctypes.byref(sz), st))
+    ws = torch.full((sz.value + 8192,), 0xA5, dtype=torch.uint8, device=DEV)
+    L.check(engine.psgdk_kron2d_apply(*args, ctypes.c_void_p(ws.data_ptr() + 4096), ctypes.byref(sz), st))
+    assert (ws[:4096] == 0xA5).all() and (ws[4096 + sz.value:] == 0xA5).all()
+    for b in range(2):
+        x = P[b][0].double() @ G[b].double() @ P[b][1].double()
+        assert rel_err_norm(pre[b], x) < 1e-6
+        rms = x.square().mean().sqrt()
+        step = (x * (0.5 / rms) if rms > 0.5 else x).clamp(-1.0, 1.0)
+        assert rel_err_norm(W[b].double() - dW[b].double().cpu(), 1e-3 * step) < 1e-4  # W - step rounds at 2^-24 of W

@@ -194,6 +194,31 @@ def test_workspace_queries_need_no_device():
                                    None) == L.EWORKSPACE
 
 
+@pytest.mark.parametrize("m,n", [(1032, 1032), (1531, 700), (24, 5000)])
+def test_apply_workspace_holds_every_configurations_partials(m, n):
+    """The application's workspace has room for the sum-of-squares partials (two floats per tile) of the converting
+    engine's smallest tile of that epilogue, 32 x 64, whatever option 13 says when the size is queried and when the
+    application runs."""
+    lib, sz, sizes = L.lib(), C.c_size_t(0), set()
+    g = L.Kron2d()
+    g.nb, g.prec, g.m, g.n = 2, L.PREC_F32, m, n
+    g.kind[0] = g.kind[1] = L.FACTOR_DENSE
+    for b in range(2):
+        g.G[b] = 0x1000
+        for f in range(2):
+            g.Q[f][b] = g.P[f][b] = g.L[f][b] = 0x1000
+    try:
+        for cfg in (-1, 0, 1, 2, 3):
+            assert lib.psgdk_set_option(13, cfg) == 0
+            assert lib.psgdk_kron2d_apply(g, L.ApplyOpts(1e-3, 2.0, 10.0, 0), None, None, None, None, C.byref(sz),
+                                          None) == L.OK
+            sizes.add(sz.value)
+    finally:
+        lib.psgdk_set_option(13, -1)
+    tiles = -(-m // 32) * -(-n // 64)
+    assert len(sizes) == 1 and sizes.pop() >= 2 * 4 * (2 * m * n + 2 * tiles)
+
+
 def test_group_validation():
     lib = L.lib()
     sz = C.c_size_t(0)
