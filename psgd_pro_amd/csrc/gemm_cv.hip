@@ -5,11 +5,13 @@
 // The operands are read as stored, converted in registers and staged in LDS as k-contiguous bf16, so that all of them
 // run on the bf16 MFMA (2.5 PFLOP/s dense; the fp32 MFMA does 0.157):
 //   bf16 precision: each value rounded to bfloat16 (round to nearest even), one product.
-//   fp32 precision: each value x split exactly into three bfloat16 planes, x = h + m + l with h = bf16(x),
+//   fp32 precision: each value times 2^16, x, split exactly into three bfloat16 planes, x = h + m + l with h = bf16(x),
 //     m = bf16(x - h), l = bf16(x - h - m) (8 + 8 + 8 significant bits; both differences are exact), and the six
 //     products h h', h m', m h', m m', h l', l h' accumulated in fp32. The three dropped ones are below 2^-23 |x x'|
 //     together in the worst case and about 2^-27 with either sign on random values, under the 2^-24 of the
-//     accumulation itself.
+//     accumulation itself. The factor, taken out of the sums again, changes no rounding, and with it the split is exact
+//     down to the least subnormal: bfloat16 ends at 2^-133 (the MFMA keeps its subnormals), so that below 2^-110 an
+//     unscaled l, and then m, lose their bits (operands near 1e-36: error 2.6e-5).
 // The k loop accumulates blocks of k and folds each block into a second accumulator set: one fp32 chain over all of K
 // carries several times the rounding error of blocked summation.
 //
@@ -25,8 +27,8 @@
 //   128 x 256 tiles: registers for one accumulator set per block only; blocks of 64 k, and every other block is
 //     computed negated and subtracted, so that what truncation is left cancels between blocks (1.8e-7 at k 3072,
 //     against 2.2e-7).
-// Infinities, NaNs and values over the bfloat16 range leave NaN in x - h, hence non-finite sums: a workgroup whose
-// accumulators are not all finite repeats its tile with fp32 MFMAs (mma_f32), whose results are IEEE's.
+// Infinities, NaNs, values from 2^112 on and sums from 2^96 on leave non-finite sums: a workgroup whose accumulators are
+// not all finite repeats its tile with fp32 MFMAs (mma_f32), whose results are IEEE's.
 //
 // What bounds it. fp32, 128 x 256: a 32-k stage is 3072 MFMA cycles per SIMD pair of waves against about 180 VALU
 // instructions of address, split and store per converting wave, 72 KB of LDS writes and 144 KB of fragment reads: two
@@ -54,6 +56,7 @@ typedef float f32x4u_t __attribute__((ext_vector_type(4), aligned(4)));
 
 constexpr int NT = 256;      // threads that stage one operand tile together
 constexpr int KS32 = 32;     // k of one LDS slice (a plane row of 64 bytes)
+constexpr float kSplitScale = 65536.f;  // lifts fp32's last bit, 2^-149, to bfloat16's, 2^-133
 
 __device__ __forceinline__ uint32_t cvt2(float lo, float hi) {  // two values to bfloat16, round to nearest even
   return __builtin_bit_cast(uint32_t, __builtin_convertvector(f32x2_t{lo, hi}, bf16x2_t));
@@ -218,14 +221,12 @@ struct CvTile {
   }
 
   // into NP bf16 planes of KS slices of TROWS rows x 32 k, from row `row0` on (a multiple of 16)
-  // (flip: the sign bit to negate the values by, or 0)
-  template <int NP, int TROWS, bool FLIP>
-  __device__ __forceinline__ void store(unsigned char* lds, int row0, const CvOperand& o, uint32_t flip = 0) const {
+  // (three planes: of the values times `scale`, +- kSplitScale)
+  template <int NP, int TROWS>
+  __device__ __forceinline__ void store(unsigned char* lds, int row0, const CvOperand& o, float scale) const {
     lds += row0 * 64;
     each(o, [&](unsigned row, unsigned kv, int i, f32x4_t x) {
-      if constexpr (FLIP)
-        x = f32x4_t{__uint_as_float(__float_as_uint(x.x) ^ flip), __uint_as_float(__float_as_uint(x.y) ^ flip),
-                    __uint_as_float(__float_as_uint(x.z) ^ flip), __uint_as_float(__float_as_uint(x.w) ^ flip)};
+      if constexpr (NP == 3) x = f32x4_t{x.x * scale, x.y * scale, x.z * scale, x.w * scale};
       // rows i apart (below 4 from a multiple of 4, or a multiple of 16) keep the slot's XOR: a constant offset
       unsigned char* q = lds + (kv >> 3) * (TROWS * 64) + cv_slot(row, (kv & 7) >> 1) + (kv & 1) * 8 + i * 64;
       const uint2 h = make_uint2(cvt2(x.x, x.y), cvt2(x.z, x.w));
@@ -459,9 +460,9 @@ __global__ void __launch_bounds__(WN == 4 || KG == 2 ? 512 : 256, 2) gemm_cv_ker
   // each operand's tile in registers is converted and stored and the tile kt requested into its place at once
   // (neg: A's values negated)
   auto stage = [&](unsigned char* st, bool neg, int kt) INL {
-    la.template store<NP, BM, NP == 3 && SHARE>(st, ha, oa, neg ? 0x80000000u : 0u);
+    la.template store<NP, BM>(st, ha, oa, neg ? -kSplitScale : kSplitScale);
     load_a(kt);
-    lb.template store<NP, BN, false>(st + NP * AB, hb, ob);
+    lb.template store<NP, BN>(st + NP * AB, hb, ob, kSplitScale);
     load_b(kt);
   };
   // tile i holds the own k of its rows, in a Gram product's diagonal tile
@@ -531,6 +532,7 @@ __global__ void __launch_bounds__(WN == 4 || KG == 2 ? 512 : 256, 2) gemm_cv_ker
     }
   }
   const bool out = SHARE || h == 0;  // the wave holds results
+  if constexpr (NP == 3) each_acc([&](int i, int j, int e) INL { acc[i][j][e] *= 1.f / (kSplitScale * kSplitScale); });
   if constexpr (NP == 3) {  // the same tile by fp32 MFMAs: on request, or where a sum is not finite
     bool fin = !p.f32;
     if (out) each_acc([&](int i, int j, int e) INL { fin = fin && fabsf(acc[i][j][e]) < INFINITY; });

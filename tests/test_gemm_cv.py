@@ -82,6 +82,24 @@ def test_converting_engine(engine, m, n, k, bf16):
     _check(C[ok], A[ok], B, False, "finite rows")
 
 
+def test_operands_far_from_one(engine):
+    """fp32 products keep fp32's accuracy over its range: operands down to its subnormals (whole matrices, and single rows
+    and columns of ordinary ones), sums beyond what the scaled split can hold, and operands beyond it."""
+    m, n, k = 70, 130, 96
+    A, B = _rnd(m, k, 5), _rnd(k, n, 6)
+    for ea, eb in ((-100, 90), (-113, 100), (-121, 100), (-126, 110), (-136, 100), (100, -113), (90, -136), (60, 50),
+                   (120, -30), (-126, 120)):
+        a, b = torch.ldexp(A, torch.tensor(ea, device=DEV)), torch.ldexp(B, torch.tensor(eb, device=DEV))
+        _check(K.gemm(a, b, False, False, False), a, b, False, (ea, eb))
+        _check(K.symm_right(a.T, torch.ldexp(_rnd(m, m, 7), torch.tensor(eb, device=DEV)), -1, False), a.T,
+               (lambda u: u - u.T)(torch.ldexp(torch.triu(_rnd(m, m, 7), 1), torch.tensor(eb, device=DEV))), False, "symm")
+    rows = torch.tensor([-120 if i % 5 == 3 else -136 if i % 5 == 1 else 0 for i in range(m)], device=DEV)
+    cols = torch.tensor([-119 if j % 7 == 2 else 0 for j in range(n)], device=DEV)
+    a, b = torch.ldexp(A, rows[:, None]), torch.ldexp(B, cols[None])
+    C = K.gemm(a, torch.ldexp(b, torch.tensor(40, device=DEV)), False, False, False)
+    _check(C, a, torch.ldexp(b, torch.tensor(40, device=DEV)), False, "rows")
+
+
 @pytest.mark.parametrize("cfg", [-1, 1, 3])
 def test_gram_diagonal_keeps_its_small_squares(cfg):
     """X^T X for X near the identity: the small squares beside a diagonal entry's large one are not lost to its
