@@ -16,7 +16,8 @@
 // carries several times the rounding error of blocked summation.
 //
 // Rounding. Measured on gfx950: the bf16 MFMA aligns the 8 products of a lane to the largest of them and truncates each
-// toward zero there at 24 bits, then adds the lane groups' sums and C with rounding. fp32 sums must not pay for that:
+// toward zero there at 24 bits (1 + 2^-25 and 1 - 2^-25 give 1); the lane groups' sums and C are then added to the nearest,
+// but for what a much larger C leaves of them (below). fp32 sums must not pay for that:
 //   64- and 32-row tiles: h h' enters an MFMA with C = 0 and is added to the block by a VALU add, and the five small
 //     products have accumulators of their own, so nothing small is aligned to a large sum. Relative error (Frobenius, k
 //     1024 normals) 7.4e-8; one fp32 MFMA chain folded every 128 k: 2.1e-7.
@@ -24,9 +25,12 @@
 //     preconditioner factor) one square outweighs the other 7 of its lane, whose truncation then always lowers the
 //     diagonal (by 7e-8 of it, which the norm bound of the next product sees doubled): there a row's
 //     own k has an h h' MFMA to itself. Gram products keep to these tiles.
-//   128 x 256 tiles: registers for one accumulator set per block only; blocks of 64 k, and every other block is
-//     computed negated and subtracted, so that what truncation is left cancels between blocks (1.8e-7 at k 3072,
-//     against 2.2e-7).
+//   128 x 256 tiles: registers for one accumulator set per block only, with all six products on top of it. Bits of a
+//     small product below the last of a large C are dropped downward (mean error of 3072^3 -5e-8 of the results' rms), so
+//     every other block is computed negated and subtracted (mean below 1e-10). Longer blocks cost roundings inside them,
+//     more blocks cost roundings of the whole sum, which matter for operands of one sign: blocks of 64 k up to k 1280, of
+//     128 above. Errors of 64, of 128 and of fp32 MFMA chains of 128, in 1e-8: random signs, k 1024 14.7, 18.3, 21.1, k 3072
+//     17.9, 19.7, 22.3; one sign, k 1280 7.2, 6.9, 7.4, k 1536 7.13, 6.6, 7.06, k 3072 9.5, 7.4, 7.6.
 // Infinities, NaNs, values from 2^112 on and sums from 2^96 on leave non-finite sums: a workgroup whose accumulators are
 // not all finite repeats its tile with fp32 MFMAs (mma_f32), whose results are IEEE's.
 //
@@ -321,8 +325,11 @@ __global__ void __launch_bounds__(WN == 4 || KG == 2 ? 512 : 256, 2) gemm_cv_ker
   // sums folded so far, the current block's, and (three planes, small tiles) all five small products' of the whole k range
   constexpr bool SM = NP == 3 && !SHARE;
   constexpr bool GRAM = SM && EPI == EPI_STORE && BM == BN && LAY == 3;  // X^T X among them
-  // k tiles per accumulation block: of 64 k where truncation is left to cancel (see the file's comment), else of 128
-  constexpr int BT = (SHARE && NP == 3 ? 64 : 128) / BK;
+  // an accumulation block has 2^bs k tiles: 128 k, or the large tile's 64 (see the file's comment)
+  constexpr int BT = 128 / BK, BS = BT == 4 ? 2 : 1;
+  static_assert(BT == 1 << BS, "a power of two");
+  const int bs = SHARE && NP == 3 && p.K <= 1280 ? BS - 1 : BS;
+  auto block_end = [&](int kt, int n) INL { return (kt + 1 & (1 << bs) - 1) == 0 || kt + 1 == n; };
   Acc acc[FM][FN], blk[FM][FN], sm[FM][FN];
   auto each_acc = [&](auto f) INL {
 #pragma unroll
@@ -469,7 +476,7 @@ __global__ void __launch_bounds__(WN == 4 || KG == 2 ? 512 : 256, 2) gemm_cv_ker
   static_assert(!GRAM || BK == BM, "the k of a diagonal tile's rows are one tile");
   auto gram = [&](int i) INL { return GRAM && p.tri && m0 == n0 && kbeg + (KG * i + h) * BK == m0; };
   // tile i belongs to a negated block
-  auto odd = [&](int i) INL { return NP == 3 && SHARE && (i / BT & 1) != 0; };
+  auto odd = [&](int i) INL { return NP == 3 && SHARE && (i >> bs & 1) != 0; };
   zero();
   if (nk > 0 && (NP == 1 || !p.f32)) {
     if constexpr (SHARE) {
@@ -485,7 +492,7 @@ __global__ void __launch_bounds__(WN == 4 || KG == 2 ? 512 : 256, 2) gemm_cv_ker
         __syncthreads();
         if (kt >= 0) {
           mma_planes(at(kt), false);
-          if ((kt + 1) % BT == 0 || kt + 1 == nk) fold(odd(kt));
+          if (block_end(kt, nk)) fold(odd(kt));
           __syncthreads();
         }
       }
@@ -502,7 +509,7 @@ __global__ void __launch_bounds__(WN == 4 || KG == 2 ? 512 : 256, 2) gemm_cv_ker
         stage(st, odd(i), (i + 1) * KG + h);
         __syncthreads();
         mma_planes(st, gram(i));
-        if ((i + 1) % BT == 0 || i + 1 == n) fold(odd(i));
+        if (block_end(i, n)) fold(odd(i));
         __syncthreads();
       }
       if (KG == 2 && h == 0) __syncthreads();
@@ -548,7 +555,7 @@ __global__ void __launch_bounds__(WN == 4 || KG == 2 ? 512 : 256, 2) gemm_cv_ker
         __syncthreads();
         if (out) {
           mma_f32();
-          if ((kt + 1) % BT == 0 || kt + 1 == nk) fold(false);
+          if (block_end(kt, nk)) fold(false);
         }
         __syncthreads();
       }

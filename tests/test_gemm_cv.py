@@ -82,6 +82,28 @@ def test_converting_engine(engine, m, n, k, bf16):
     _check(C[ok], A[ok], B, False, "finite rows")
 
 
+@pytest.mark.parametrize("k", [512, 1280, 1288, 3072])
+@pytest.mark.parametrize("sign", [False, True])
+def test_split_products_are_no_further_off_than_fp32_mfmas(engine, k, sign):
+    """Against float64, the fp32 products by splits are as close as fp32 MFMA chains of 128 k (option 8 = 0, 64 x 64
+    tiles) for operands of random and of one sign: there the sum of the blocks bounds both, which the splits must not cut
+    shorter for long k. One percent for the two samples of the same rounding."""
+    g = torch.Generator().manual_seed(k)
+    A, B = torch.randn(256, k, generator=g), torch.randn(k, 512, generator=g)
+    if sign:
+        A, B = A.abs(), B.abs()
+    a, b, R = A.to(DEV), B.to(DEV), A.double() @ B.double()
+    C = K.gemm(a, b, False, False, False)
+    cfg = ctypes.c_int(0)
+    L.check(engine.psgdk_get_option(13, ctypes.byref(cfg)))
+    L.check(engine.psgdk_set_option(13, 1))
+    L.check(engine.psgdk_set_option(8, 0))
+    ref = rel_err_norm(K.gemm(a, b, False, False, False), R)
+    L.check(engine.psgdk_set_option(8, 1))
+    L.check(engine.psgdk_set_option(13, cfg.value))
+    assert rel_err_norm(C, R) < 1.01 * ref, (rel_err_norm(C, R), ref)
+
+
 def test_operands_far_from_one(engine):
     """fp32 products keep fp32's accuracy over its range: operands down to its subnormals (whole matrices, and single rows
     and columns of ordinary ones), sums beyond what the scaled split can hold, and operands beyond it."""
