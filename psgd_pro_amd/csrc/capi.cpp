@@ -536,7 +536,7 @@ int nlb_vmm(int64_t n, int sign, int nb, const float* const* A, int64_t lda, con
   return run_gemm(PSGDK_PREC_F32, nb, NLB_K, n, n, oa, ob, C, n, e, 0, 0, 0, w.splits, w.kchunk, st);
 }
 
-// Row statistics of matrices read from their upper triangle, then (a.Vin set) V0.
+// Row statistics of matrices read from their upper triangle, then V0.
 int nlb_tri_start(NlbArgs a, hipStream_t st) {
   PSGDK_HIP(nlb_rownorm_launch(a, st), "tri_rownorm");
   for (int b = 0; b < a.nb; ++b) { a.rpart[b] = a.rstat[b]; a.cpart[b] = a.rstat[b] + a.n; }
@@ -1800,9 +1800,8 @@ int psgdk_tri_rownorm2(int64_t n, int sign, int nb, const float* const* A, int64
   if (sign != 1 && sign != -1) return fail(PSGDK_EINVAL, "sign = %d", sign);
   if (lda < n) return fail(PSGDK_ESHAPE, "lda < n");
   NlbArgs a = nlb_args(n, sign, nb, A, lda, nw);
-  for (int b = 0; b < nb; ++b) { a.rn2[b] = rn2[b]; a.amax_out[b] = amax[b]; a.Vin[b] = nullptr; }
-  hipStream_t st = (hipStream_t)stream;
-  return nlb_tri_start(a, st);
+  for (int b = 0; b < nb; ++b) { a.rn2[b] = rn2[b]; a.amax_out[b] = amax[b]; }
+  return hip_check(nlb_rownorm_launch(a, (hipStream_t)stream), "tri_rownorm");
 }
 
 int psgdk_tri_vmm(int64_t n, int sign, int nb, const float* const* V, const float* const* A, int64_t lda,

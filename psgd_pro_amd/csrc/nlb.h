@@ -45,7 +45,7 @@ struct NlbArgs {
   float* rstat[MAXB];       // 2 n: per row max |A_ij| (of its tile row), then the diagonal
   float* rn2[MAXB];         // n squared row norms
   float* scal[MAXB];        // NLB_NSCAL scalars
-  float* amax_out[MAXB];    // optional: max |A_ij| of the stored triangle (init)
+  float* amax_out[MAXB];    // optional: max |A_ij| of the stored triangle (tri_rowstats)
 };
 
 enum : int { NLB_FINAL_NONE = 0, NLB_FINAL_FACTOR = 1, NLB_FINAL_SCALE = 2 };
@@ -77,7 +77,7 @@ hipError_t nlb_rownorm_launch(const NlbArgs& a, hipStream_t st);
 hipError_t nlb_reduce_launch(const NlbArgs& a, int normalize_in, hipStream_t st);
 hipError_t nlb_final_launch(const NlbArgs& a, const NlbFinal& f, hipStream_t st);
 // fully stored matrices: stage 0 row norms (rn2, rpart = row max |A|, cpart = diagonal), 1 init, 2 one V A product,
-// 4 init from the upper triangle only (fp32; without Vin the row statistics' results alone),
+// 4 init from the upper triangle only (fp32),
 // 3 the stage-0 outputs of a skew matrix from the per-(row, 64-column block) partials its producer left in part
 hipError_t nlb_full_launch(const NlbArgs& a, int stage, int a_bf16, int normalize, hipStream_t st);
 // the whole bound (a.Vin the start) of fully stored matrices of at most NLB_SMALL_N, bf16 in the 16-byte layout

@@ -78,6 +78,7 @@ __global__ void __launch_bounds__(256) tri_rownorm_kernel(const NlbArgs p) {
 // in order, then the four), rstat[i] = the largest |A_ij| over the stored tiles of row i's tile row (its maximum over all
 // rows is max |A|), rstat[n + i] = A_ii. One workgroup per 64 rows. (As part of a one-workgroup init kernel these sums,
 // n ceil(n / 64) dependent loads by one workgroup, and V0 took 70 us at n 2048; 4.5 us here and 9 us there now.)
+// amax_out (row norms without a bound): max |A| itself, by the first workgroup of the matrix from all of tmax.
 // grid: nb * T workgroups of 256 threads.
 __global__ void __launch_bounds__(256) tri_rowstats_kernel(const NlbArgs p) {
   __shared__ float ps[4][RT];
@@ -92,6 +93,12 @@ __global__ void __launch_bounds__(256) tri_rowstats_kernel(const NlbArgs p) {
   const float* __restrict__ tm = p.tmax[b] + (long long)X * T - (long long)X * (X - 1) / 2;
   for (int t = tid; t < T - X; t += 256) m = fmaxf(m, tm[t]);
   m = block_max(m, red);
+  if (X == 0 && p.amax_out[b]) {
+    float am = 0.f;
+    for (int t = tid; t < T * (T + 1) / 2; t += 256) am = fmaxf(am, p.tmax[b][t]);
+    am = block_max(am, red);
+    if (tid == 0) p.amax_out[b][0] = am;
+  }
   if (q == 0 && i < n) {
     p.rn2[b][i] = (((ps[0][r] + ps[1][r]) + ps[2][r]) + ps[3][r]) + p.cpart[b][i];
     p.rstat[b][i] = m;
@@ -301,8 +308,7 @@ __device__ __forceinline__ void store4(float* dst, const float (&x)[4]) {
 // :49-57). Workgroup r = 0 also publishes nf and j. The scans read 4 (statistics) or 8 (rows) elements per thread
 // and step with the loads of several steps in flight; the rows take the element path unless n % 8 == 0, A's row
 // stride is a multiple of 16 bytes and the bases are 16-byte aligned. TRI: only A's upper triangle is read (row j's part
-// left of the diagonal from column j); without a start V (of any matrix) one workgroup per matrix publishes the row
-// statistics' results alone.
+// left of the diagonal from column j).
 template <typename T, bool TRI>
 __global__ void __launch_bounds__(256) nlb_init_full_kernel(const NlbArgs p) {
   __shared__ float red[4];
@@ -310,16 +316,14 @@ __global__ void __launch_bounds__(256) nlb_init_full_kernel(const NlbArgs p) {
   __shared__ int sidx[4];
   __shared__ float snf;
   __shared__ int sj;
-  const int rows = !TRI || p.Vin[0] ? NLB_K : 1;  // workgroups per matrix
-  const int b = blockIdx.x / rows, r = blockIdx.x % rows;
+  const int b = blockIdx.x / NLB_K, r = blockIdx.x % NLB_K;
   const int tid = threadIdx.x, n = p.n;
   const float* __restrict__ rn2 = p.rn2[b];
   const float* __restrict__ rmax = p.rpart[b];
   const float* __restrict__ diag = p.cpart[b];
   float best = -1.f, am = 0.f, dm = -INFINITY;
   int bi = 0x7fffffff;
-  // workspace arrays: 256-byte aligned bases (rn2 may be the caller's)
-  if ((n & 3) == 0 && (!TRI || (reinterpret_cast<uintptr_t>(rn2) & 15) == 0)) {
+  if ((n & 3) == 0) {  // workspace arrays: 256-byte aligned bases
     const int n4 = n >> 2;
 #pragma unroll 4
     for (int i = tid; i < n4; i += 256) {
@@ -360,10 +364,8 @@ __global__ void __launch_bounds__(256) nlb_init_full_kernel(const NlbArgs p) {
     if (r == 0) {
       p.scal[b][NLB_NF] = nf;
       p.scal[b][NLB_J] = (float)sj;
-      if (TRI && p.amax_out[b]) p.amax_out[b][0] = am;
     }
   }
-  if (TRI && !p.Vin[b]) return;
   __syncthreads();
   const T* __restrict__ arow = reinterpret_cast<const T*>(p.A[b]) + (long long)sj * p.lda;
   const int j = sj;
@@ -1540,7 +1542,7 @@ hipError_t nlb_full_launch(const NlbArgs& a, int stage, int a_bf16, int normaliz
     if (a_bf16) hipLaunchKernelGGL((nlb_init_full_kernel<bf16_t, false>), grid, dim3(256), 0, st, a);
     else hipLaunchKernelGGL((nlb_init_full_kernel<float, false>), grid, dim3(256), 0, st, a);
   } else if (stage == 4) {
-    hipLaunchKernelGGL((nlb_init_full_kernel<float, true>), dim3(a.nb * (a.Vin[0] ? NLB_K : 1)), dim3(256), 0, st, a);
+    hipLaunchKernelGGL((nlb_init_full_kernel<float, true>), dim3(a.nb * NLB_K), dim3(256), 0, st, a);
   } else if (a.vmm_cols) {
     const dim3 grid(((a.n + VMC - 1) / VMC) * a.nb);
     if (a.vmm_cols == 4) {
