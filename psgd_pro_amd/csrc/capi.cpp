@@ -577,13 +577,14 @@ int nlb_iterate(NlbArgs a, const NlbFinal& fin, const NlbWs& w, hipStream_t st, 
   return hip_check(nlb_final_launch(a, fin, st), "nlb_final");
 }
 
-// The 16-column V A kernel reads any fp32 matrix of less than 2 GiB (and bf16 ones in the layout above).
+// The 16-column V A kernel reads any fp32 matrix whose chunks of 512 rows are under 2 GiB (and bf16 ones in the layout
+// above).
 bool strip_ok(int64_t n, int64_t lda, int a_bf16) {
-  return !a_bf16 && n * lda < ((int64_t)1 << 29) && NLB_K * n < ((int64_t)1 << 29);
+  return !a_bf16 && lda < (1 << 20) && NLB_K * n < ((int64_t)1 << 29);
 }
 
-// Bounds of matrices read from their upper triangle only: the 16-column kernel below 2 GiB, else split-K products on the
-// converting engine.
+// Bounds of matrices read from their upper triangle only: the 16-column kernel, or (rows 4 MiB apart or more) split-K products
+// on the converting engine.
 int run_nlb(int64_t n, int sign, int nb, const float* const* A, int64_t lda, const float* const* V, const NlbFinal& fin,
             const NlbWs& w, hipStream_t st) {
   NlbArgs a = nlb_args(n, sign, nb, A, lda, w);

@@ -7,7 +7,7 @@
 //                 (deterministic partial slots, no float atomics) and per-tile max |A_ij|
 //   tri_rowstats: a workgroup per 64 rows: squared row norms (partials in a fixed order), row maxima, the diagonal
 //   nlb_init    : a workgroup per (matrix, row of V): argmax (first maximum), nf, V0 (nlb_init_full_kernel)
-//   V A products: vmm_strip_kernel; for matrices of 2 GiB and more, the converting engine (M = 32, B read from the
+//   V A products: vmm_strip_kernel; for leading dimensions from 2^20 on, the converting engine (M = 32, B read from the
 //                 triangle), split over k, partials in ws, and
 //   nlb_reduce  : sums the k-split partials in a fixed order, scales the rows by 1/nf and by the input row
 //                 normalisation 1/(|V_in,r| + smallest normal) (exact: the product is linear in each row of V),
@@ -954,11 +954,13 @@ __global__ void __launch_bounds__(256) vmm_rows_kernel(const NlbArgs p, int norm
 // whose 64-column blocks would leave CUs idle (n 1024: 64 workgroups instead of 16; every workgroup reads all of V, 32
 // rows against its 16 of A, from L2). The k range goes through LDS in chunks of 2 KB per row; wave w multiplies the k
 // eighth w of a chunk (4 MFMA steps, V fragments straight from global memory); the next chunk's loads are in flight
-// meanwhile. The waves' partial blocks are summed through LDS in the order w = 0..7.
+// meanwhile. STEPS of them (4: 64 k in fp32) are summed by themselves, the waves' partial blocks through LDS in pairs (one
+// chain over a wave's k: the product of n 4096 4.2e-7 off float64 normwise, now 1.9e-7; fp32 n 2048 bound 97 us, now 98).
 // TRI (fp32): A is read from its upper triangle. Column c's k below the block's first column c0 are stored in rows k:
 // chunks of 512 rows x 16 columns, [k][c] in LDS (rows of 20 floats: the 64 lanes of a fragment read hit 64 banks),
 // negated for skew matrices; from c0 on they are stored in row c, and the 16 x 16 block at the diagonal is completed in
-// LDS from its upper half. (A_sym^T is what is multiplied, as by the kernels that read rows in full.)
+// LDS from its upper half. (A_sym^T is what is multiplied, as by the kernels that read rows in full. STEPS 2: a
+// product by itself, without scal and ssout, times the sign instead, V A_sym; its chains are two steps: 1.5e-7.)
 // Latency-bound at these sizes: about 8 us per product of n 2048 fp32 from full storage (21 on 64-column blocks), 13 from
 // the triangle (18 and a 4 us reduce by split-K products).
 // bf16 needs the operand layout of vmm_cols_kernel; fp32 rows may start at any 4-byte boundary (16-byte loads checked by
@@ -966,7 +968,7 @@ __global__ void __launch_bounds__(256) vmm_rows_kernel(const NlbArgs p, int norm
 // grid: nb * ceil(n / 16).
 constexpr int VS_C = 16, VS_LD = 20;  // columns per workgroup; row pitch (floats) of a [k][c] chunk
 
-template <typename T, bool TRI, bool ODD>
+template <typename T, bool TRI, bool ODD, int STEPS>
 __global__ void __launch_bounds__(512, 4) vmm_strip_kernel(const NlbArgs p, int normalize) {
   constexpr int CE = 16 / sizeof(T), CK = 2048 / sizeof(T);  // elements per 16-byte piece; k per chunk
   constexpr int KS = 4 * CE;                                 // k per MFMA step
@@ -979,17 +981,19 @@ __global__ void __launch_bounds__(512, 4) vmm_strip_kernel(const NlbArgs p, int 
   const int r16 = lane & 15, g = lane >> 4;
   const T* __restrict__ V = reinterpret_cast<const T*>(p.Vin[b]);
   const __amdgpu_buffer_rsrc_t rv = make_rsrc(V, (long long)NLB_K * n * sizeof(T));
-  const __amdgpu_buffer_rsrc_t ra = make_rsrc(p.A[b], ((n - 1) * p.lda + n) * (long long)sizeof(T));
   const int lda = (int)p.lda;
   uint4 st[4], vn[4][2];
   // chunk of k kc .. kc + CK - 1, none at or past kend: A's rows c0 .. (piece tid % 128 of rows tid / 128 + 4 i), or
-  // (cols) rows kc .. (piece tid % 4 of rows tid / 4 + 128 i)
+  // (cols) rows kc .. (piece tid % 4 of rows tid / 4 + 128 i). Offsets are relative to the first of these rows.
   auto load = [&](int kc, int kend, bool cols) {
+    const int row0 = cols ? kc : c0;
+    const __amdgpu_buffer_rsrc_t ra = make_rsrc(reinterpret_cast<const T*>(p.A[b]) + row0 * p.lda,
+                                                ((n - 1 - row0) * p.lda + n) * (long long)sizeof(T));
 #pragma unroll
     for (int i = 0; i < 4; ++i) {
-      const int row = cols ? kc + (tid >> 2) + 128 * i : c0 + (tid >> 7) + 4 * i;
+      const int row = cols ? (tid >> 2) + 128 * i : (tid >> 7) + 4 * i;
       const int col = cols ? c0 + (tid & 3) * CE : kc + (tid & 127) * CE;
-      const bool in = cols ? row < kend && col < n : row < n && col < kend;
+      const bool in = cols ? row0 + row < kend && col < n : row0 + row < n && col < kend;
       st[i] = __builtin_bit_cast(
           uint4, __builtin_amdgcn_raw_buffer_load_b128(ra, in ? (row * lda + col) * (int)sizeof(T) : kOob, 0, 0));
     }
@@ -1002,14 +1006,14 @@ __global__ void __launch_bounds__(512, 4) vmm_strip_kernel(const NlbArgs p, int 
                                                  rv, k < kend ? ((i * 16 + r16) * n + k) * (int)sizeof(T) : kOob, 0, 0));
     }
   };
-  f32x4_t acc[2] = {};
+  f32x4_t sum[2] = {};
   const int split = TRI ? c0 : 0;  // k below it are read from rows k
   bool cols = split > 0;
   int kc = 0;
   load(0, cols ? split : n, cols);
   {  // row scales: 16 threads per row
     const int r = tid >> 4, q0 = tid & 15;
-    float sc = 1.f / p.scal[b][NLB_NF];
+    float sc = STEPS == 4 ? 1.f / p.scal[b][NLB_NF] : (float)p.sign;
     if (normalize) {
       float s = 0.f;
       for (int q = q0; q < nbk; q += 16) s += p.ssin[b][r * nbk + q];
@@ -1029,7 +1033,7 @@ __global__ void __launch_bounds__(512, 4) vmm_strip_kernel(const NlbArgs p, int 
       u.w = end ? 0 : u.w;
     };
     int t = tid;
-    if constexpr (TRI && ODD) asm volatile("" : "+v"(t));  // its addresses recomputed per chunk: few registers
+    if constexpr (ODD) asm volatile("" : "+v"(t));  // its addresses recomputed per chunk: few registers
 #pragma unroll
     for (int i = 0; i < 4; ++i) {
       const int row = (t >> 7) + 4 * i;
@@ -1063,6 +1067,7 @@ __global__ void __launch_bounds__(512, 4) vmm_strip_kernel(const NlbArgs p, int 
         __syncthreads();
       }
     }
+    f32x4_t acc[2] = {};
 #pragma unroll
     for (int s = 0; s < 4; ++s) {
       const int piece = wave * 16 + s * 4 + g;  // 16-byte piece of the row this lane's fragment reads
@@ -1088,6 +1093,13 @@ __global__ void __launch_bounds__(512, 4) vmm_strip_kernel(const NlbArgs p, int 
             acc[i] = __builtin_amdgcn_mfma_f32_16x16x4f32(__uint_as_float((&vc[s][i].x)[s4]),
                                                           __uint_as_float((&af.x)[s4]), acc[i], 0, 0, 0);
       }
+      if ((s + 1) % STEPS == 0) {
+#pragma unroll
+        for (int i = 0; i < 2; ++i) {
+          sum[i] += acc[i];
+          acc[i] = {};
+        }
+      }
     }
     __syncthreads();
     if (!more) break;
@@ -1098,17 +1110,18 @@ __global__ void __launch_bounds__(512, 4) vmm_strip_kernel(const NlbArgs p, int 
 #pragma unroll
   for (int i = 0; i < 2; ++i)
 #pragma unroll
-    for (int e = 0; e < 4; ++e) red[wave][16 * i + 4 * g + e][r16] = acc[i][e];
+    for (int e = 0; e < 4; ++e) red[wave][16 * i + 4 * g + e][r16] = sum[i][e];
   __syncthreads();
   const int row = tid >> 4, c = tid & 15;
-  float w = red[0][row][c];
+  float wq[4];
 #pragma unroll
-  for (int q = 1; q < 8; ++q) w += red[q][row][c];
+  for (int q = 0; q < 4; ++q) wq[q] = red[2 * q][row][c] + red[2 * q + 1][row][c];
+  float w = (wq[0] + wq[1]) + (wq[2] + wq[3]);
   w = c0 + c < n ? w * rsl[row] : 0.f;
   if (c0 + c < n) reinterpret_cast<T*>(p.Vout[b])[(long long)row * n + c0 + c] = from_f32<T>(w);
   float sq = w * w;
   for (int o = 1; o < 16; o <<= 1) sq += __shfl_xor(sq, o, 64);
-  if (c == 0) p.ssout[b][row * nbk + cb] = sq;
+  if (STEPS == 4 && c == 0) p.ssout[b][row * nbk + cb] = sq;
 }
 
 // ---------------------------------------------------------------------------------------------------------------
@@ -1548,11 +1561,11 @@ hipError_t nlb_full_launch(const NlbArgs& a, int stage, int a_bf16, int normaliz
     if (a.vmm_cols == 4) {
       const dim3 gs(((a.n + VS_C - 1) / VS_C) * a.nb);
       const bool odd = (a.n & 3) != 0;
-      if (a_bf16) hipLaunchKernelGGL((vmm_strip_kernel<bf16_t, false, false>), gs, dim3(512), 0, st, a, normalize);
-      else if (a.tri && odd) hipLaunchKernelGGL((vmm_strip_kernel<float, true, true>), gs, dim3(512), 0, st, a, normalize);
-      else if (a.tri) hipLaunchKernelGGL((vmm_strip_kernel<float, true, false>), gs, dim3(512), 0, st, a, normalize);
-      else if (odd) hipLaunchKernelGGL((vmm_strip_kernel<float, false, true>), gs, dim3(512), 0, st, a, normalize);
-      else hipLaunchKernelGGL((vmm_strip_kernel<float, false, false>), gs, dim3(512), 0, st, a, normalize);
+      auto go = [&](auto k) { hipLaunchKernelGGL(k, gs, dim3(512), 0, st, a, normalize); };
+      if (a_bf16) go(vmm_strip_kernel<bf16_t, false, false, 4>);
+      else if (a.tri && !a.scal[0]) odd ? go(vmm_strip_kernel<float, true, true, 2>) : go(vmm_strip_kernel<float, true, false, 2>);
+      else if (a.tri) odd ? go(vmm_strip_kernel<float, true, true, 4>) : go(vmm_strip_kernel<float, true, false, 4>);
+      else odd ? go(vmm_strip_kernel<float, false, true, 4>) : go(vmm_strip_kernel<float, false, false, 4>);
     } else if (a.vmm_cols == 3) {  // bf16, square, n a multiple of 128 (an even number of 64-tiles)
       const int T = a.n / VMC;
       hipLaunchKernelGGL(vmm_tri_kernel, dim3(8 * ((a.nb + 7) / 8) * T), dim3(256), 0, st, a, normalize);

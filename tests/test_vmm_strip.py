@@ -65,3 +65,18 @@ def test_row_norms_of_several_matrices(nb, n):
     for m, r, a in zip(mats, rn2, amax):
         assert float(a) == float(m.abs().max())
         assert rel_err_norm(r, m.double().square().sum(1)) < 1e-6
+
+
+@pytest.mark.parametrize("lda", [2 ** 20 - 4, 2 ** 20])
+def test_triangles_past_two_gib(lda):
+    """Rows so far apart that the matrix spans 2.3 GiB: up to 2^20 the 16-column kernel, whose offsets are relative to a
+    chunk's first row, from there on split products of the converting engine. Errors as in the tests above."""
+    n = 600
+    g = torch.Generator().manual_seed(n)
+    X = torch.randn(n, n + 8, generator=g)
+    S, V = X @ X.T / n, torch.randn(32, n, generator=g)
+    wide = torch.full((n, lda), float("nan"), device=DEV)
+    wide[:, :n] = torch.where(torch.ones(n, n).triu().bool(), S, torch.tensor(float("nan"))).to(DEV)
+    dv = V.to(DEV)
+    r = float(norm_lower_bound(S.double(), V.double(), skew=False))
+    assert _bound(L.lib().psgdk_norm_lower_bound, [wide], [dv], 1) == [pytest.approx(r, rel=1e-5)]
