@@ -1824,6 +1824,20 @@ int psgdk_tri_vmm(int64_t n, int sign, int nb, const float* const* V, const floa
   if (sign != 1 && sign != -1) return fail(PSGDK_EINVAL, "sign = %d", sign);
   if (lda < n) return fail(PSGDK_ESHAPE, "lda < n");
   hipStream_t st = (hipStream_t)stream;
+  // the 16-column kernel writes W while other workgroups still read V and A: only where they lie apart
+  bool apart = true;
+  for (int b = 0; b < nb; ++b)
+    for (int c = 0; c < nb; ++c) {
+      const float *w0 = W[b], *w1 = w0 + NLB_K * n;
+      apart = apart && (w1 <= V[c] || V[c] + NLB_K * n <= w0) && (w1 <= A[c] || A[c] + (n - 1) * lda + n <= w0);
+    }
+  if (apart && strip_ok(n, lda, 0)) {
+    NlbArgs a;
+    std::memset(&a, 0, sizeof a);
+    a.nb = nb; a.n = (int)n; a.sign = sign; a.lda = lda; a.vmm_cols = 4; a.tri = 1;
+    for (int b = 0; b < nb; ++b) { a.A[b] = A[b]; a.Vin[b] = V[b]; a.Vout[b] = W[b]; }
+    return hip_check(nlb_full_launch(a, 2, 0, 0, st), "V A");
+  }
   Opnd oa, ob;
   oa.mode = KC; oa.ld = n;
   ob.mode = SYM; ob.sign = sign; ob.ld = lda;

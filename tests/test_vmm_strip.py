@@ -1,6 +1,6 @@
 """Norm bounds of one launch (csrc/nlb.hip, nlb_small_kernel) and those whose V A products run on 16-column workgroups
 (vmm_strip_kernel): matrices read from their upper triangle, launches of few fully stored ones and rows at odd addresses,
-at the edges of the kernels' sides, column blocks and k chunks; and the row norms of groups of triangles."""
+at the edges of the kernels' sides, column blocks and k chunks; and row norms and products of groups of triangles."""
 import pytest
 import torch
 
@@ -67,6 +67,25 @@ def test_row_norms_of_several_matrices(nb, n):
         assert rel_err_norm(r, m.double().square().sum(1)) < 1e-6
 
 
+@pytest.mark.parametrize("in_place", [False, True])
+@pytest.mark.parametrize("n", [7, 130, 513, 1028])
+@pytest.mark.parametrize("sign", [1, -1])
+def test_products_of_triangles(n, sign, in_place):
+    """psgdk_tri_vmm on a group of three, into outputs of its own or over V: V A_sym, NaN below the triangles. Sums of n
+    products in fp32 stay below 1e-6 normwise, as for one matrix."""
+    g = torch.Generator().manual_seed(n)
+    S = [torch.randn(n, n, generator=g) for _ in range(3)]
+    S = [s + s.T if sign > 0 else s - s.T for s in S]
+    V = [torch.randn(32, n, generator=g) for _ in S]
+    up = [torch.where(torch.ones(n, n).triu().bool(), s, torch.tensor(float("nan"))).to(DEV) for s in S]
+    dv = [v.to(DEV) for v in V]
+    W = dv if in_place else [torch.empty_like(v) for v in dv]
+    L.call_ws(L.lib().psgdk_tri_vmm, n, sign, 3, L.ptrs(dv), L.ptrs(up), n, L.ptrs(W), ws=L.Workspace(),
+              device=up[0].device, stream=L.stream_of(up[0]))
+    for w, v, s in zip(W, V, S):
+        assert rel_err_norm(w, v.double() @ s.double()) < 1e-6
+
+
 @pytest.mark.parametrize("lda", [2 ** 20 - 4, 2 ** 20])
 def test_triangles_past_two_gib(lda):
     """Rows so far apart that the matrix spans 2.3 GiB: up to 2^20 the 16-column kernel, whose offsets are relative to a
@@ -77,6 +96,26 @@ def test_triangles_past_two_gib(lda):
     S, V = X @ X.T / n, torch.randn(32, n, generator=g)
     wide = torch.full((n, lda), float("nan"), device=DEV)
     wide[:, :n] = torch.where(torch.ones(n, n).triu().bool(), S, torch.tensor(float("nan"))).to(DEV)
-    dv = V.to(DEV)
+    dv, W = V.to(DEV), torch.empty(32, n, device=DEV)
     r = float(norm_lower_bound(S.double(), V.double(), skew=False))
     assert _bound(L.lib().psgdk_norm_lower_bound, [wide], [dv], 1) == [pytest.approx(r, rel=1e-5)]
+    L.call_ws(L.lib().psgdk_tri_vmm, n, 1, 1, L.ptrs([dv]), L.ptrs([wide]), lda, L.ptrs([W]), ws=L.Workspace(),
+              device=wide.device, stream=L.stream_of(wide))
+    assert rel_err_norm(W, V.double() @ S.double()) < 1e-6
+
+
+def test_products_of_triangles_sum_in_short_chains():
+    """P = 0.5 I + A A^T / 2 at n 4096: V P within 2.5e-7 of float64 normwise. Every rounding after the diagonal's term is
+    of its size, uniform in 2^-24 of it or less: chains of 32 k, 16 sums and 3 of the waves come to 1.5e-7 (measured), one
+    chain over a wave's 512 k to 4.2e-7."""
+    n = 4096
+    g = torch.Generator().manual_seed(1)
+    a = torch.randn(n, n, generator=g).to(DEV) / n ** 0.5
+    P = 0.5 * (a @ a.T)
+    P.diagonal().add_(0.5)
+    P = 0.5 * (P + P.T)
+    V = torch.randn(32, n, generator=g).to(DEV)
+    W = torch.empty_like(V)
+    L.call_ws(L.lib().psgdk_tri_vmm, n, 1, 1, L.ptrs([V]), L.ptrs([P]), n, L.ptrs([W]), ws=L.Workspace(), device=P.device,
+              stream=L.stream_of(P))
+    assert rel_err_norm(W, V.double() @ P.double()) < 2.5e-7
