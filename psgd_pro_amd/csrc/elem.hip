@@ -878,7 +878,8 @@ hipError_t vec_update_launch(const EwArgs& a, hipStream_t st) {
 }
 
 // A vector's whole application: pre = G P (in2 = P, into out where given), its RMS, then clip_update_kernel's arithmetic.
-// in = param (dtype dt), aux = G (dtype i1), out2 = clipped (optional); f0 .. f2 as there. One workgroup per vector.
+// in = param (dtype dt), aux = G (dtype i1), out2 = clipped (optional); f0 .. f2 as there. One workgroup per vector. out may
+// be G or P itself: the second pass reads pre from there.
 __global__ void __launch_bounds__(1024) vec_apply_kernel(const EwArgs a) {
   __shared__ float red[16];
   const int b = blockIdx.x;
@@ -897,7 +898,7 @@ __global__ void __launch_bounds__(1024) vec_apply_kernel(const EwArgs a) {
   void* prm = const_cast<void*>(a.in[b]);
   float* gout = reinterpret_cast<float*>(a.out2[b]);
   for (long long i = threadIdx.x; i < a.m; i += blockDim.x) {
-    float g = pre(i);
+    float g = a.out[b] ? a.out[b][i] : pre(i);
     if (scale) g *= sc;
     g = clamp_keep_nan(g, a.f1);
     if (gout) gout[i] = g;
