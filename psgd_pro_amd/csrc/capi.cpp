@@ -413,7 +413,7 @@ int run_gemm(int prec, int nb, int64_t M, int64_t N, int64_t K, const Opnd& A, c
     a.A[b] = A.p[b]; a.B[b] = B.p[b]; a.C[b] = C[b];
     a.X1[b] = e.X1[b]; a.X2[b] = e.X2[b]; a.s[b] = e.s[b]; a.part[b] = e.part[b];
   }
-  const int cfg = cv_cfg(prec, M, N, tri, nb, e.epi, !gemm_cv_wide(a),
+  const int cfg = cv_cfg(prec, M, N, tri, nb, e.epi, !gemm_cv_wide(a, prec),
                          prec == PSGDK_PREC_F32 && tri && e.epi == EPI_STORE && A.mode == MC);
   if (ntiles) *ntiles = gemm_cv_tiles(M, N, tri, cfg);
   if (!g_prof.on) return hip_check(gemm_cv_launch(a, prec, cfg, st), "gemm launch");

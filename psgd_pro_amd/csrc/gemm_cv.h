@@ -37,9 +37,9 @@ struct CvArgs {
   float* part[MAXB];
 };
 
-// Tile configurations: 0 = 128 x 256 (fp32 rows, not A m- with B k-contiguous: gemm_cv_wide), 1 = 64 x 64, 2 = 32 x 64
-// (EPI_STORE and EPI_SUMSQ only), 3 = 64 x 64 with k split over two wave groups
-bool gemm_cv_wide(const CvArgs& a);
+// Tile configurations: 0 = 128 x 256 (plain rows of one storage type, not A m- with B k-contiguous: gemm_cv_wide), 1 = 64
+// x 64, 2 = 32 x 64 (EPI_STORE and EPI_SUMSQ only), 3 = 64 x 64 with k split over two wave groups
+bool gemm_cv_wide(const CvArgs& a, int prec);
 int gemm_cv_tiles(long long M, long long N, int tri, int cfg);
 hipError_t gemm_cv_launch(CvArgs& a, int prec, int cfg, hipStream_t st);
 

@@ -100,11 +100,11 @@ __device__ __forceinline__ float ld_elem(const void* __restrict__ p, const CvOpe
 // One operand's tile of ROWS x (32 KS) in registers, as fp32, staged by 256 threads. H_KC / H_ELEM: thread t holds the
 // 4-k chunks of k 4 (t % KV) of rows t / KV + i (256 / KV). H_MC: the 4 x 4 block of rows 4 (t % RB) .. and k
 // 4 (t / RB) .., one register quad per k, transposed on the way to LDS (a wave reads whole 4 ROWS-byte runs).
-// MODE KC or MC: fp32 rows in that layout, whose loads no branch surrounds (registers that meet at the end of a branch
+// MODE KC or MC: rows in that layout, fp32 or (BF) bf16, whose loads no branch surrounds (registers that meet at the end of a branch
 // are copied there, and the copy waits for the load) and whose addresses are one register plus constants: with every
 // chunk's offsets and bounds checks computed apart, a tile's staging took 430 VALU instructions, 180 of them the
 // conversion. MODE SYM: any operand, its layout and storage known at run time.
-template <int ROWS, int KS, int MODE>
+template <int ROWS, int KS, int MODE, bool BF>
 struct CvTile {
   static constexpr bool ANY = MODE == SYM;
   static constexpr int KV = 8 * KS;        // chunks per row
@@ -175,7 +175,7 @@ struct CvTile {
     }
     // the stored rows and columns this tile reads start at (r0, c0); the buffer ends with the operand's last element
     // (whole dwords: each is checked by itself)
-    const int sh = ANY && o.bf16 ? 1 : 2, stride = (int)o.ld;
+    const int sh = BF || (ANY && o.bf16) ? 1 : 2, stride = (int)o.ld;
     const bool kc = h == H_KC;
     const int r0 = kc ? mn0 : k0, c0 = kc ? k0 : mn0, nrow = kc ? rows : kend, ncol = kc ? kend : rows;
     const __amdgpu_buffer_rsrc_t rs =
@@ -192,9 +192,11 @@ struct CvTile {
         else load_mc(f4, 2, stride);
       }
     } else if constexpr (MODE == KC) {
-      load_kc(f4, 2, stride);
+      if constexpr (BF) load_kc(b4, 1, stride);
+      else load_kc(f4, 2, stride);
     } else {
-      load_mc(f4, 2, stride);
+      if constexpr (BF) load_mc(b4, 1, stride);
+      else load_mc(f4, 2, stride);
     }
   }
 
@@ -268,7 +270,8 @@ constexpr int cv_smem(int NP, int BM, int BN, int WN, int KG) {
 
 }  // namespace
 
-// LAY: bit 0 = A stored m-contiguous, bit 1 = B stored n-contiguous; 4: any operands
+// LAY: bit 0 = A stored m-contiguous, bit 1 = B stored n-contiguous, bits 3 and 4 = A and B in bf16 (else fp32); 4: any
+// operands
 template <int NP, int BM, int BN, int WN, int KG, int EPI, int LAY>
 __global__ void __launch_bounds__(WN == 4 || KG == 2 ? 512 : 256, 2) gemm_cv_kernel(const CvArgs p) {
   // Two groups of four waves, half a step apart, or (KG = 1) one. WN = 4: the groups own the upper and lower half of the
@@ -349,8 +352,8 @@ __global__ void __launch_bounds__(WN == 4 || KG == 2 ? 512 : 256, 2) gemm_cv_ker
   };
   constexpr int RA = SHARE ? BM / 2 : BM, RB = SHARE ? BN / 2 : BN;  // rows a group stages
   const int ha = SHARE ? h * RA : 0, hb = SHARE ? h * RB : 0;
-  CvTile<RA, KS, LAY == 4 ? SYM : LAY & 1 ? MC : KC> la;
-  CvTile<RB, KS, LAY == 4 ? SYM : LAY & 2 ? MC : KC> lb;
+  CvTile<RA, KS, LAY == 4 ? SYM : LAY & 1 ? MC : KC, (LAY & 8) != 0> la;
+  CvTile<RB, KS, LAY == 4 ? SYM : LAY & 2 ? MC : KC, (LAY & 16) != 0> lb;
   auto load_a = [&](int kt) INL { la.load(Ap, oa, m0 + ha, kbeg + kt * BK, p.M, kend); };
   auto load_b = [&](int kt) INL { lb.load(Bp, ob, n0 + hb, kbeg + kt * BK, p.N, kend); };
   // One stage's MFMAs, the products that need only B's first plane first. On the large tile, whose waves multiply alone
@@ -711,12 +714,14 @@ __global__ void __launch_bounds__(WN == 4 || KG == 2 ? 512 : 256, 2) gemm_cv_ker
   }
 }
 
-// operands beyond fp32 rows
-static bool gemm_cv_any(const CvArgs& a) {
-  auto any = [](const CvOperand& o) { return o.bf16 || o.mode == SYM || !o.vec; };
+// operands beyond plain rows (bf16 ones: plain stores of the bf16 precision)
+static bool gemm_cv_any(const CvArgs& a, int prec) {
+  auto any = [&](const CvOperand& o) { return (o.bf16 && !(prec == 1 && a.epi == EPI_STORE)) || o.mode == SYM || !o.vec; };
   return any(a.a) || any(a.b);
 }
-bool gemm_cv_wide(const CvArgs& a) { return !gemm_cv_any(a) && !(a.a.mode == MC && a.b.mode == KC); }
+bool gemm_cv_wide(const CvArgs& a, int prec) {
+  return !gemm_cv_any(a, prec) && !(a.a.mode == MC && a.b.mode == KC) && a.a.bf16 == a.b.bf16;
+}
 
 static void cv_tile(int cfg, int& bm, int& bn) {
   bm = cfg == 0 ? 128 : cfg == 2 ? 32 : 64;
@@ -748,11 +753,32 @@ static hipError_t launch_cv(const CvArgs& a, hipStream_t st) {
   return e;
 }
 
+// Plain stores of the bf16 precision with operands in bf16 (bits 8: A, 16: B). With the storage type known only at run
+// time a tile's loads had no step to arrive in: 2048^3 130 us, now 50, 16 x 4096 x 4096 172-192, now 45-52.
+template <int BM, int BN, int WN, int KG, int ST>
+static hipError_t launch_cv_b16(const CvArgs& a, int lay, hipStream_t st) {
+  switch (lay) {
+    case 0: return launch_cv<1, BM, BN, WN, KG, EPI_STORE, ST>(a, st);
+    case 1:
+      if constexpr (BM < 128) return launch_cv<1, BM, BN, WN, KG, EPI_STORE, ST + 1>(a, st);
+      return hipErrorInvalidValue;
+    case 2: return launch_cv<1, BM, BN, WN, KG, EPI_STORE, ST + 2>(a, st);
+    default: return launch_cv<1, BM, BN, WN, KG, EPI_STORE, ST + 3>(a, st);
+  }
+}
+
 // The layouts each epilogue's callers have: plain stores any, sums of squares (P1 X, X P2) A k-contiguous, the factor
 // and Procrustes products (term1 Q, R Q, R RQ, M Q) A k- and B n-contiguous, the trace SYRK k-contiguous.
 template <int NP, int BM, int BN, int WN, int KG>
 static hipError_t launch_cv_epi(const CvArgs& a, hipStream_t st) {
   const int lay = (a.a.mode == MC ? 1 : 0) | (a.b.mode == MC ? 2 : 0);
+  if constexpr (NP == 1) {
+    if (a.a.bf16 && a.b.bf16) return launch_cv_b16<BM, BN, WN, KG, 24>(a, lay, st);
+    if constexpr (BM < 128) {
+      if (a.a.bf16) return launch_cv_b16<BM, BN, WN, KG, 8>(a, lay, st);
+      if (a.b.bf16) return launch_cv_b16<BM, BN, WN, KG, 16>(a, lay, st);
+    }
+  }
   if (a.epi == EPI_STORE) {
     switch (lay) {
       case 0: return launch_cv<NP, BM, BN, WN, KG, EPI_STORE, 0>(a, st);
@@ -774,7 +800,7 @@ static hipError_t launch_cv_epi(const CvArgs& a, hipStream_t st) {
   return hipErrorInvalidValue;
 }
 
-// Operands beyond fp32 rows (gemm_cv_any): 64- and 32-row tiles. Beside the plain products only the factor update's A
+// Operands beyond plain rows (gemm_cv_any): 64- and 32-row tiles. Beside the plain products only the factor update's A
 // may be a triangle; the other epilogues' operands are fp32 rows short of 2^21 (their sides).
 template <int NP, int BM, int KG>
 static hipError_t launch_cv_any(const CvArgs& a, hipStream_t st) {
@@ -791,7 +817,7 @@ static hipError_t launch_cv_any(const CvArgs& a, hipStream_t st) {
 
 template <int NP>
 static hipError_t launch_cv_cfg(const CvArgs& a, int cfg, hipStream_t st) {
-  if (gemm_cv_any(a)) {
+  if (gemm_cv_any(a, NP == 1)) {
     if (cfg == 2) return launch_cv_any<NP, 32, 2>(a, st);
     return cfg == 3 ? launch_cv_any<NP, 64, 2>(a, st) : launch_cv_any<NP, 64, 1>(a, st);
   }

@@ -82,6 +82,23 @@ def test_converting_engine(engine, m, n, k, bf16):
     _check(C[ok], A[ok], B, False, "finite rows")
 
 
+@pytest.mark.parametrize("m,n,k", [(2, 2, 2), (31, 63, 33), (65, 129, 127), (129, 257, 130), (200, 500, 321)])
+def test_operands_stored_in_bf16(engine, m, n, k):
+    """Products of the bf16 precision with one or both operands in bf16, at rows of even stride (read four elements at a
+    time, whatever the rows' length) and of odd stride."""
+    for dA, dB in ((torch.bfloat16, torch.bfloat16), (torch.bfloat16, torch.float32), (torch.float32, torch.bfloat16)):
+        for pad in (3, 4):
+            def put(x, dt):
+                y = torch.full((x.shape[0], x.shape[1] // 2 * 2 + pad), float("nan"), dtype=dt, device=DEV)
+                y[:, 2:2 + x.shape[1]] = x
+                return y[:, 2:2 + x.shape[1]]
+            for ta in (False, True):
+                for tb in (False, True):
+                    a = put(_rnd(*((k, m) if ta else (m, k)), seed=m), dA)
+                    b = put(_rnd(*((n, k) if tb else (k, n)), seed=n), dB)
+                    _check(K.gemm(a, b, ta, tb, True), a.T if ta else a, b.T if tb else b, True, (ta, tb, dA, dB, pad))
+
+
 @pytest.mark.parametrize("k", [512, 1280, 1288, 3072])
 @pytest.mark.parametrize("sign", [False, True])
 def test_split_products_are_no_further_off_than_fp32_mfmas(engine, k, sign):
