@@ -348,9 +348,9 @@ int psgdk_profile_stop(psgdk_prof_record_t* out, int max_records, int* n_records
  * splits (1, default) or on fp32 MFMAs (0, three to four times slower); option 9 = the most
  * factors of one side >= 2048 that psgdk_kron2d_update_groups batches into one launch (1 .. 64, default 64; smaller
  * batches of one side run on different side streams); option 10 = plain-store bf16 GEMMs on k-contiguous operands
- * whose launch has fewer 128 x 128 tiles than this take the small-problem kernel (64 x 64 tiles, k in chunks of 512
- * bytes per row with two in flight); and fp32 products of fewer than 64 64 x 64 tiles (default 128,
- * 0: never; not with a forced tile configuration, option 1); option 11 = of those, a launch with fewer 64 x 64 tiles
+ * whose launch has fewer 128 x 128 tiles than this (SYRKs up to k 1024: than 1.5 times this) take the small-problem
+ * kernel (64 x 64 tiles, k in chunks of 512 bytes per row with two in flight); and fp32 products of fewer than 64
+ * 64 x 64 tiles (default 128, 0: never; not with a forced tile configuration, option 1); option 11 = of those, a launch with fewer 64 x 64 tiles
  * than this takes the tiny-product kernel (32 x 32 tiles whose four waves split k; results rounded in another
  * order than the other kernels' k-order sums; default 64, 0: never); option 12 = whether launches given 256 x 256
  * or 128 x 128 tiles by size take the configurations with load-only waves (option 1 values 3 and 4) rather than 0

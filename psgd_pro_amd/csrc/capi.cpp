@@ -177,8 +177,8 @@ thread_local int g_split = 1;  // option 8: fp32 products as six bf16 products o
 thread_local int g_cv_cfg = -1;  // option 13: tile configuration of the converting engine (-1 chosen by size)
 thread_local int g_big_batch = MAXB;  // option 9: items per batch of the grouped update for factor sides >= 2048
 thread_local int g_small = 128;       // option 10: bf16 plain-store GEMMs with fewer 128 x 128 tiles than this (over
-                                      // the launch) take the small-problem kernel; bf16 SYRKs below 1.5 times it, fp32
-                                      // products below 3 times it (0: never)
+                                      // the launch) take the small-problem kernel, SYRKs up to k 1024 below 1.5 times
+                                      // it (0: never, nor fp32 ones)
 thread_local int g_tiny = 64;         // option 11: of those, launches with fewer 64 x 64 tiles than this take the
                                       // tiny-product kernel (32-tiles, k split over the four waves; 0: never)
 
@@ -304,10 +304,13 @@ int run_b16(int nb, int64_t M, int64_t N, int64_t K, const void* const* A, int64
   const int cfg = b16_cfg(M, N, K, tri, nb, e.epi);
   // a plain store whose 128-tiles would leave most of the chip idle: the small-problem kernel (64-tiles, k in
   // 512-byte chunks, two in flight). Measured crossovers against the pipelined kernels (launch of nb problems, in
-  // 128-tiles): about 130 for products and for SYRKs (one SYRK, k = n, small against pipelined: n 1792, 105 tiles, 19.4
-  // us against 22.0; n 2048, 136 tiles, 32.0 against 24.2; n 2304, k 768, 171 tiles, 16.5 against 15.1).
+  // 128-tiles): about 130 for products and long SYRKs, about 190 for SYRKs up to k 1024, whose pipeline hardly fills (one
+  // SYRK, a call, small against pipelined, us: 105 tiles, k 1024 15.5, 22.6, k 4096 35.8, 44.6; 136 tiles, k 1024 22.2,
+  // 23.0, k 1536 28.3, 26.8; 171 tiles, k 768 18.9, 21.3, k 1536 28.1, 26.9; 190 tiles, k 1024 22.8, 23.4; 210 tiles, k 768
+  // 22.2, 21.6).
   const int64_t t128 = (int64_t)gemm_bf16_tiles(M, N, tri, 1) * nb;
-  const bool small = esz == 4 || (e.epi == EPI_STORE && !kbeg && !kper && g_force_cfg < 0 && t128 < g_small);
+  const int64_t small_max = tri && K <= 1024 ? 3 * (int64_t)g_small / 2 : g_small;
+  const bool small = esz == 4 || (e.epi == EPI_STORE && !kbeg && !kper && g_force_cfg < 0 && t128 < small_max);
   // ... and one whose 64-tiles would still fill only a fraction of the CUs: the tiny-product kernel
   const bool tiny = small && (int64_t)gemm_small_tiles(M, N, tri) * nb < g_tiny;
   if (ntiles)
