@@ -363,16 +363,17 @@ int run_b16(int nb, int64_t M, int64_t N, int64_t K, const void* const* A, int64
 
 // The converting engine's tiles: 32 x 64 for products of at most 32 rows; 64 x 64 on two wave groups that split k where
 // that is at most one workgroup per CU (1024^3 fp32: 25 us against 30 on one group); 128 x 256 where its tiles fill more
-// than half of the CUs (fp32: 6 products of 1536 x 512 x 512, 144 tiles, 46 us against 50; 1531^3, 72 tiles, 115 against
-// 78), in bf16, whose conversion is a larger part, more than one and a half rounds of them (3072^3, 288 tiles, 173 us
-// against 154; two of them 264 against 311); 64 x 64 otherwise, and for fp32 Gram
+// than half of the CUs (fp32, us, 128 x 256 against 64 x 64, k 512 and 3072: 100 tiles 42, 41 and 195, 208; 128 tiles 43, 41
+// and 197, 209; 144 tiles 42, 47 and 196, 244; 192 tiles 44, 56 and 208, 294; 288 tiles 87, 84 and 436, 454; 416 tiles 88,
+// 116 and 438, 625), in bf16, whose conversion is a larger part, more than one and a half rounds of them (3072^3, 288
+// tiles, 173 us against 154; two of them 264 against 311); 64 x 64 otherwise, and for fp32 Gram
 // products X^T X, whose diagonal only those tiles sum closely enough (gemm_cv.hip).
 int cv_cfg(int prec, int64_t M, int64_t N, int tri, int nb, int epi, bool narrow, bool gram) {
   const bool narrow_ok = !tri && (epi == EPI_STORE || epi == EPI_SUMSQ);
   if (g_cv_cfg == 2 ? narrow_ok : g_cv_cfg >= 0) return narrow && g_cv_cfg == 0 ? 1 : g_cv_cfg;
   if (M <= 32 && narrow_ok) return 2;
   if ((int64_t)gemm_cv_tiles(M, N, tri, 3) * nb <= 256) return 3;
-  return !narrow && !gram && (int64_t)gemm_cv_tiles(M, N, tri, 0) * nb >= (prec == PSGDK_PREC_F32 ? 144 : 400) ? 0 : 1;
+  return !narrow && !gram && (int64_t)gemm_cv_tiles(M, N, tri, 0) * nb > (prec == PSGDK_PREC_F32 ? 128 : 400) ? 0 : 1;
 }
 
 int run_gemm(int prec, int nb, int64_t M, int64_t N, int64_t K, const Opnd& A, const Opnd& B, float* const* C,

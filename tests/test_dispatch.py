@@ -25,3 +25,15 @@ def test_bf16_syrk(n, k, small):
     assert [i // 1000 for i in ids] == [7 if small else 5]
     x = X.double()
     assert ((C - x @ x.T).abs() <= k * 2.0 ** -24 * (x.abs() @ x.abs().T)).all()
+
+
+@pytest.mark.parametrize("m,n,k,wide", [(2048, 2048, 96, False), (2048, 2049, 96, True), (2944, 1500, 64, True)])
+def test_fp32_product(m, n, k, wide):
+    """128 x 256 tiles from 129 of them on (2048 x 2048: 128; 2048 x 2049: 144; 2944 x 1500: 138), else 64 x 64. k 2^-24 of
+    |A||B| bounds both."""
+    g = torch.Generator().manual_seed(m + n)
+    A, B = torch.randn(m, k, generator=g).to(DEV), torch.randn(k, n, generator=g).to(DEV)
+    C, ids = _launches(lambda: K.gemm(A, B, False, False, False))
+    assert ids == [6000 + (0 if wide else 10)]
+    a, b = A.double(), B.double()
+    assert ((C - a @ b).abs() <= k * 2.0 ** -24 * (a.abs() @ b.abs())).all()
