@@ -131,6 +131,7 @@ struct Opnd {
 struct EpiSpec {
   int epi = EPI_STORE;
   float alpha = 1.f, beta = 0.f;
+  bool gram = false;  // SYRK whose operand may be near a multiple of the identity, as a factor is
   int64_t ldx = 0;
   const float* X1[MAXB] = {};
   const float* X2[MAXB] = {};
@@ -367,7 +368,7 @@ int run_b16(int nb, int64_t M, int64_t N, int64_t K, const void* const* A, int64
 // and 197, 209; 144 tiles 42, 47 and 196, 244; 192 tiles 44, 56 and 208, 294; 288 tiles 87, 84 and 436, 454; 416 tiles 88,
 // 116 and 438, 625), in bf16, whose conversion is a larger part, more than one and a half rounds of them (3072^3, 288
 // tiles, 173 us against 154; two of them 264 against 311); 64 x 64 otherwise, and for fp32 Gram
-// products X^T X, whose diagonal only those tiles sum closely enough (gemm_cv.hip).
+// products X^T X, and X X^T of a factor, whose diagonal only those tiles sum closely enough (gemm_cv.hip).
 int cv_cfg(int prec, int64_t M, int64_t N, int tri, int nb, int epi, bool narrow, bool gram) {
   const bool narrow_ok = !tri && (epi == EPI_STORE || epi == EPI_SUMSQ);
   if (g_cv_cfg == 2 ? narrow_ok : g_cv_cfg >= 0) return narrow && g_cv_cfg == 0 ? 1 : g_cv_cfg;
@@ -417,8 +418,8 @@ int run_gemm(int prec, int nb, int64_t M, int64_t N, int64_t K, const Opnd& A, c
     a.A[b] = A.p[b]; a.B[b] = B.p[b]; a.C[b] = C[b];
     a.X1[b] = e.X1[b]; a.X2[b] = e.X2[b]; a.s[b] = e.s[b]; a.part[b] = e.part[b];
   }
-  const int cfg = cv_cfg(prec, M, N, tri, nb, e.epi, !gemm_cv_wide(a, prec),
-                         prec == PSGDK_PREC_F32 && tri && e.epi == EPI_STORE && A.mode == MC);
+  a.gram = prec == PSGDK_PREC_F32 && tri && e.epi == EPI_STORE && (e.gram || A.mode == MC);
+  const int cfg = cv_cfg(prec, M, N, tri, nb, e.epi, !gemm_cv_wide(a, prec), a.gram);
   if (ntiles) *ntiles = gemm_cv_tiles(M, N, tri, cfg);
   if (!g_prof.on) return hip_check(gemm_cv_launch(a, prec, cfg, st), "gemm launch");
   ProfRec r;
@@ -1668,6 +1669,7 @@ int psgdk_syrk(int prec, int trans, int out_mode, int64_t n, int64_t k, int a_dt
   a.mode = trans ? MC : KC; a.ld = lda; a.dt = a_dtype;
   for (int b = 0; b < nb; ++b) a.p[b] = A[b];
   EpiSpec e;
+  e.gram = true;
   return run_gemm(prec, nb, n, n, k, a, a, C, out_mode == PSGDK_OUT_PACKED ? n : ldc, e, 1, out_mode, 0, 1, 0,
                   (hipStream_t)stream);
 }

@@ -21,6 +21,7 @@ struct CvArgs {
   float alpha, beta;
   int epi;
   int tri;              // 1: upper-triangular tile grid (SYRK: M == N, B is A)
+  int gram;             // tri, EPI_STORE, fp32: A may be near a multiple of the identity (64 x 64 tiles keep the diagonal)
   int out_mode;         // tri: 0 upper triangle only, 1 mirrored full matrix, 2 packed upper triangle
   int kbeg;             // 1: A is upper-triangular (A[i][k] = 0 for k < i): a tile's k loop starts at its first row
   int splitk, kchunk;   // split-K (EPI_STORE only): split s covers k in [s kchunk, (s+1) kchunk) and writes its

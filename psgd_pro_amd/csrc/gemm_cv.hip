@@ -21,10 +21,11 @@
 //   64- and 32-row tiles: h h' enters an MFMA with C = 0 and is added to the block by a VALU add, and the five small
 //     products have accumulators of their own, so nothing small is aligned to a large sum. Relative error (Frobenius, k
 //     1024 normals) 7.4e-8; one fp32 MFMA chain folded every 128 k: 2.1e-7.
-//   The diagonal tile of a Gram product X^T X, at the k of its own rows: for X near a multiple of the identity (a
+//   The diagonal tile of a Gram product X^T X or X X^T, at the k of its own rows: for X near a multiple of the identity (a
 //     preconditioner factor) one square outweighs the other 7 of its lane, whose truncation then always lowers the
-//     diagonal (by 7e-8 of it, which the norm bound of the next product sees doubled): there a row's
-//     own k has an h h' MFMA to itself. Gram products keep to these tiles.
+//     diagonal (by up to 2e-7 of it, which the norm bound of the next product sees doubled): there a row's
+//     own k is left out of A's planes and added to the sum by one fp32 multiply-add (mean below 1e-8). Gram products of
+//     factors keep to these tiles.
 //   128 x 256 tiles: registers for one accumulator set per block only, with all six products on top of it. Bits of a
 //     small product below the last of a large C are dropped downward (mean error of 3072^3 -5e-8 of the results' rms), so
 //     every other block is computed negated and subtracted (mean below 1e-10). Longer blocks cost roundings inside them,
@@ -226,6 +227,20 @@ struct CvTile {
     }
   }
 
+  // zeroes the elements whose row is their k (a tile that starts at equal rows and k)
+  __device__ __forceinline__ void clear_own() {
+    const unsigned t = thread();
+    if (ANY ? how == H_MC : MODE == MC) {
+#pragma unroll
+      for (int j = 0; j < 4; ++j) r[j][j] = t % RB == t / RB ? 0.f : r[j][j];
+    } else {
+#pragma unroll
+      for (int i = 0; i < NC; ++i)
+#pragma unroll
+        for (int e = 0; e < 4; ++e) r[i][e] = t / KV + i * RS == t % KV * 4 + e ? 0.f : r[i][e];
+    }
+  }
+
   // into NP bf16 planes of KS slices of TROWS rows x 32 k, from row `row0` on (a multiple of 16)
   // (three planes: of the values times `scale`, +- kSplitScale)
   template <int NP, int TROWS>
@@ -270,8 +285,8 @@ constexpr int cv_smem(int NP, int BM, int BN, int WN, int KG) {
 
 }  // namespace
 
-// LAY: bit 0 = A stored m-contiguous, bit 1 = B stored n-contiguous, bits 3 and 4 = A and B in bf16 (else fp32); 4: any
-// operands
+// LAY: bit 0 = A stored m-contiguous, bit 1 = B stored n-contiguous, bits 3 and 4 = A and B in bf16 (else fp32),
+// bit 5 = Gram product with its rows' own k apart; 4: any operands
 template <int NP, int BM, int BN, int WN, int KG, int EPI, int LAY>
 __global__ void __launch_bounds__(WN == 4 || KG == 2 ? 512 : 256, 2) gemm_cv_kernel(const CvArgs p) {
   // Two groups of four waves, half a step apart, or (KG = 1) one. WN = 4: the groups own the upper and lower half of the
@@ -327,7 +342,7 @@ __global__ void __launch_bounds__(WN == 4 || KG == 2 ? 512 : 256, 2) gemm_cv_ker
 
   // sums folded so far, the current block's, and (three planes, small tiles) all five small products' of the whole k range
   constexpr bool SM = NP == 3 && !SHARE;
-  constexpr bool GRAM = SM && EPI == EPI_STORE && BM == BN && LAY == 3;  // X^T X among them
+  constexpr bool GRAM = (LAY & 32) != 0;
   // an accumulation block has 2^bs k tiles: 128 k, or the large tile's 64 (see the file's comment)
   constexpr int BT = 128 / BK, BS = BT == 4 ? 2 : 1;
   static_assert(BT == 1 << BS, "a power of two");
@@ -352,14 +367,14 @@ __global__ void __launch_bounds__(WN == 4 || KG == 2 ? 512 : 256, 2) gemm_cv_ker
   };
   constexpr int RA = SHARE ? BM / 2 : BM, RB = SHARE ? BN / 2 : BN;  // rows a group stages
   const int ha = SHARE ? h * RA : 0, hb = SHARE ? h * RB : 0;
-  CvTile<RA, KS, LAY == 4 ? SYM : LAY & 1 ? MC : KC, (LAY & 8) != 0> la;
-  CvTile<RB, KS, LAY == 4 ? SYM : LAY & 2 ? MC : KC, (LAY & 16) != 0> lb;
+  CvTile<RA, KS, LAY & 4 ? SYM : LAY & 1 ? MC : KC, (LAY & 8) != 0> la;
+  CvTile<RB, KS, LAY & 4 ? SYM : LAY & 2 ? MC : KC, (LAY & 16) != 0> lb;
   auto load_a = [&](int kt) INL { la.load(Ap, oa, m0 + ha, kbeg + kt * BK, p.M, kend); };
   auto load_b = [&](int kt) INL { lb.load(Bp, ob, n0 + hb, kbeg + kt * BK, p.N, kend); };
   // One stage's MFMAs, the products that need only B's first plane first. On the large tile, whose waves multiply alone
   // on their SIMD, A fragments are read one row of tiles ahead (and B's next k step with them) and the MFMAs start before
   // all of a step's fragments have arrived; the small tiles' waves overlap each other, and fewer registers are better.
-  auto mma_planes = [&](const unsigned char* As, bool own_k) INL {
+  auto mma_planes = [&](const unsigned char* As) INL {
     const unsigned char* Bs = As + NP * AB;
     constexpr int NK = BK / KM, NQ = NK * FM;  // k steps, rows of tiles
     bf16x8_t aq[2][NP], bq[2][NP][FN];
@@ -406,21 +421,6 @@ __global__ void __launch_bounds__(WN == 4 || KG == 2 ? 512 : 256, 2) gemm_cv_ker
         Acc top[FN];
 #pragma unroll
         for (int j = 0; j < FN; ++j) top[j] = mfma(0, 0, j, nil);
-        if constexpr (GRAM) {
-          if (own_k) {  // the row's own k apart from the others (see the file's comment)
-            const int e = wm * TM + i * MT + r - t * KM - 8 * g;
-            union { bf16x8_t v; unsigned u[4]; } own, rest = {aq[q & 1][0]};
-#pragma unroll
-            for (int d = 0; d < 4; ++d) {
-              own.u[d] = rest.u[d] & (d == e >> 1 ? 0xffffu << 16 * (e & 1) : 0u);
-              rest.u[d] ^= own.u[d];
-            }
-#pragma unroll
-            for (int j = 0; j < FN; ++j)
-              top[j] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(rest.v, bq[t & 1][0][j], nil, 0, 0, 0) +
-                       __builtin_amdgcn_mfma_f32_16x16x32_bf16(own.v, bq[t & 1][0][j], nil, 0, 0, 0);
-          }
-        }
         term(sm[i], 2, 0);
         term(sm[i], 1, 0);
         term(sm[i], 1, 1);
@@ -475,9 +475,9 @@ __global__ void __launch_bounds__(WN == 4 || KG == 2 ? 512 : 256, 2) gemm_cv_ker
     lb.template store<NP, BN>(st + NP * AB, hb, ob, kSplitScale);
     load_b(kt);
   };
-  // tile i holds the own k of its rows, in a Gram product's diagonal tile
-  static_assert(!GRAM || BK == BM, "the k of a diagonal tile's rows are one tile");
-  auto gram = [&](int i) INL { return GRAM && p.tri && m0 == n0 && kbeg + (KG * i + h) * BK == m0; };
+  // k tile kt holds the own k of its rows, in a Gram product's diagonal tile
+  static_assert(!GRAM || (SM && BK == BM && BM == BN), "the k of a diagonal tile's rows are one tile");
+  auto own_k = [&](int kt) INL { return m0 == n0 && kbeg + kt * BK == m0; };
   // tile i belongs to a negated block
   auto odd = [&](int i) INL { return NP == 3 && SHARE && (i >> bs & 1) != 0; };
   zero();
@@ -494,7 +494,7 @@ __global__ void __launch_bounds__(WN == 4 || KG == 2 ? 512 : 256, 2) gemm_cv_ker
         stage(at(kt + h), odd(kt + h), kt + h + 1);
         __syncthreads();
         if (kt >= 0) {
-          mma_planes(at(kt), false);
+          mma_planes(at(kt));
           if (block_end(kt, nk)) fold(odd(kt));
           __syncthreads();
         }
@@ -509,9 +509,10 @@ __global__ void __launch_bounds__(WN == 4 || KG == 2 ? 512 : 256, 2) gemm_cv_ker
       unsigned char* const st = smem + h * STAGE;
       if (h == 1) __syncthreads();
       for (int i = 0; i < n; ++i) {
+        if (GRAM && own_k(KG * i + h)) la.clear_own();
         stage(st, odd(i), (i + 1) * KG + h);
         __syncthreads();
-        mma_planes(st, gram(i));
+        mma_planes(st);
         if (block_end(i, n)) fold(odd(i));
         __syncthreads();
       }
@@ -546,7 +547,18 @@ __global__ void __launch_bounds__(WN == 4 || KG == 2 ? 512 : 256, 2) gemm_cv_ker
   if constexpr (NP == 3) {  // the same tile by fp32 MFMAs: on request, or where a sum is not finite
     bool fin = !p.f32;
     if (out) each_acc([&](int i, int j, int e) INL { fin = fin && fabsf(acc[i][j][e]) < INFINITY; });
-    if (__syncthreads_or(!fin)) {
+    const bool again = __syncthreads_or(!fin);
+    if constexpr (GRAM) {  // the rows' own k: one exact product, one rounding
+      if (!again && out && m0 == n0)
+        each_acc([&](int i, int j, int e) INL {
+          const int row = m0 + wm * TM + i * MT + acc_row(g, e), col = n0 + wn * TN + j * MT + r;
+          auto at = [&](int mn) INL {
+            return oa.bf16 ? ld_elem<bf16_t>(Ap, oa, mn, row, p.M, p.K) : ld_elem<float>(Ap, oa, mn, row, p.M, p.K);
+          };
+          acc[i][j][e] = fmaf(at(row), at(col), acc[i][j][e]);
+        });
+    }
+    if (again) {
       zero();
       for (int kt = 0; kt < nk; ++kt) {
         if (out) {
@@ -779,6 +791,10 @@ static hipError_t launch_cv_epi(const CvArgs& a, hipStream_t st) {
       if (a.b.bf16) return launch_cv_b16<BM, BN, WN, KG, 16>(a, lay, st);
     }
   }
+  if constexpr (NP == 3 && BM == 64) {
+    if (a.gram && lay == 0) return launch_cv<NP, BM, BN, WN, KG, EPI_STORE, 32>(a, st);
+    if (a.gram && lay == 3) return launch_cv<NP, BM, BN, WN, KG, EPI_STORE, 35>(a, st);
+  }
   if (a.epi == EPI_STORE) {
     switch (lay) {
       case 0: return launch_cv<NP, BM, BN, WN, KG, EPI_STORE, 0>(a, st);
@@ -804,6 +820,9 @@ static hipError_t launch_cv_epi(const CvArgs& a, hipStream_t st) {
 // may be a triangle; the other epilogues' operands are fp32 rows short of 2^21 (their sides).
 template <int NP, int BM, int KG>
 static hipError_t launch_cv_any(const CvArgs& a, hipStream_t st) {
+  if constexpr (NP == 3 && BM == 64) {
+    if (a.gram) return launch_cv<NP, BM, 64, 2, KG, EPI_STORE, 36>(a, st);
+  }
   switch (a.epi) {
     case EPI_STORE: return launch_cv<NP, BM, 64, 2, KG, EPI_STORE, 4>(a, st);
     case EPI_SUMSQ: return launch_cv<NP, BM, 64, 2, KG, EPI_SUMSQ, 4>(a, st);

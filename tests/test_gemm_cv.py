@@ -187,3 +187,23 @@ def test_application_in_every_configuration(engine, m, n):
         rms = x.square().mean().sqrt()
         step = (x * (0.5 / rms) if rms > 0.5 else x).clamp(-1.0, 1.0)
         assert rel_err_norm(W[b].double() - dW[b].double().cpu(), 1e-3 * step) < 1e-4  # W - step rounds at 2^-24 of W
+
+
+@pytest.mark.parametrize("cfg", [-1, 1, 3])
+@pytest.mark.parametrize("n", [192, 1601, 3072])
+@pytest.mark.parametrize("trans,dt", [(False, torch.float32), (True, torch.float32), (False, torch.bfloat16)])
+def test_gram_diagonal_is_unbiased(n, trans, dt, cfg):
+    """X X^T and X^T X for X near the identity, at sizes that take the 128 x 256 tiles otherwise: no entry of the diagonal
+    loses the seven squares beside its large one. Without their own MFMA the mean is -2e-7 here; the roundings of n entries
+    of either sign leave less than 2^-24 / 8."""
+    X = (torch.eye(n) + 2.0 ** -10 * torch.randn(n, n, generator=torch.Generator().manual_seed(5))).to(DEV).to(dt)
+    L.check(L.lib().psgdk_set_option(13, cfg))
+    L.check(L.lib().psgdk_set_option(10, 0))
+    try:
+        C = K.syrk(X, trans, L.OUT_MIRROR, False)
+    finally:
+        L.check(L.lib().psgdk_set_option(13, -1))
+        L.check(L.lib().psgdk_set_option(10, 128))
+    x = X.double()
+    d = C.diagonal().double() - x.square().sum(0 if trans else 1)
+    assert d.mean().abs().item() < 2.0 ** -27, d.mean()
