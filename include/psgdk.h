@@ -305,7 +305,7 @@ int psgdk_fill_normal(void* out, int64_t n, int dtype, uint64_t seed, uint64_t s
  * bracketed by a pair of HIP events on its stream. psgdk_profile_stop ends the recording and, with out non-NULL,
  * waits for the recorded events and fills one record per launch: the kernel instantiation id
  * (bf16 engine: 5000 + cfg * 10 + epilogue, cfg as option 1 below, epilogue 0 = store, 1 = factor update, 2 = Procrustes
- * step, 4 = R Q with its trace partials, 5 = store with sums of squares, 6 = the r2 trace SYRK's scale
+ * step, 3 = scale, 4 = R Q with its trace partials, 5 = store with sums of squares, 6 = the r2 trace SYRK's scale
  * applied twice, 7 = Procrustes step reading (R Q)^T in bf16;
  * converting engine: 6000 (fp32) or 8000 (bf16 precision) + cfg * 10 + epilogue, cfg as option 13; the small-problem kernels: 7000 / 7001 on 64 x 64 tiles, 7002 / 7003
  * the tiny-product kernel, bf16 / fp32 operands), whether it was a

@@ -12,6 +12,7 @@ enum Epi : int {
   EPI_STORE = 0,   // C = alpha * acc + beta * C
   EPI_FACTOR = 1,  // C = X1 - s[0] * (acc - s[1] * X1)              (Q - lr/L (term1 Q - term2 Q))
   EPI_PROC = 2,    // C = X1 + a X2 + a^2/2 * s[1] * acc, a = s[0]    (Procrustes: Q + a RQ + a^2/2 R RQ)
+  EPI_SCALE = 3,   // C = s[0] * acc
   EPI_RQ = 4,      // C = s[0] * acc and trace partials of tr(C), tr(s[0] X1 C) into part[]  (Procrustes RQ)
   EPI_SUMSQ = 5,   // C = alpha * acc and partial sums of C^2 into part[]                    (apply + clip stats)
   EPI_PROCB = 7,   // bf16 kernel only: EPI_PROC with X2 = (R Q)^T in bf16, row stride ldx (the transposed copy

@@ -30,6 +30,11 @@ using T = bf16_t;
 // in the kernel), padded by 4 otherwise.
 constexpr int epi_pitch(int hr, int wc) { return hr == 64 && wc == 64 ? wc : wc + 4; }
 
+__device__ __forceinline__ int remap_xcd(int w, int G) {
+  const int cnt = G / 8, rem = G % 8, xcd = w % 8, slot = w / 8;
+  return xcd < rem ? xcd * (cnt + 1) + slot : rem * (cnt + 1) + (xcd - rem) * cnt + slot;
+}
+
 
 // LDS slot of the 16-byte k chunk c (0..7) of tile row `row`. Rows are 128 bytes with no padding; the XOR spreads
 // the 16 rows of an MFMA fragment read (16 lanes, one chunk each) over 16 distinct 16-byte bank groups, which
@@ -104,7 +109,7 @@ __global__ void __launch_bounds__(64 * (WGM * WGN + PW)) gemm_bf16_kernel(const 
   T* const Bs0 = As0 + 2 * BM * KP;
 
   const int G = p.ntiles * p.nb;
-  const int logical = p.vec ? xcd_run(blockIdx.x, G) : (int)blockIdx.x;
+  const int logical = p.vec ? remap_xcd(blockIdx.x, G) : (int)blockIdx.x;
   const int b = logical / p.ntiles, tile = logical % p.ntiles;
   // this problem's k extent and leading dimensions (kper: its own K, rows of exactly K)
   const int K = p.kper ? p.kp[b] : p.K;
@@ -388,7 +393,8 @@ __global__ void __launch_bounds__(64 * (WGM * WGN + PW)) gemm_bf16_kernel(const 
   const float* __restrict__ X1 = p.X1[b];
   const float* __restrict__ X2 = p.X2[b];
   float s0 = 0.f, s1 = 0.f;
-  if constexpr (EPI == EPI_FACTOR || EPI == EPI_PROC || EPI == EPI_PROCB || EPI == EPI_RQ || EPI == EPI_STRACE)
+  if constexpr (EPI == EPI_FACTOR || EPI == EPI_PROC || EPI == EPI_PROCB || EPI == EPI_SCALE || EPI == EPI_RQ ||
+                EPI == EPI_STRACE)
     s0 = p.s[b][0];
   if constexpr (EPI == EPI_FACTOR || EPI == EPI_PROC || EPI == EPI_PROCB) s1 = p.s[b][1];
   const bool mirror = p.tri && p.out_mode == 1;
@@ -442,9 +448,9 @@ __global__ void __launch_bounds__(64 * (WGM * WGN + PW)) gemm_bf16_kernel(const 
           v[e] = ok[e] ? q1[e] + v[e] : 0.f;
         } else if constexpr (EPI == EPI_STRACE) {
           v[e] = (s0 * v[e]) * s0;
-        } else if constexpr (EPI == EPI_RQ) {
+        } else if constexpr (EPI == EPI_SCALE || EPI == EPI_RQ) {
           v[e] = s0 * v[e];
-          if (ok[e] && row == col + e) t1 += v[e];
+          if (EPI == EPI_RQ && ok[e] && row == col + e) t1 += v[e];
         } else {
           v[e] = p.alpha * v[e];
           if (EPI == EPI_SUMSQ && ok[e]) t1 += v[e] * v[e];
@@ -772,6 +778,7 @@ static hipError_t launch_epi(GB16Args& a, hipStream_t st) {
   switch (a.epi) {
     case EPI_FACTOR: return launch_b16<BM, BN, WGM, WGN, EPI_FACTOR, PW>(a, st);
     case EPI_PROC: return launch_b16<BM, BN, WGM, WGN, EPI_PROC, PW>(a, st);
+    case EPI_SCALE: return launch_b16<BM, BN, WGM, WGN, EPI_SCALE, PW>(a, st);
     case EPI_SUMSQ: return launch_b16<BM, BN, WGM, WGN, EPI_SUMSQ, PW>(a, st);
     case EPI_STRACE: return launch_b16<BM, BN, WGM, WGN, EPI_STRACE, PW>(a, st);
     case EPI_STORE: return launch_b16<BM, BN, WGM, WGN, EPI_STORE, PW>(a, st);
