@@ -61,6 +61,12 @@ __device__ __forceinline__ float wave_max(float v) {
   return v;
 }
 
+// Tile of workgroup w of G (workgroup w runs on XCD w % 8): each XCD gets one contiguous run of tiles.
+__device__ __forceinline__ int xcd_run(int w, int G) {
+  const int cnt = G / 8, rem = G % 8, xcd = w % 8, slot = w / 8;
+  return xcd < rem ? xcd * (cnt + 1) + slot : rem * (cnt + 1) + (xcd - rem) * cnt + slot;
+}
+
 // Raw buffer resource over [base, base + bytes): loads at offsets >= bytes (clamped to 0 .. 2^31 - 1; a tile wholly
 // past its operand has a negative extent, which as an unsigned record count would let every offset through) return
 // zero, so a lane with nothing to load passes offset 0x7fffffff instead of branching.

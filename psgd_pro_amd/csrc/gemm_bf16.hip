@@ -30,11 +30,6 @@ using T = bf16_t;
 // in the kernel), padded by 4 otherwise.
 constexpr int epi_pitch(int hr, int wc) { return hr == 64 && wc == 64 ? wc : wc + 4; }
 
-__device__ __forceinline__ int remap_xcd(int w, int G) {
-  const int cnt = G / 8, rem = G % 8, xcd = w % 8, slot = w / 8;
-  return xcd < rem ? xcd * (cnt + 1) + slot : rem * (cnt + 1) + (xcd - rem) * cnt + slot;
-}
-
 
 // LDS slot of the 16-byte k chunk c (0..7) of tile row `row`. Rows are 128 bytes with no padding; the XOR spreads
 // the 16 rows of an MFMA fragment read (16 lanes, one chunk each) over 16 distinct 16-byte bank groups, which
@@ -109,7 +104,7 @@ __global__ void __launch_bounds__(64 * (WGM * WGN + PW)) gemm_bf16_kernel(const 
   T* const Bs0 = As0 + 2 * BM * KP;
 
   const int G = p.ntiles * p.nb;
-  const int logical = p.vec ? remap_xcd(blockIdx.x, G) : (int)blockIdx.x;
+  const int logical = p.vec ? xcd_run(blockIdx.x, G) : (int)blockIdx.x;
   const int b = logical / p.ntiles, tile = logical % p.ntiles;
   // this problem's k extent and leading dimensions (kper: its own K, rows of exactly K)
   const int K = p.kper ? p.kp[b] : p.K;

@@ -269,11 +269,6 @@ struct CvTile {
   }
 };
 
-__device__ __forceinline__ int xcd_run(int w, int G) {
-  const int cnt = G / 8, rem = G % 8, xcd = w % 8, slot = w / 8;
-  return xcd < rem ? xcd * (cnt + 1) + slot : rem * (cnt + 1) + (xcd - rem) * cnt + slot;
-}
-
 constexpr int cv_ks(int BM) { return BM == 64 ? 2 : 1; }          // 32-k slices per LDS stage
 constexpr int cv_hr(int BM) { return BM == 128 ? 32 : BM / 2; }  // rows of a wave's block per epilogue pass
 constexpr int cv_smem(int NP, int BM, int BN, int WN, int KG) {
