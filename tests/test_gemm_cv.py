@@ -8,6 +8,7 @@ import torch
 from psgd_pro_amd import _lib as L
 from psgd_pro_amd import ops as K
 from tests.metrics import rel_err_norm
+from tests.test_gpu_parity import assert_fp32, run_pair
 
 pytestmark = pytest.mark.gpu
 DEV = "cuda"
@@ -34,12 +35,15 @@ def _check(C, A, B, bf16, what):
     """|C - A B| <= c |A| |B| elementwise. fp32: the split drops under 2^-23 of each product, and a product takes part in
     at most 6 roundings per 16 k of its 128-k block (a truncation counting two) and one per block, each 2^-24 of sums
     that |A| |B| bounds. bf16: two operand
-    roundings of 2^-8 besides. (The last term: results below the smallest normal.)"""
+    roundings of 2^-8 besides. (The last term: results below the smallest normal.) And fp32 normwise 1e-6, five times the
+    measured 2e-7: without a third plane, or without m m', random operands are 2e-6 to 6e-6 off."""
     A, B = A.double().cpu(), B.double().cpu()
     u = 2.0 ** -24
     c = u * (2 + 2 * 6 * 8 + A.shape[1] / 64 + 4) + (2.0 ** -7 + 2.0 ** -16 if bf16 else 0.0)
     bad = (C.double().cpu() - A @ B).abs() > c * (A.abs() @ B.abs()) + 2.0 ** -126
     assert not bad.any(), (what, int(bad.sum()))
+    if not bf16 and (A @ B).norm() > 2.0 ** -100:
+        assert rel_err_norm(C, A @ B) < 1e-6, (what, rel_err_norm(C, A @ B))
 
 
 @pytest.mark.parametrize("m,n,k", [(1, 1, 1), (31, 63, 33), (64, 64, 64), (65, 129, 127), (129, 257, 130),
@@ -207,3 +211,67 @@ def test_gram_diagonal_is_unbiased(n, trans, dt, cfg):
     x = X.double()
     d = C.diagonal().double() - x.square().sum(0 if trans else 1)
     assert d.mean().abs().item() < 2.0 ** -27, d.mean()
+
+
+@pytest.mark.parametrize("r2", [False, True])
+def test_steps_at_the_edges_of_tiles(engine, r2):
+    """Whole fp32 steps against the float64 oracle at the fp32 bar, in every tile configuration: the epilogues of the factor
+    update, of both Procrustes steps (their traces, their reads of Q and R Q, the triangular grid) and of the application,
+    at sides one past a tile, inside one, and past two tile rows of 128."""
+    worst, base = run_pair([(129, 257), (390, 64)], steps=2, skew=float("inf"), r2=r2,
+                           grad_eps=float(torch.finfo(torch.float32).eps))
+    assert_fp32(worst, base)
+
+
+def _epilogue_results(hip, d, value):
+    """The outputs of the factor update, both Procrustes steps and the application with `value` in single places."""
+    g = torch.Generator().manual_seed(d)
+    ws, st = L.Workspace(), L.stream_of(torch.empty(1, device=DEV))
+    dev = torch.device(DEV)
+    Q = torch.eye(d) + 0.05 * torch.randn(d, d, generator=g)
+    X = torch.randn(d, d, generator=g) / d ** 0.5
+    T = X @ X.T
+    T[d // 3, d // 2] = T[d // 2, d // 3] = value
+    V = torch.randn(32, d, generator=g).to(DEV)
+    out = []
+    q, t, Lv = Q.to(DEV), T.to(DEV), torch.full((1,), 1.0, device=DEV)
+    qo = torch.empty_like(q)
+    L.call_ws(hip.psgdk_factor_update, 0, d, 1, L.ptrs([t]), 0, L.ptrs([q]), L.ptrs([qo]), L.ptrs([Lv]), L.ptrs([V]), 0.1,
+              0.9, 3.0, ws=ws, device=dev, stream=st)
+    out += [qo, Lv]
+    Q[d // 4, d // 5] = value
+    q = Q.to(DEV)
+    for fn in (hip.psgdk_procrustes, hip.psgdk_procrustes_r2):
+        out.append(torch.empty_like(q))
+        L.call_ws(fn, 0, d, 1, L.ptrs([q]), L.ptrs([out[-1]]), L.ptrs([V]), ws=ws, device=dev, stream=st)
+    G = torch.randn(d, d, generator=g)
+    G[1, 2] = value
+    G, P = G.to(DEV), (T.clamp(max=1.0) + torch.eye(d)).to(DEV)
+    W, pre = torch.zeros(d, d, device=DEV), torch.empty(d, d, device=DEV)
+    k = L.Kron2d()
+    k.nb, k.prec, k.m, k.n, k.g_dtype, k.p_dtype = 1, L.PREC_F32, d, d, L.F32, L.F32
+    k.kind[0] = k.kind[1] = L.FACTOR_DENSE
+    k.G[0] = G.data_ptr()
+    for f in range(2):
+        k.P[f][0] = k.Q[f][0] = k.L[f][0] = P.data_ptr()
+    L.call_ws(hip.psgdk_kron2d_apply, k, L.ApplyOpts(1e-3, 0.5, 1.0, 0), L.ptrs([W]), L.ptrs([pre]), None, ws=ws,
+              device=dev, stream=st)
+    return [o.cpu() for o in out + [pre, W]]
+
+
+@pytest.mark.parametrize("value", [float("inf"), float("nan"), 3.4e38, 2.0 ** 113, 2.0 ** 60])
+@pytest.mark.parametrize("d", [130, 300])
+def test_epilogues_of_sums_that_are_not_finite(engine, d, value):
+    """Values that the split cannot hold, in front of every epilogue: infinities and NaNs fall where fp32 MFMAs (option 8 = 0)
+    put them, and what is finite agrees row by row to 1e-5 of the row's largest value (both are fp32 sums, 3e-7, of
+    products that reach the outputs through up to three more)."""
+    got = _epilogue_results(engine, d, value)
+    L.check(engine.psgdk_set_option(8, 0))
+    ref = _epilogue_results(engine, d, value)
+    L.check(engine.psgdk_set_option(8, 1))
+    for i, (x, y) in enumerate(zip(got, ref)):
+        assert torch.equal(torch.isnan(x), torch.isnan(y)) and torch.equal(torch.isinf(x), torch.isinf(y)), i
+        fin = torch.isfinite(y)
+        assert torch.equal(x[~fin & ~torch.isnan(y)], y[~fin & ~torch.isnan(y)]), i
+        x, y = (torch.where(fin, v, 0.0).double().reshape(-1, v.shape[-1]) for v in (x, y))
+        assert ((x - y).abs() <= 1e-5 * y.abs().amax(1, keepdim=True)).all(), i
