@@ -8,7 +8,8 @@
  * *ws_bytes and return PSGDK_OK; otherwise *ws_bytes must be at least that size.
  * Return value: PSGDK_OK or an error code; psgdk_last_error() describes the last error of the calling thread.
  *
- * Precision: prec = PSGDK_PREC_F32 multiplies fp32 inputs on the fp32 MFMA path; PSGDK_PREC_BF16 rounds the inputs
+ * Precision: prec = PSGDK_PREC_F32 multiplies fp32 inputs to fp32 accuracy, over fp32's whole range (as exact three-way
+ * bfloat16 splits, or on fp32 MFMAs: option 8 of psgdk_set_option); PSGDK_PREC_BF16 rounds the inputs
  * of every contraction to bfloat16 (round to nearest even) and multiplies on the bf16 MFMA path. Accumulation and
  * all outputs are fp32 in both cases. Operand storage dtypes (PSGDK_F32 / PSGDK_BF16) are independent of prec.
  *
@@ -27,7 +28,9 @@ extern "C" {
 typedef struct ihipStream_t* psgdk_stream_t; /* hipStream_t */
 typedef struct ihipEvent_t* psgdk_event_t;   /* hipEvent_t */
 
-#define PSGDK_VERSION 4
+/* 5: option 8 chooses how fp32 products are summed (in 4: whether a k-contiguous fp32 kernel is taken), option 13, kernel
+ * ids 6000 and 8000 (in 4: other engines' ids below 5000 and at 6000), smaller workspaces of psgdk_trmm_ws. */
+#define PSGDK_VERSION 5
 #define PSGDK_MAXB 16 /* problems per grouped call */
 #define PSGDK_MAX_GROUPS 64 /* groups per psgdk_kron2d_update_groups call */
 #define PSGDK_NLB_K 32 /* rows of the random start of the norm lower bounds */
@@ -307,8 +310,8 @@ int psgdk_fill_normal(void* out, int64_t n, int dtype, uint64_t seed, uint64_t s
  * (bf16 engine: 5000 + cfg * 10 + epilogue, cfg as option 1 below, epilogue 0 = store, 1 = factor update, 2 = Procrustes
  * step, 3 = scale, 4 = R Q with its trace partials, 5 = store with sums of squares, 6 = the r2 trace SYRK's scale
  * applied twice, 7 = Procrustes step reading (R Q)^T in bf16;
- * converting engine: 6000 (fp32) or 8000 (bf16 precision) + cfg * 10 + epilogue, cfg as option 13; the small-problem kernels: 7000 / 7001 on 64 x 64 tiles, 7002 / 7003
- * the tiny-product kernel, bf16 / fp32 operands), whether it was a
+ * converting engine: 6000 (fp32) or 8000 (bf16 precision) + cfg * 10 + epilogue, cfg as option 13; the small-problem
+ * kernels: 7000 / 7001 on 64 x 64 tiles, 7002 / 7003 the tiny-product kernel, bf16 / fp32 operands), whether it was a
  * SYRK (triangular grid), the problems in the launch, its device time, its algorithmic flop count (SYRK n(n+1)k,
  * TRMM n(n+1)p, GEMM 2mnk, per problem) and its algorithmic bytes (operands read once, outputs written once). With out NULL only *n_records is set (records kept). */
 typedef struct psgdk_prof_record {
@@ -327,15 +330,15 @@ int psgdk_profile_stop(psgdk_prof_record_t* out, int max_records, int* n_records
 
 /* Tuning switches, one set per host thread (a thread's settings apply to the calls it makes and never change
  * another thread's results; a new thread starts from the defaults, so a switch set on one thread does not reach
- * calls that other threads make, such as a framework's worker threads): option 0 = tile order of the bf16 kernel (0 problem-major, 1 contiguous runs per
- * XCD, 2 = 1 with tile rows grouped by 4 so that the tiles an XCD runs at once share operand panels; default 2);
+ * calls that other threads make, such as a framework's worker threads): option 0 = tile order of the bf16 kernel (0
+ * problem-major, 1 contiguous runs per XCD, 2 = 1 with tile rows grouped by 4 so that the tiles an XCD runs at once share operand panels; default 2);
  * option 1 = its tile configuration (-1 chosen by size, 0 = 256 x 256 on 8 waves, 1 = 128 x 128, 2 = 256 x 256 on 4
  * waves, 3 = 256 x 256 on 8 MFMA waves fed by 4 load-only waves, 4 = 128 x 128 on 4 MFMA waves fed by 4 load-only
  * waves; other values are refused); option 2 = workgroups
  * per split-K V A product of the norm lower bound (default 1024); option 3 = MFMA steps per load batch of the V A
  * kernels (2, 4 or 8; default 4; the column-block kernel takes 2 or 4); option 4 = the V A kernel of full-storage
- * norm bounds (-1 by shape: 3 for bf16 launches of at least 16 matrices and 512 workgroups, one launch for the whole bound up to n 128 (256 in
- * bf16 or where fp32 rows are not 16-byte aligned), workgroups of 16 columns for launches of at most 128 64-column blocks
+ * norm bounds (-1 by shape: 3 for bf16 launches of at least 16 matrices and 512 workgroups, one launch for the whole
+ * bound up to n 128 (256 in bf16 or where fp32 rows are not 16-byte aligned), workgroups of 16 columns for launches of at most 128 64-column blocks
  * and unaligned fp32 rows, else 2; 0 split-K products plus a reduce kernel, 1 one workgroup
  * per 64 output columns over the whole k range, 2 the same with A staged through LDS in row-contiguous runs, 3 bf16
  * matrices of an even number of 64-tiles read from their upper tiles only, in tournament-paired rounds (else as 2);

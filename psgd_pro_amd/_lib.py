@@ -110,7 +110,7 @@ _SIGS = {
 }
 
 EXPORTED = tuple(_SIGS)
-ABI_VERSION = 4  # PSGDK_VERSION of include/psgdk.h that these signatures and structures follow
+ABI_VERSION = 5  # PSGDK_VERSION of include/psgdk.h that these signatures and structures follow
 
 _lib = None
 

@@ -111,7 +111,7 @@ def test_gemm_grouped_and_alpha_beta(hip):
 def test_syrk(hip, n, k, trans, prec):
     """Every output mode against float64 within the GEMM bound; the mirrored result exactly symmetric; the upper and
     mirrored modes (one kernel) bitwise equal on the upper triangle. With the tiny-product kernel off (option 11 = 0)
-    every kernel sums k in order, and the packed mode (the general engine) is bitwise the mirrored one."""
+    every kernel sums k in order, and the packed mode (the converting engine) is bitwise the mirrored one."""
     A = rnd(*((k, n) if trans else (n, k)), seed=n * 7 + k)
     Ad = A.to(DEV)
     X64 = (bf(A) if prec else A).double()
@@ -493,9 +493,9 @@ def test_gemm_bf16_k_contiguous(hip, b16cfg, m, n, k):
 @pytest.mark.parametrize("nb,m,n,k", [(1, 256, 256, 256), (1, 100, 70, 36), (1, 1, 50, 76), (1, 264, 520, 72),
                                       (1, 3072, 768, 768), (1, 1024, 1024, 3072), (12, 768, 768, 768)])
 def test_gemm_f32_k_contiguous(hip, nb, m, n, k):
-    """A (m x k) B^T with both fp32 operands k-contiguous (k a multiple of 4): the fp32 twin of the bf16 kernel (128
-    tiles, k summed in blocks of 128). Against float64: the elementwise bound of the other GEMM tests, and a worst
-    error no more than twice the general fp32 engine's on the same product (psgdk_set_option 8 = 0)."""
+    """A (m x k) B^T with both fp32 operands k-contiguous (k a multiple of 4): products by three-way splits, or the
+    small-problem kernels. Against float64: the elementwise bound of the other GEMM tests, and a worst error no more
+    than twice that of fp32 MFMAs on the same product (psgdk_set_option 8 = 0)."""
     As = [rnd(m, k, seed=m + i) for i in range(nb)]
     Bs = [rnd(n, k, seed=n + 7 * i + 1) for i in range(nb)]
     Ad = [a.to(DEV) for a in As]
