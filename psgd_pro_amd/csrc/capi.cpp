@@ -609,6 +609,16 @@ int run_nlb(int64_t n, int sign, int nb, const float* const* A, int64_t lda, con
   });
 }
 
+// Small fully stored matrices: the whole bound in one launch. Up to 256 where the products are bf16 or the column kernels
+// cannot read the rows, else up to 128: one workgroup's fp32 MFMAs take longer than seven launches beyond (whole bounds, us,
+// seven to eleven launches -> one: fp32 n 10 33 -> 20, 128 39 -> 32, 256 40 -> 75, 250 89 -> 61; bf16 64 34 -> 17, 256 36 ->
+// 31).
+bool nlb_one_launch(int64_t n, int nb, const void* const* A, int64_t lda, int a_bf16, const NlbWs& w) {
+  const bool wide = vmm_cols_ok(n, nb, A, lda, a_bf16 ? 2 : 4, w);
+  return g_vmm_cols == -1 && (!a_bf16 || wide) && n <= (a_bf16 || !wide ? NLB_SMALL_N : NLB_SMALL_N / 2) &&
+         n * lda < ((int64_t)1 << 29);
+}
+
 // stats_in_part: the producer of the (skew) matrices left per-(row, column block) row statistics in w.part
 // (rform_kernel's aux output; rform_stats_fit says where they fit), reduced here instead of a pass over A.
 int run_nlb_full(int64_t n, int sign, int nb, const void* const* A, int64_t lda, int a_bf16, const float* const* V,
@@ -616,16 +626,11 @@ int run_nlb_full(int64_t n, int sign, int nb, const void* const* A, int64_t lda,
   const float* Af[MAXB];
   for (int b = 0; b < nb; ++b) Af[b] = reinterpret_cast<const float*>(A[b]);
   NlbArgs a = nlb_args(n, sign, nb, Af, lda, w);
-  // small matrices: the whole bound in one launch. Up to 256 where the products are bf16 or the column kernels below
-  // cannot read the rows, else up to 128: one workgroup's fp32 MFMAs take longer than seven launches beyond (whole
-  // bounds, us, seven to eleven launches -> one: fp32 n 10 33 -> 20, 128 39 -> 32, 256 40 -> 75, 250 89 -> 61; bf16 64
-  // 34 -> 17, 256 36 -> 31).
-  const bool wide = vmm_cols_ok(n, nb, A, lda, a_bf16 ? 2 : 4, w);
-  if (g_vmm_cols == -1 && (!a_bf16 || wide) && n <= (a_bf16 || !wide ? NLB_SMALL_N : NLB_SMALL_N / 2) &&
-      n * lda < ((int64_t)1 << 29)) {
+  if (nlb_one_launch(n, nb, A, lda, a_bf16, w)) {
     for (int b = 0; b < nb; ++b) a.Vin[b] = V[b];
     return hip_check(nlb_small_launch(a, fin, a_bf16, st), "small norm bound");
   }
+  const bool wide = vmm_cols_ok(n, nb, A, lda, a_bf16 ? 2 : 4, w);
   nlb_full_plan(n, nb, w.part_cols, a.ksplit, a.kslice);
   a.vmm_u = g_vmm_u;
   a.vmm_cols = g_vmm_cols != 0 && wide ? (g_vmm_cols != 1 ? 2 : 1) : 0;
@@ -1060,7 +1065,10 @@ int b16_items(const std::vector<B16Item*>& it, const psgdk_update_opts_t* o, con
   }
   // R = Qn^T - Qn -> bf16 (r2: and the partials of sum R * Qn), with the skew bound's row statistics of the bf16 R
   // as a by-product (no separate pass over R)
-  const bool rstats = rform_stats_fit(d, nw);
+  // (none for the bounds that take one launch, which read R themselves)
+  const void* Rc[MAXB];
+  for (int b = 0; b < nb; ++b) Rc[b] = it[b]->Rb;
+  const bool rstats = rform_stats_fit(d, nw) && !nlb_one_launch(d, nb, Rc, d, 1, nw);
   {
     EwArgs a;
     std::memset(&a, 0, sizeof a);
@@ -1075,9 +1083,8 @@ int b16_items(const std::vector<B16Item*>& it, const psgdk_update_opts_t* o, con
     NlbFinal fin;
     std::memset(&fin, 0, sizeof fin);
     fin.mode = NLB_FINAL_SCALE;
-    const void* Rc[MAXB];
     const float* Vk[MAXB];
-    for (int b = 0; b < nb; ++b) { fin.coef[b] = it[b]->rs; Rc[b] = it[b]->Rb; Vk[b] = it[b]->Vk; }
+    for (int b = 0; b < nb; ++b) { fin.coef[b] = it[b]->rs; Vk[b] = it[b]->Vk; }
     PSGDK_TRY(run_nlb_full(d, -1, nb, Rc, d, 1, Vk, fin, nw, st, rstats));
   }
   if (o->r2) {  // procrustes_step_r2 (psgd_pro_fast.py:141-153)
