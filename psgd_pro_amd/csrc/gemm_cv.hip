@@ -544,14 +544,32 @@ __global__ void __launch_bounds__(WN == 4 || KG == 2 ? 512 : 256, 2) gemm_cv_ker
     if (out) each_acc([&](int i, int j, int e) INL { fin = fin && fabsf(acc[i][j][e]) < INFINITY; });
     const bool again = __syncthreads_or(!fin);
     if constexpr (GRAM) {  // the rows' own k: one exact product, one rounding
-      if (!again && out && m0 == n0)
+      // element (mn, k) of A, both from m0 on; plain rows by 32-bit offsets from (m0, m0), zero past the operand
+      const int ld = (int)oa.ld, nrow = (LAY & 1 ? p.K : p.M) - m0, ncol = (LAY & 1 ? p.M : p.K) - m0;
+      const __amdgpu_buffer_rsrc_t rs = make_rsrc(reinterpret_cast<const float*>(Ap) + m0 * (oa.ld + 1),
+                                                  ((nrow - 1) * oa.ld + ncol) * 4);
+      auto at = [&](int mn, int k) INL {
+        if constexpr (LAY & 4) {
+          return oa.bf16 ? ld_elem<bf16_t>(Ap, oa, m0 + mn, m0 + k, p.M, p.K)
+                         : ld_elem<float>(Ap, oa, m0 + mn, m0 + k, p.M, p.K);
+        } else {
+          const int off = LAY & 1 ? k * ld + mn : mn * ld + k;
+          return __builtin_bit_cast(float, __builtin_amdgcn_raw_buffer_load_b32(rs, m0 + k < p.K ? off * 4 : kOob, 0, 0));
+        }
+      };
+      if (!again && out && m0 == n0 && m0 < p.K) {
+        float d[FM][NE];
+#pragma unroll
+        for (int i = 0; i < FM; ++i)
+#pragma unroll
+          for (int e = 0; e < NE; ++e) {
+            const int k = wm * TM + i * MT + acc_row(g, e);
+            d[i][e] = at(k, k);
+          }
         each_acc([&](int i, int j, int e) INL {
-          const int row = m0 + wm * TM + i * MT + acc_row(g, e), col = n0 + wn * TN + j * MT + r;
-          auto at = [&](int mn) INL {
-            return oa.bf16 ? ld_elem<bf16_t>(Ap, oa, mn, row, p.M, p.K) : ld_elem<float>(Ap, oa, mn, row, p.M, p.K);
-          };
-          acc[i][j][e] = fmaf(at(row), at(col), acc[i][j][e]);
+          acc[i][j][e] = fmaf(d[i][e], at(wn * TN + j * MT + r, wm * TM + i * MT + acc_row(g, e)), acc[i][j][e]);
         });
+      }
     }
     if (again) {
       zero();
