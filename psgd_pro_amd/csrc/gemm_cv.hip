@@ -38,12 +38,12 @@
 // What bounds it. fp32, 128 x 256: a 32-k stage is 3072 MFMA cycles per SIMD pair of waves against about 180 VALU
 // instructions of address, split and store per converting wave, 72 KB of LDS writes and 144 KB of fragment reads: two
 // groups of four waves a half step apart, so that one converts while the other multiplies (a single group left the matrix
-// cores idle during every conversion). 3072^3: 671 us on the fp32 MFMA kernel this replaces, now 470; two at once 1065,
-// now 709; 4096^3 1188, now 741. 64 x 64: latency and occupancy; k split over two wave groups while a launch has at most
-// a tile per CU (1024^3: 86 us, now 24; symmetric 2304 x 768 from its triangle: 289, now 125; 1001 x 770 x 770, unaligned
+// cores idle during every conversion). 3072^3: 671 us on the fp32 MFMA kernel this replaces, now 437; two at once 1065,
+// now 683; 4096^3 1188, now 663. 64 x 64: latency and occupancy; k split over two wave groups while a launch has at most
+// a tile per CU (1024^3: 86 us, now 24; symmetric 2304 x 768 from its triangle: 287, now 118; 1001 x 770 x 770, unaligned
 // rows: 148, now 22). Beyond, 64-tiles in groups of four waves; 128 x 256 tiles once they fill half the chip.
 // bf16 precision from fp32 or transposed operands: 3 to 8 times faster than reading them into bf16 LDS tiles element by
-// element (1531^3 38 us, 4096^3 281).
+// element (1531^3 36 us, 4096^3 255).
 #include <type_traits>
 
 #include "gemm_cv.h"
