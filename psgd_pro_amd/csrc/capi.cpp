@@ -420,7 +420,7 @@ int run_gemm(int prec, int nb, int64_t M, int64_t N, int64_t K, const Opnd& A, c
     a.A[b] = A.p[b]; a.B[b] = B.p[b]; a.C[b] = C[b];
     a.X1[b] = e.X1[b]; a.X2[b] = e.X2[b]; a.s[b] = e.s[b]; a.part[b] = e.part[b];
   }
-  a.gram = prec == PSGDK_PREC_F32 && tri && e.epi == EPI_STORE && (e.gram || A.mode == MC);
+  a.gram = prec == PSGDK_PREC_F32 && tri && e.epi == EPI_STORE && (e.gram || A.mode == MC) && A.ld < (1 << 21);
   const int cfg = cv_cfg(prec, M, N, tri, nb, e.epi, !gemm_cv_wide(a, prec), a.gram);
   if (ntiles) *ntiles = gemm_cv_tiles(M, N, tri, cfg);
   if (!g_prof.on) return hip_check(gemm_cv_launch(a, prec, cfg, st), "gemm launch");
@@ -474,11 +474,18 @@ struct NlbWs {
   int64_t part_cols;  // capacity of part[b] in columns of 32 rows
 };
 
-// Split of the V A products read from the triangle: one workgroup (32 x 64 tile, one k range) per CU, k ranges of at
-// least 128 (n 2048: 8 ranges of 256, 18 us per product; 32 ranges of 64 on 1024 workgroups took 30).
+// Split of the V A products read from the triangle, a workgroup per 32 x 64 tile and k range: k ranges of at least 128, in
+// the number that makes the rounds of 256 workgroups times the range shortest, one percent of a whole range charged for
+// each (n 2048: 8 ranges of 256, one round, 18 us per product; 32 ranges of 64 took 30. Calls: n 3072 65 us with 6 ranges in
+// a round and an eighth, 45 with 5 in one; n 4097 96 with 4, 76 with 7).
 void nlb_plan(int64_t n, int nb, int& splits, int64_t& kchunk) {
   const int64_t tiles = (n + 63) / 64 * nb;
-  const int64_t s = std::max<int64_t>(1, std::min((256 + tiles - 1) / tiles, n / 128));
+  int64_t s = 1;
+  double best = 0;
+  for (int64_t t = 1; t <= std::max<int64_t>(1, std::min<int64_t>(16, n / 128)); ++t) {
+    const double cost = (double)((tiles * t + 255) / 256) / (double)t + 0.01 * (double)t;
+    if (t == 1 || cost < best) { best = cost; s = t; }
+  }
   kchunk = ((n + s - 1) / s + 63) / 64 * 64;
   splits = (int)((n + kchunk - 1) / kchunk);
 }
@@ -1839,14 +1846,16 @@ int psgdk_tri_vmm(int64_t n, int sign, int nb, const float* const* V, const floa
   if (sign != 1 && sign != -1) return fail(PSGDK_EINVAL, "sign = %d", sign);
   if (lda < n) return fail(PSGDK_ESHAPE, "lda < n");
   hipStream_t st = (hipStream_t)stream;
-  // the 16-column kernel writes W while other workgroups still read V and A: only where they lie apart
+  // Matrices over 2 GiB, whose tiles alone are more than a round: the 16-column kernel (n 23200: 800 us against 1825; its
+  // fp32 MFMA chains of 32 k are 2.2e-7 off float64, split products 1.9e-7, and below 2 GiB 1.4e-7 against 9e-8). It
+  // writes W while other workgroups still read V and A: only where they lie apart.
   bool apart = true;
   for (int b = 0; b < nb; ++b)
     for (int c = 0; c < nb; ++c) {
       const float *w0 = W[b], *w1 = w0 + NLB_K * n;
       apart = apart && (w1 <= V[c] || V[c] + NLB_K * n <= w0) && (w1 <= A[c] || A[c] + (n - 1) * lda + n <= w0);
     }
-  if (apart && strip_ok(n, lda, 0)) {
+  if (apart && n * lda >= ((int64_t)1 << 29) && strip_ok(n, lda, 0)) {
     NlbArgs a;
     std::memset(&a, 0, sizeof a);
     a.nb = nb; a.n = (int)n; a.sign = sign; a.lda = lda; a.vmm_cols = 4; a.tri = 1;
