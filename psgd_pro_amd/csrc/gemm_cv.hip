@@ -544,18 +544,17 @@ __global__ void __launch_bounds__(WN == 4 || KG == 2 ? 512 : 256, 2) gemm_cv_ker
     if (out) each_acc([&](int i, int j, int e) INL { fin = fin && fabsf(acc[i][j][e]) < INFINITY; });
     const bool again = __syncthreads_or(!fin);
     if constexpr (GRAM) {  // the rows' own k: one exact product, one rounding
-      // element (mn, k) of A, both from m0 on; plain rows by 32-bit offsets from (m0, m0), zero past the operand
-      const int ld = (int)oa.ld, nrow = (LAY & 1 ? p.K : p.M) - m0, ncol = (LAY & 1 ? p.M : p.K) - m0;
-      const __amdgpu_buffer_rsrc_t rs = make_rsrc(reinterpret_cast<const float*>(Ap) + m0 * (oa.ld + 1),
-                                                  ((nrow - 1) * oa.ld + ncol) * 4);
+      // element (mn, k) of A, both from m0 on, by 32-bit offsets from (m0, m0); zero past the operand's end
+      constexpr bool ANY = (LAY & 4) != 0;  // rows in bf16, in either layout
+      const bool mc = ANY ? oa.mode == MC : (LAY & 1) != 0;
+      const int ld = (int)oa.ld, nrow = (mc ? p.K : p.M) - m0, ncol = (mc ? p.M : p.K) - m0;
+      const int sm = mc ? 1 : ld, sk = mc ? ld : 1, sh = ANY ? 1 : 2;
+      const __amdgpu_buffer_rsrc_t rs = make_rsrc(reinterpret_cast<const char*>(Ap) + ((m0 * (oa.ld + 1)) << sh),
+                                                  ((nrow - 1) * oa.ld + ncol) << sh);
       auto at = [&](int mn, int k) INL {
-        if constexpr (LAY & 4) {
-          return oa.bf16 ? ld_elem<bf16_t>(Ap, oa, m0 + mn, m0 + k, p.M, p.K)
-                         : ld_elem<float>(Ap, oa, m0 + mn, m0 + k, p.M, p.K);
-        } else {
-          const int off = LAY & 1 ? k * ld + mn : mn * ld + k;
-          return __builtin_bit_cast(float, __builtin_amdgcn_raw_buffer_load_b32(rs, m0 + k < p.K ? off * 4 : kOob, 0, 0));
-        }
+        const int off = m0 + k < p.K ? (mn * sm + k * sk) << sh : kOob;
+        if constexpr (ANY) return bf16_to_f32(__builtin_amdgcn_raw_buffer_load_b16(rs, off, 0, 0));
+        else return __builtin_bit_cast(float, __builtin_amdgcn_raw_buffer_load_b32(rs, off, 0, 0));
       };
       if (!again && out && m0 == n0 && m0 < p.K) {
         float d[FM][NE];
@@ -566,9 +565,17 @@ __global__ void __launch_bounds__(WN == 4 || KG == 2 ? 512 : 256, 2) gemm_cv_ker
             const int k = wm * TM + i * MT + acc_row(g, e);
             d[i][e] = at(k, k);
           }
-        each_acc([&](int i, int j, int e) INL {
-          acc[i][j][e] = fmaf(d[i][e], at(wn * TN + j * MT + r, wm * TM + i * MT + acc_row(g, e)), acc[i][j][e]);
-        });
+#pragma unroll
+        for (int i = 0; i < FM; ++i)
+#pragma unroll
+          for (int j = 0; j < FN; ++j) {
+            const int mn = wn * TN + j * MT + r, k = wm * TM + i * MT + acc_row(g, 0);
+            f32x4_t x;  // k .. k + 3: one load where they are neighbours (past K they are another row's)
+            if constexpr (!ANY && !(LAY & 1)) x = ld_f32x4(rs, m0 + k < p.K ? (mn * ld + k) * 4 : kOob);
+            else x = f32x4_t{at(mn, k), at(mn, k + 1), at(mn, k + 2), at(mn, k + 3)};
+#pragma unroll
+            for (int e = 0; e < NE; ++e) acc[i][j][e] = fmaf(d[i][e], m0 + k + e < p.K ? x[e] : 0.f, acc[i][j][e]);
+          }
       }
     }
     if (again) {

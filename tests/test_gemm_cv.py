@@ -275,3 +275,17 @@ def test_epilogues_of_sums_that_are_not_finite(engine, d, value):
         assert torch.equal(x[~fin & ~torch.isnan(y)], y[~fin & ~torch.isnan(y)]), i
         x, y = (torch.where(fin, v, 0.0).double().reshape(-1, v.shape[-1]) for v in (x, y))
         assert ((x - y).abs() <= 1e-5 * y.abs().amax(1, keepdim=True)).all(), i
+
+
+@pytest.mark.parametrize("n,k", [(130, 70), (129, 129), (200, 333), (64, 1)])
+@pytest.mark.parametrize("dt", [torch.float32, torch.bfloat16])
+def test_gram_products_beside_their_own_k(engine, n, k, dt):
+    """X X^T and X^T X from rows amid NaN, with fewer, as many and more k than rows: the rows' own k end inside a diagonal
+    tile, and what lies beyond must not reach it."""
+    for trans in (False, True):
+        r, c = (k, n) if trans else (n, k)
+        wide = torch.full((r + 2, c + 5), float("nan"), device=DEV, dtype=dt)
+        X = wide[1:1 + r, 3:3 + c]
+        X.copy_(torch.randn(r, c, generator=torch.Generator().manual_seed(n + k)))
+        x = X.T if trans else X
+        _check(K.syrk(X, trans, L.OUT_MIRROR, False), x, x.T, False, (n, k, trans, dt))
